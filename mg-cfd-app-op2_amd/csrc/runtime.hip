@@ -1128,7 +1128,7 @@ static int build_partplan(InvPlan& P, op_map m, const std::vector<int>& ptr, con
     P.pt_rs = (lds_bound || (long long)parts.size() < 4LL * R.n_cu) ? 5 : kPRec;
     if (P.pt_rs_set) P.pt_rs = P.pt_rs_set;
     P.pt_lds = sizeof(double) * ((size_t)rec_cap * P.pt_rs + (size_t)kPart * 5);
-    P.pt_lds32 = sizeof(double) * (((size_t)rec_cap * PartRec<float>::kStride * sizeof(float) + 7) / 8 +
+    P.pt_lds32 = sizeof(double) * (((size_t)rec_cap * kPRec32 * sizeof(float) + 7) / 8 +
                                    (size_t)kPart * 5);   // FP32 records, FP64 accumulators
     return 0;
 }
@@ -1430,14 +1430,14 @@ static int refresh_plan_weights(int variant, InvPlan& P, op_dat w)
     if (mixed_variant(variant) && P.pt_parts > 0 &&
         (!P.d_pt_w32 || P.pt_w32dat != (const void*)w || P.pt_w32ver != D(w)->version)) {
         if (!P.d_pt_w32) HIPCHK(hipMalloc(&P.d_pt_w32, sizeof(float) * 3 * std::max<size_t>(1, (size_t)P.pt_nloc)));
-        k_pack_part_weights32<<<nblk((size_t)P.pt_nloc), kBlock, 0, cur_stream()>>>(P.pt_nloc, P.d_pt_eid, dptr(w),
+        k_pack_part_weights<float><<<nblk((size_t)P.pt_nloc), kBlock, 0, cur_stream()>>>(P.pt_nloc, P.d_pt_eid, dptr(w),
                                                                               P.d_pt_w32);
         TRY(check_launch());
         P.pt_w32dat = w;
         P.pt_w32ver = D(w)->version;
     }
     if (part_variant(variant) && P.pt_parts > 0 && (P.pt_wdat != (const void*)w || P.pt_wver != D(w)->version)) {
-        k_pack_part_weights<<<nblk((size_t)P.pt_nloc), kBlock, 0, cur_stream()>>>(P.pt_nloc, P.d_pt_eid, dptr(w),
+        k_pack_part_weights<double><<<nblk((size_t)P.pt_nloc), kBlock, 0, cur_stream()>>>(P.pt_nloc, P.d_pt_eid, dptr(w),
                                                                             P.d_pt_w);
         TRY(check_launch());
         P.pt_wdat = w;
@@ -1518,7 +1518,7 @@ static int launch_part_t(bool coloured, const InvPlan& P, const Real* w, size_t 
         if (P.pt_rs == 5 || st)
             return launch_part_rs<Real, T, EPT, NPT, 5>(coloured, P, w, lds, var, flux, status, fresh, st);
     }
-    return launch_part_rs<Real, T, EPT, NPT, PartRec<Real>::kStride>(coloured, P, w, lds, var, flux, status, fresh,
+    return launch_part_rs<Real, T, EPT, NPT, (sizeof(Real) == sizeof(float) ? kPRec32 : kPRec)>(coloured, P, w, lds, var, flux, status, fresh,
                                                                     st);
 }
 
