@@ -493,14 +493,27 @@ __device__ __forceinline__ void part_apply(double* acc, unsigned code, const O i
 // FP32 records have six values; FP64 ones six, or five (40 bytes) when
 // 48-byte records would leave fewer than four workgroups per CU and in the
 // kernel with the fused stage.
-constexpr int kPRec32 = 6;
+constexpr int kPRec32 = 6;     // values an FP32 record takes up (24 bytes: 8-byte aligned), with or without speed
+
+template <typename R, int RS>
+__host__ __device__ constexpr int part_stride()
+{
+    static_assert(RS == 5 || RS == 6, "record size");
+    return sizeof(R) == sizeof(double) ? RS : kPRec32;
+}
+
+// Doubles that 'n' records take up.
+template <typename R, int RS>
+__host__ __device__ constexpr size_t part_rec_doubles(int n)
+{
+    return ((size_t)n * part_stride<R, RS>() * sizeof(R) + sizeof(double) - 1) / sizeof(double);
+}
 
 template <typename R, int RS>
 __device__ __forceinline__ PState<R> part_rec_state(const R* r)
 {
-    static_assert(RS == 6 || (RS == 5 && sizeof(R) == sizeof(double)), "record size");
     PState<R> t;
-    if constexpr (RS == 6) {
+    if constexpr (part_stride<R, RS>() == 6) {
         using R2 = typename std::conditional<sizeof(R) == 8, double2, float2>::type;
         const R2* q = reinterpret_cast<const R2*>(r);
         const R2 a = q[0], b = q[1], c = q[2];
@@ -562,7 +575,7 @@ __device__ __forceinline__ void part_store_records(const PartInfo& P, int t, con
         const int sl = t + k * T;
         if (sl < nrec) {
             const R x0 = (R)U[k][0], x1 = (R)U[k][1], x2 = (R)U[k][2], x3 = (R)U[k][3], x4 = (R)U[k][4];
-            R* r = rec + sl * RS;
+            R* r = rec + sl * part_stride<R, RS>();
             r[0] = x0; r[1] = x1; r[2] = x2; r[3] = x3; r[4] = x4;
             if constexpr (RS > 5) r[5] = part_speed<R>(x0, x1, x2, x3, x4);
         }
@@ -620,21 +633,62 @@ __device__ __forceinline__ void part_edges_atomic(const R* rec, double* acc, con
 #pragma unroll
     for (int i = 0; i < EPT; i++) {
         if (!code[i]) continue;
-        const PState<R> a = part_rec_state<R, RS>(rec + (code[i] & 1023u) * RS);
-        const PState<R> b = part_rec_state<R, RS>(rec + ((code[i] >> 10) & 1023u) * RS);
+        const PState<R> a = part_rec_state<R, RS>(rec + (code[i] & 1023u) * part_stride<R, RS>());
+        const PState<R> b = part_rec_state<R, RS>(rec + ((code[i] >> 10) & 1023u) * part_stride<R, RS>());
         R inc[5];
         part_increment<R, R>(a, b, w0[i], w1[i], w2[i], sc, inc);
         part_apply(acc, code[i], inc);
     }
 }
 
+// Accumulates the part's local edges (codes and weights in registers) into
+// the LDS accumulators; ends with a barrier.  LAZY (coloured only): form each
+// edge's increment in its colour's phase instead of all of them up front, so
+// no increments are held across the phases (fewer registers, for the kernel
+// with the fused stage).
+template <typename R, int EPT, bool COLOURED, int RS, bool LAZY>
+__device__ __forceinline__ void part_edges(const PartInfo& P, const R* rec, double* acc, const unsigned code[EPT],
+                                           const R w0[EPT], const R w1[EPT], const R w2[EPT], R sc)
+{
+    constexpr int ST = part_stride<R, RS>();
+    if constexpr (COLOURED && LAZY) {
+        for (int c = 0; c < P.ncol; c++) {
+#pragma unroll
+            for (int i = 0; i < EPT; i++)
+                if (code[i] && (int)(code[i] >> 22) == c) {
+                    const PState<R> a = part_rec_state<R, RS>(rec + (code[i] & 1023u) * ST);
+                    const PState<R> b = part_rec_state<R, RS>(rec + ((code[i] >> 10) & 1023u) * ST);
+                    R inc[5];
+                    part_increment<R, R>(a, b, w0[i], w1[i], w2[i], sc, inc);
+                    part_apply(acc, code[i], inc);
+                }
+            __syncthreads();
+        }
+    } else if constexpr (COLOURED) {
+        R inc[EPT][5];      // held in the arithmetic's precision until the colour walk
+#pragma unroll
+        for (int i = 0; i < EPT; i++)
+            if (code[i]) {
+                const PState<R> a = part_rec_state<R, RS>(rec + (code[i] & 1023u) * ST);
+                const PState<R> b = part_rec_state<R, RS>(rec + ((code[i] >> 10) & 1023u) * ST);
+                part_increment<R, R>(a, b, w0[i], w1[i], w2[i], sc, inc[i]);
+            }
+        for (int c = 0; c < P.ncol; c++) {
+#pragma unroll
+            for (int i = 0; i < EPT; i++)
+                if (code[i] && (int)(code[i] >> 22) == c) part_apply(acc, code[i], inc[i]);
+            __syncthreads();
+        }
+    } else {
+        part_edges_atomic<R, EPT, RS>(rec, acc, code, w0, w1, w2, sc);
+        __syncthreads();
+    }
+}
+
 // Stages one part and accumulates its local edges: returns the FP64
 // accumulators (in LDS, after a barrier) holding the edge flux of the part's
 // owned nodes, started from the flux dat or, with fresh, from zero.
-// LAZY (coloured only): form each edge's increment in its colour's phase
-// instead of all of them up front, so no increments are held across the
-// phases (fewer registers, for the kernel with the fused stage).
-template <typename R, int T, int EPT, int NPT, bool COLOURED, int RS, bool LAZY>
+template <typename R, int T, int EPT, int NPT, bool COLOURED, int RS>
 __device__ __forceinline__ double* part_accumulate(const PartInfo& P, const int* __restrict__ halo,
                                                    const unsigned* __restrict__ ecode, const R* __restrict__ ew,
                                                    long long nloc, int rec_cap, const double* __restrict__ var,
@@ -644,7 +698,7 @@ __device__ __forceinline__ double* part_accumulate(const PartInfo& P, const int*
     constexpr int FL = (5 * kPart + T - 1) / T;
     const int t = threadIdx.x;
     R* rec = reinterpret_cast<R*>(sm);
-    double* acc = sm + ((size_t)rec_cap * RS * sizeof(R) + sizeof(double) - 1) / sizeof(double);
+    double* acc = sm + part_rec_doubles<R, RS>(rec_cap);
     // 1. loads: halo entries, edge codes and weights, then node states and
     // the owned flux; records (with |u| + c) and accumulators into LDS
     int nd[NPT];
@@ -659,39 +713,7 @@ __device__ __forceinline__ double* part_accumulate(const PartInfo& P, const int*
     part_store_flux<T, FL>(P, t, fl, acc);
     __syncthreads();
     // 2./3. edges
-    const R sc = (R)k.sc;
-    if constexpr (COLOURED && LAZY) {
-        for (int c = 0; c < P.ncol; c++) {
-#pragma unroll
-            for (int i = 0; i < EPT; i++)
-                if (code[i] && (int)(code[i] >> 22) == c) {
-                    const PState<R> a = part_rec_state<R, RS>(rec + (code[i] & 1023u) * RS);
-                    const PState<R> b = part_rec_state<R, RS>(rec + ((code[i] >> 10) & 1023u) * RS);
-                    R inc[5];
-                    part_increment<R, R>(a, b, w0[i], w1[i], w2[i], sc, inc);
-                    part_apply(acc, code[i], inc);
-                }
-            __syncthreads();
-        }
-    } else if constexpr (COLOURED) {
-        R inc[EPT][5];      // held in the arithmetic's precision until the colour walk
-#pragma unroll
-        for (int i = 0; i < EPT; i++)
-            if (code[i]) {
-                const PState<R> a = part_rec_state<R, RS>(rec + (code[i] & 1023u) * RS);
-                const PState<R> b = part_rec_state<R, RS>(rec + ((code[i] >> 10) & 1023u) * RS);
-                part_increment<R, R>(a, b, w0[i], w1[i], w2[i], sc, inc[i]);
-            }
-        for (int c = 0; c < P.ncol; c++) {
-#pragma unroll
-            for (int i = 0; i < EPT; i++)
-                if (code[i] && (int)(code[i] >> 22) == c) part_apply(acc, code[i], inc[i]);
-            __syncthreads();
-        }
-    } else {
-        part_edges_atomic<R, EPT, RS>(rec, acc, code, w0, w1, w2, sc);
-        __syncthreads();
-    }
+    part_edges<R, EPT, COLOURED, RS, false>(P, rec, acc, code, w0, w1, w2, (R)k.sc);
     return acc;
 }
 
@@ -711,8 +733,7 @@ __global__ __launch_bounds__(T) void k_flux_part(
     const int halt = status_of(status);     // tested before the store
     const PartInfo P = parts[xcd_block()];
     const double* acc =
-        part_accumulate<R, T, EPT, NPT, COLOURED, RS, false>(P, halo, ecode, ew, nloc, rec_cap, var, flux, k, fresh,
-                                                             sm);
+        part_accumulate<R, T, EPT, NPT, COLOURED, RS>(P, halo, ecode, ew, nloc, rec_cap, var, flux, k, fresh, sm);
     if (halt) return;
     // 4. store
     double* fw = flux + (size_t)P.n0 * 5;
@@ -1201,29 +1222,37 @@ struct StageArgs {
     const int* status;
 };
 
-// First stage: the minimum dt of the workgroup's mesh, reduced from the
-// mesh's slots that the kernel computing dt filled (min_publish); the mesh's
-// first workgroup raises abort code 1 on a negative value
-// (euler3d.cpp:476-484).  Second stage: the slots are reset for the next
-// smoothing step.
-template <int NT>
-__device__ __forceinline__ double stage_min_dt(const StageArgs& a, int seg, bool first)
+// Minimum over the 64 lanes of a wave, in every lane: row shifts leave each
+// row's minimum in its last lane, two broadcasts carry it to lane 63.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double wave_min_step(double x)
 {
-    // the slot minimum over the images (unsigned order), with uniform loads:
-    // the reduction stays in scalar registers, off the vector registers the
-    // edge phase needs
-    const unsigned* sl = reinterpret_cast<const unsigned*>(a.mslots + (size_t)seg * kMinSlots);
-    unsigned khi = (unsigned)(kMinEmpty >> 32), klo = (unsigned)kMinEmpty;
-#pragma unroll 8
-    for (int j = 0; j < kMinSlots; j++) {
-        const unsigned yhi = __builtin_amdgcn_readfirstlane(sl[2 * j + 1]);
-        const unsigned ylo = __builtin_amdgcn_readfirstlane(sl[2 * j]);
-        const bool lt = yhi < khi || (yhi == khi && ylo < klo);
-        khi = lt ? yhi : khi;
-        klo = lt ? ylo : klo;
-    }
-    const double m = min_unkey(((unsigned long long)khi << 32) | klo);
-    const double mdt = (m < DBL_MAX) ? m : DBL_MAX;
+    const int lo = __double2loint(x), hi = __double2hiint(x);
+    const double y = __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, CTRL, ROWS, 0xf, false),
+                                      __builtin_amdgcn_update_dpp(lo, lo, CTRL, ROWS, 0xf, false));
+    return y < x ? y : x;
+}
+__device__ __forceinline__ double wave_min(double x)
+{
+    x = wave_min_step<0x111, 0xf>(x);      // row_shr 1, 2, 4, 8
+    x = wave_min_step<0x112, 0xf>(x);
+    x = wave_min_step<0x114, 0xf>(x);
+    x = wave_min_step<0x118, 0xf>(x);
+    x = wave_min_step<0x142, 0xa>(x);      // row_bcast 15
+    x = wave_min_step<0x143, 0xc>(x);      // row_bcast 31
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), 63),
+                            __builtin_amdgcn_readlane(__double2loint(x), 63));
+}
+
+// First stage: the minimum dt of the workgroup's mesh, reduced by each wave
+// from the mesh's slots that the kernel computing dt filled (min_publish;
+// 'slot' is this lane's, loaded early); the mesh's first workgroup raises
+// abort code 1 on a negative value (euler3d.cpp:476-484).  Second stage: the
+// slots are reset for the next smoothing step.
+static_assert(kMinSlots == kWave, "one slot per lane");
+__device__ __forceinline__ double stage_min_dt(const StageArgs& a, int seg, unsigned long long slot, bool first)
+{
+    const double mdt = wave_min(min_candidate(min_unkey(slot)));
     if (first && threadIdx.x == 0) {
         if (mdt < 0.0 && a.mstatus[seg] == 0) a.mstatus[seg] = 1;
         if (a.zero) *a.zero = 0;
@@ -1238,9 +1267,38 @@ __device__ __forceinline__ void stage_reset_min(const StageArgs& a)
         for (int i = threadIdx.x; i < a.nmslots; i += NT) a.mslots[i] = kMinEmpty;
 }
 
+// A node's boundary and far-field increments (flux.h:14-39) added to its flux
+// f in boundary-element order; U: its state, [q0, q1): its elements.
+__device__ __forceinline__ void stage_bnd(const StageArgs& a, const Consts& k, const double U[5], int q0, int q1,
+                                          double f[5])
+{
+#pragma clang fp contract(off)
+    Th b;
+    thermo_exact(U, b);
+    for (int q = q0; q < q1; q++) {
+        const double4 bq = a.bnw[q];
+        const int g = (int)bq.w;
+        const double w0 = bq.x, w1 = bq.y, w2 = bq.z;
+        if (g <= 2) {
+            f[0] = f[0] + 0.0;
+            f[1] = f[1] + w0 * b.p;
+            f[2] = f[2] + w1 * b.p;
+            f[3] = f[3] + w2 * b.p;
+            f[4] = f[4] + 0.0;
+        } else if (g <= 7) {
+            const double fx = 0.5 * w0, fy = 0.5 * w1, fz = 0.5 * w2;
+            f[0] += fx * (k.ffv[1] + b.mx) + fy * (k.ffv[2] + b.my) + fz * (k.ffv[3] + b.mz);
+            f[4] += fx * (k.ffde[0] + b.fdx) + fy * (k.ffde[1] + b.fdy) + fz * (k.ffde[2] + b.fdz);
+            f[1] += fx * (k.ffmx[0] + b.fxx) + fy * (k.ffmx[1] + b.fxy) + fz * (k.ffmx[2] + b.fxz);
+            f[2] += fx * (k.ffmy[0] + b.fxy) + fy * (k.ffmy[1] + b.fyy) + fz * (k.ffmy[2] + b.fyz);
+            f[3] += fx * (k.ffmz[0] + b.fxz) + fy * (k.ffmz[1] + b.fyz) + fz * (k.ffmz[2] + b.fzz);
+        }
+    }
+}
+
 // One node of a Runge-Kutta stage, in the reference's order: f holds node
 // i's edge flux; the node's boundary and far-field increments are added
-// (flux.h:14-39, its state read from vin), the step factor is formed on the
+// (stage_bnd, its state read from vin), the step factor is formed on the
 // first stage (time_stepping_kernels.h:43-64), the update written to a.var
 // (:66-86), the flux reset when asked, and on the last stage the residual
 // with its square sum and NaN/Inf count (validation.h:27-44,102-115).
@@ -1254,30 +1312,9 @@ __device__ __forceinline__ void stage_node(const StageArgs& a, const Consts& k0,
 #pragma clang fp contract(off)
     double u[5];
     if (q0 < q1) {
-        const Consts& k = a.kseg ? a.kseg[seg] : k0;
         double U[5];
         load5(vin, i, U);
-        Th b;
-        thermo_exact(U, b);
-        for (int q = q0; q < q1; q++) {
-            const double4 bq = a.bnw[q];
-            const int g = (int)bq.w;
-            const double w0 = bq.x, w1 = bq.y, w2 = bq.z;
-            if (g <= 2) {
-                f[0] = f[0] + 0.0;
-                f[1] = f[1] + w0 * b.p;
-                f[2] = f[2] + w1 * b.p;
-                f[3] = f[3] + w2 * b.p;
-                f[4] = f[4] + 0.0;
-            } else if (g <= 7) {
-                const double fx = 0.5 * w0, fy = 0.5 * w1, fz = 0.5 * w2;
-                f[0] += fx * (k.ffv[1] + b.mx) + fy * (k.ffv[2] + b.my) + fz * (k.ffv[3] + b.mz);
-                f[4] += fx * (k.ffde[0] + b.fdx) + fy * (k.ffde[1] + b.fdy) + fz * (k.ffde[2] + b.fdz);
-                f[1] += fx * (k.ffmx[0] + b.fxx) + fy * (k.ffmx[1] + b.fxy) + fz * (k.ffmx[2] + b.fxz);
-                f[2] += fx * (k.ffmy[0] + b.fxy) + fy * (k.ffmy[1] + b.fyy) + fz * (k.ffmy[2] + b.fyz);
-                f[3] += fx * (k.ffmz[0] + b.fxz) + fy * (k.ffmz[1] + b.fyz) + fz * (k.ffmz[2] + b.fzz);
-            }
-        }
+        stage_bnd(a, a.kseg ? a.kseg[seg] : k0, U, q0, q1, f);
     }
     double sfi;
     if (a.rk == 0) {
@@ -1354,7 +1391,7 @@ __global__ __launch_bounds__(kBlock) void k_stage(StageArgs a, Consts k0)
     }
     double mdt = 0.0;
     if (a.rk == 0) {
-        mdt = stage_min_dt<kBlock>(a, seg, first);
+        mdt = stage_min_dt(a, seg, a.mslots[(size_t)seg * kMinSlots + threadIdx.x % kMinSlots], first);
         if (mdt < 0.0 && a.status) return;   // a halting context aborts before any update
     }
     double s = 0.0;
@@ -1374,48 +1411,136 @@ __global__ __launch_bounds__(kBlock) void k_stage(StageArgs a, Consts k0)
 // owned nodes, so the stage update of those nodes runs in the same
 // workgroup.  Other parts read the stage's input state as their halo while
 // this one writes its update, so the input (vin) and the update (a.var) are
-// different buffers.  The edge flux starts from the flux dat on the first
-// stage (fresh == 0) and from zero after it; it is not written back.
+// different buffers.  The edge flux starts from the flux dat where that may
+// hold something (fresh == 0), else from zero; it is not written back.
 // pseg / pfirst: segment of each part and first part of each segment
 // (batched solves), null for one mesh.  Returns false when the context has
 // halted or aborts (negative minimum dt).
+//
+// Bound by memory traffic on levels that fill the chip, by one workgroup's
+// latency on smaller ones.  A part's owned nodes are one run of 5 * cnt
+// doubles in every [n][5] array, and the stage update is the same for each
+// double, so the owned state, the old state, the old flux and all results
+// move as that run, consecutive doubles by consecutive lanes (per-node
+// accesses at a 40-byte stride touch three times as many lines); only the
+// halo is gathered node by node.  Cycle of a 1M-node solve 908 -> 863 us,
+// 300K nodes 397 -> 384 us, 10K 213 -> 196 us (the minimum-dt slots, one per
+// lane, are loaded early too).  NPT: halo nodes per thread.
 template <typename R, int T, int EPT, int NPT, bool COLOURED, int RS>
 __device__ __forceinline__ bool part_stage_one(
     int p, const PartInfo* __restrict__ parts, const int* __restrict__ halo, const unsigned* __restrict__ ecode,
     const R* __restrict__ ew, long long nloc, int rec_cap, const double* __restrict__ vin, int fresh,
     const StageArgs& a, const Consts& k0, const int* __restrict__ pseg, const int* __restrict__ pfirst, double* sm)
 {
+    constexpr int ST = part_stride<R, RS>();
+    constexpr int FL = (5 * kPart + T - 1) / T;
+    static_assert(T >= kPart, "one owned node per thread");
     // a halted context writes nothing: the status is tested after the edge
     // phase (which writes only LDS), so its load overlaps the staging loads
     const int halt = status_of(a.status);
     const PartInfo P = parts[p];
     const int seg = word_or_zero(pseg, p);
-    static_assert(T >= kPart, "one owned node per thread");
-    // the owned node's old state and volume / step factor, in flight through
-    // the edge phase (clamped to a valid node for threads without one)
     const int t = threadIdx.x;
-    const int i = P.n0 + min(t, max(P.cnt - 1, 0));
-    double o[5];
-    load5(a.old, i, o);
-    const double vs = a.rk == 0 ? a.vol[i] : a.sf[i];
-    const int q0 = a.bptr ? a.bptr[i] : 0, q1 = a.bptr ? a.bptr[i + 1] : 0;
-    double* acc = part_accumulate<R, T, EPT, NPT, COLOURED, RS, true>(P, halo, ecode, ew, nloc, rec_cap, vin,
-                                                                      a.flux, k0, fresh, sm);
+    R* rec = reinterpret_cast<R*>(sm);
+    double* acc = sm + part_rec_doubles<R, RS>(rec_cap);
+    double* fac = acc + 5 * kPart;
+    // 1. loads, all clamped into the part so that they issue without branches
+    const int last = 5 * P.cnt - 1;
+    const size_t base = (size_t)P.n0 * 5;
+    int nd[NPT];
+    unsigned code[EPT];
+    R w0[EPT], w1[EPT], w2[EPT];
+    double x[FL], o[FL], U[NPT][5];
+    const int hmax = max(P.nh - 1, 0);
+#pragma unroll
+    for (int k = 0; k < NPT; k++) nd[k] = halo[P.h0 + min(t + k * T, hmax)];
+#pragma unroll
+    for (int i = 0; i < FL; i++) x[i] = vin[base + min(t + i * T, last)];
+    part_load_edges<R, T, EPT>(P, ecode, ew, nloc, t, code, w0, w1, w2);
+    const int own = P.n0 + min(t, max(P.cnt - 1, 0));
+    const double vs = a.rk == 0 ? a.vol[own] : a.sf[own];
+    const int q0 = a.bptr ? a.bptr[own] : 0, q1 = a.bptr ? a.bptr[own + 1] : 0;
+    const unsigned long long slot = a.rk == 0 ? a.mslots[(size_t)seg * kMinSlots + t % kMinSlots] : kMinEmpty;
+#pragma unroll
+    for (int k = 0; k < NPT; k++) {
+        part_ready(nd[k]);
+#pragma unroll
+        for (int v = 0; v < 5; v++) U[k][v] = vin[(size_t)nd[k] * 5 + v];
+    }
+#pragma unroll
+    for (int i = 0; i < FL; i++) o[i] = a.rk == 0 ? x[i] : a.old[base + min(t + i * T, last)];
+    // 2. records and accumulators into LDS
+#pragma unroll
+    for (int i = 0; i < FL; i++) {
+        const int j = t + i * T;
+        if (j <= last) {
+            rec[ST == 5 ? j : j + j / 5] = (R)x[i];
+            acc[j] = fresh ? 0.0 : a.flux[base + j];
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < NPT; k++)
+        if (t + k * T < P.nh) {
+            R* r = rec + (P.cnt + t + k * T) * ST;
+#pragma unroll
+            for (int v = 0; v < 5; v++) r[v] = (R)U[k][v];
+            if constexpr (RS == 6) r[5] = part_speed<R>(r[0], r[1], r[2], r[3], r[4]);
+        }
+    __syncthreads();
+    if constexpr (RS == 6) {
+        if (t < P.cnt) {
+            R* r = rec + t * ST;
+            r[5] = part_speed<R>(r[0], r[1], r[2], r[3], r[4]);
+        }
+        __syncthreads();
+    }
+    // 3. edges
+    part_edges<R, EPT, COLOURED, RS, true>(P, rec, acc, code, w0, w1, w2, (R)k0.sc);
     if (halt) return false;
-    // the minimum dt after the edge phase (which writes only LDS), before any
-    // update: fewer live registers through the edge phase
+    // 4. the owned nodes' boundary increments and step factors
     double mdt = 0.0;
     if (a.rk == 0) {
-        mdt = stage_min_dt<T>(a, seg, pseg ? p == pfirst[seg] : p == 0);
+        mdt = stage_min_dt(a, seg, slot, pseg ? p == pfirst[seg] : p == 0);
         if (mdt < 0.0 && a.status) return false;
     }
+    if (t < P.cnt) {
+        if (q0 < q1) {
+            double f[5], u[5];
+#pragma unroll
+            for (int v = 0; v < 5; v++) {
+                f[v] = acc[t * 5 + v];
+                u[v] = sizeof(R) == sizeof(double) ? (double)rec[t * ST + v] : vin[base + t * 5 + v];
+            }
+            stage_bnd(a, a.kseg ? a.kseg[seg] : k0, u, q0, q1, f);
+#pragma unroll
+            for (int v = 0; v < 5; v++) acc[t * 5 + v] = f[v];
+        }
+        double sfi = vs;
+        if (a.rk == 0) {
+            sfi = mdt / vs;
+            a.sf[own] = sfi;
+        }
+        fac[t] = sfi / (double)(3 + 1 - a.rk);
+    }
+    __syncthreads();
+    // 5. update, residual and flux reset over the run
     double s = 0.0;
     int nb = 0;
-    if (t < P.cnt) {
-        double f[5];
 #pragma unroll
-        for (int v = 0; v < 5; v++) f[v] = acc[t * 5 + v];
-        stage_node(a, k0, seg, i, vin, f, mdt, o, vs, q0, q1, s, nb);
+    for (int i = 0; i < FL; i++) {
+#pragma clang fp contract(off)
+        const int j = t + i * T;
+        if (j <= last) {
+            const double u = o[i] + fac[j / 5] * acc[j];
+            a.var[base + j] = u;
+            if (a.zero_flux) a.flux[base + j] = 0.0;
+            if (a.res) {
+                const double r = u - o[i];
+                s += r * r;
+                nb += (isnan(u) || isinf(u)) ? 1 : 0;
+                a.res[base + j] = r;
+            }
+        }
     }
     stage_sums<T>(a, p, s, nb);
     return true;

@@ -102,6 +102,7 @@ struct InvPlan {
     int pt_parts = 0;            // 0 = not available
     long long pt_nloc = 0;       // local edges over all parts
     int pt_rec_cap = 0;          // max staged nodes (owned + halo) of one part
+    int pt_halo_cap = 0;         // max halo nodes of one part
     int pt_rec_med = 0;          // median staged nodes of a part
     int pt_rs = 6;               // values per FP64 LDS record (6, or 5: see build_partplan)
     std::vector<PartInfo> h_pt_info;   // host copy of the parts
@@ -1060,7 +1061,7 @@ static int build_partplan(InvPlan& P, op_map m, const std::vector<int>& ptr, con
     std::vector<PartInfo> parts;
     std::vector<int> halo, eid;
     std::vector<unsigned> code;
-    int rec_cap = 0, max_ne = 0, max_col = 0;
+    int rec_cap = 0, halo_cap = 0, max_ne = 0, max_col = 0;
     for (auto& o : outs) {
         if (!o.err.empty()) return fail("%s", o.err.c_str());
         for (PartInfo pi : o.parts) {
@@ -1068,6 +1069,7 @@ static int build_partplan(InvPlan& P, op_map m, const std::vector<int>& ptr, con
             pi.e0 += (int)code.size();
             parts.push_back(pi);
             rec_cap = std::max(rec_cap, pi.cnt + pi.nh);
+            halo_cap = std::max(halo_cap, pi.nh);
             max_ne = std::max(max_ne, pi.ne);
             max_col = std::max(max_col, pi.ncol);
         }
@@ -1080,7 +1082,8 @@ static int build_partplan(InvPlan& P, op_map m, const std::vector<int>& ptr, con
     long long covered = 0;
     for (size_t i = 0; i < parts.size(); i++) {
         const PartInfo& pi = parts[i];
-        if (pi.cnt > kPart || pi.cnt + pi.nh > kPartSlots) return fail("internal error: part plan part too large");
+        if (pi.cnt < 1 || pi.cnt > kPart || pi.cnt + pi.nh > kPartSlots)
+            return fail("internal error: part plan part of %d + %d nodes", pi.cnt, pi.nh);
         if (i && pi.n0 != parts[i - 1].n0 + parts[i - 1].cnt) return fail("internal error: parts not contiguous");
         covered += pi.cnt;
         for (int j = 0; j < pi.ne; j++) {
@@ -1111,6 +1114,7 @@ static int build_partplan(InvPlan& P, op_map m, const std::vector<int>& ptr, con
     P.pt_gen = ++gen;
     P.pt_nloc = (long long)eid.size();
     P.pt_rec_cap = rec_cap;
+    P.pt_halo_cap = halo_cap;
     {
         std::vector<int> r(parts.size());
         for (size_t i = 0; i < parts.size(); i++) r[i] = parts[i].cnt + parts[i].nh;
@@ -1473,6 +1477,8 @@ static int launch_part_rs(bool coloured, const InvPlan& P, const Real* w, size_t
                           const int* status, int fresh, const PartStage* st)
 {
     if (st) {
+        // records, accumulators and one step factor per owned node
+        lds = sizeof(double) * (part_rec_doubles<Real, RS>(P.pt_rec_cap) + 6 * (size_t)kPart);
         const int pw = 8 * ((R.n_cu * P.pt_persist + 7) / 8);    // persistent grid: a multiple of the 8 XCDs
         if (P.pt_persist > 0 && pw < P.pt_parts) {
             if (coloured)
@@ -1518,7 +1524,7 @@ static int launch_part_t(bool coloured, const InvPlan& P, const Real* w, size_t 
         if (P.pt_rs == 5 || st)
             return launch_part_rs<Real, T, EPT, NPT, 5>(coloured, P, w, lds, var, flux, status, fresh, st);
     }
-    return launch_part_rs<Real, T, EPT, NPT, (sizeof(Real) == sizeof(float) ? kPRec32 : kPRec)>(coloured, P, w, lds, var, flux, status, fresh,
+    return launch_part_rs<Real, T, EPT, NPT, kPRec>(coloured, P, w, lds, var, flux, status, fresh,
                                                                     st);
 }
 
@@ -1530,7 +1536,8 @@ static int launch_part_e(bool coloured, const InvPlan& P, const Real* w, size_t 
 {
     constexpr int kSmall = (512 + T - 1) / T, kLarge = (768 + T - 1) / T;
     static_assert(kPartSlots <= kLarge * T, "staged nodes exceed the kernel's registers");
-    if (P.pt_rec_cap <= kSmall * T)
+    // the kernel with the fused stage gathers only the halo node by node
+    if ((st ? P.pt_halo_cap : P.pt_rec_cap) <= kSmall * T)
         return launch_part_t<Real, T, EPT, kSmall>(coloured, P, w, lds, var, flux, status, fresh, st);
     return launch_part_t<Real, T, EPT, kLarge>(coloured, P, w, lds, var, flux, status, fresh, st);
 }
@@ -1591,10 +1598,9 @@ static int launch_flux_stage(int variant, op_map map, const PartStage& st, int f
     if (!(part_variant(variant) || mixed_variant(variant)) || P.pt_parts == 0)
         return fail("edge-flux variant %d has no part plan for map %s", variant, map->name);
     if (mixed_variant(variant))
-        return launch_part<float>(variant == MGCFD_FLUX_MIXED_COLOURED, P, P.d_pt_w32, P.pt_lds32, nullptr, nullptr,
+        return launch_part<float>(variant == MGCFD_FLUX_MIXED_COLOURED, P, P.d_pt_w32, 0, nullptr, nullptr,
                                   st.a->status, fresh, &st);
-    const size_t lds5 = sizeof(double) * ((size_t)P.pt_rec_cap * 5 + (size_t)kPart * 5);   // 40-byte records
-    return launch_part<double>(variant == MGCFD_FLUX_PART_COLOURED, P, P.d_pt_w, lds5, nullptr, nullptr,
+    return launch_part<double>(variant == MGCFD_FLUX_PART_COLOURED, P, P.d_pt_w, 0, nullptr, nullptr,
                                st.a->status, fresh, &st);
 }
 
