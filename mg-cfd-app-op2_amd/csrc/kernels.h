@@ -30,7 +30,6 @@ constexpr double kGamma = 1.4;
 constexpr int kBlock = 256;
 constexpr int kWave = 64;
 constexpr int kPart = 256;       // nodes per flux workgroup (one mesh part)
-constexpr int kRec = 12;         // doubles per staged node record in LDS
 
 struct Consts {
     double sc;          // smoothing_coefficient
@@ -223,16 +222,20 @@ __device__ __forceinline__ int word_or_zero(const int* base, int i) { return *(b
 __device__ __forceinline__ int status_of(const int* status) { return word_or_zero(status, 0); }
 
 // ------------------------------------------------------------------------
-// Edge flux, blocked gather (default).  Workgroup b owns the nodes
-// [bnode.x, bnode.x + bnode.y) of one compact mesh part; inside a part the
-// nodes are ordered by decreasing degree.
-//  1. Stage: thread t evaluates the thermodynamic state of owned node t and
-//     of halo node t (neighbours owned by other parts, at most kPart per
-//     block) and stores both as kRec-double records in LDS.
+// Edge flux, blocked gather (default).  A workgroup owns the nodes
+// [n0, n0 + cnt) of one compact mesh part; inside a part the nodes are ordered
+// by decreasing degree.
+//  1. Stage: the owned nodes' states arrive as one run of 5 * cnt doubles
+//     (consecutive lanes, consecutive doubles), the halo (neighbours owned by
+//     other parts) node by node, up to NH per thread.  Each staged node's
+//     velocity, speed and speed of sound are formed once and kept with its
+//     conserved variables as kGRec doubles in LDS.  The pressure is formed
+//     again per incidence: 9 operations, against 8 bytes of every record,
+//     which at 80 bytes keep three workgroups of a 300K-node level on a CU.
 //  2. Walk: thread t adds, in the reference's edge order, the increment of
 //     each of its node's edges, reading the other endpoint from LDS.  The
 //     k-th incidences of all threads of a block are stored contiguously
-//     (jagged-diagonal order: jbase + jpref[k] + t), so the per-incidence
+//     (jagged-diagonal order: j0 + jpref[k] + t), so the per-incidence
 //     loads {LDS slot | b-role << 31} and the weight components w0 | w1 | w2
 //     (SoA) are coalesced.  They are double-buffered in registers: chunks
 //     of CH incidences, the first in flight with the staging loads, chunk
@@ -240,29 +243,53 @@ __device__ __forceinline__ int status_of(const int* status) { return word_or_zer
 //     reference's expression (flux.h:48-50).
 // Every node sums its edges in OP2's sequential order; with EXACT (no FMA
 // contraction, true divisions) the result is bitwise the reference's.
-// Deterministic, no atomics, one launch, one barrier.
+// Deterministic, no atomics, one launch.  Bound by the incidences' bytes on
+// large levels (28 per incidence, two incidences per edge) and by each
+// thread's serial walk on small ones.  930K-edge flux 35.0 us with 96-byte
+// records and at most 256 halo nodes per block, 27.5 us now; cycle of a
+// 300K-node solve 837 -> 572 us, 1M nodes 2259 -> 1341 us.
 // ------------------------------------------------------------------------
+constexpr int kGRec = 10;        // doubles per record {rho, mx, my, mz, E, ux, uy, uz, |u|, c}
+
+struct BlkInfo {
+    int n0, cnt;    // owned nodes [n0, n0 + cnt)
+    int h0, nh;     // halo ids halo[h0 .. h0 + nh)
+    int j0, p0;     // first jagged entry; start of the diagonal offsets in jpref
+    int pad0, pad1;
+};
+
+// The derived half of a record from its conserved variables r[0..4].
 template <bool EXACT>
-__device__ __forceinline__ void stage_record(double* rec, const double U[5])
+__device__ __forceinline__ void derive_record(double* r)
 {
+    double U[5];
+#pragma unroll
+    for (int v = 0; v < 5; v++) U[v] = r[v];
     Th th;
     thermo<EXACT>(U, th);
-    double2* r = reinterpret_cast<double2*>(rec);
-    r[0] = make_double2(th.rho, th.mx);
-    r[1] = make_double2(th.my, th.mz);
-    r[2] = make_double2(th.E, th.ux);
-    r[3] = make_double2(th.uy, th.uz);
-    r[4] = make_double2(th.p, th.speed);
-    r[5] = make_double2(th.c, 0.0);
+    r[5] = th.ux; r[6] = th.uy; r[7] = th.uz; r[8] = th.speed; r[9] = th.c;
+}
+
+__device__ __forceinline__ double pressure_exact(const Th& t)
+{
+#pragma clang fp contract(off)
+    const double ssq = t.ux * t.ux + t.uy * t.uy + t.uz * t.uz;
+    return (kGamma - 1.0) * (t.E - 0.5 * t.rho * ssq);
+}
+__device__ __forceinline__ double pressure_fast(const Th& t)
+{
+    const double ssq = t.ux * t.ux + t.uy * t.uy + t.uz * t.uz;
+    return (kGamma - 1.0) * (t.E - 0.5 * t.rho * ssq);
 }
 
 template <bool EXACT>
 __device__ __forceinline__ void load_record(const double* rec, Th& t)
 {
     const double2* r = reinterpret_cast<const double2*>(rec);
-    const double2 a = r[0], b = r[1], c = r[2], d = r[3], e = r[4], f = r[5];
-    t.rho = a.x; t.mx = a.y; t.my = b.x; t.mz = b.y; t.E = c.x; t.ux = c.y;
-    t.uy = d.x; t.uz = d.y; t.p = e.x; t.speed = e.y; t.c = f.x;
+    const double2 a = r[0], b = r[1], c = r[2], d = r[3], e = r[4];
+    t.rho = a.x; t.mx = a.y; t.my = b.x; t.mz = b.y; t.E = c.x;
+    t.ux = c.y; t.uy = d.x; t.uz = d.y; t.speed = e.x; t.c = e.y;
+    t.p = EXACT ? pressure_exact(t) : pressure_fast(t);
     flux_tensor<EXACT>(t);
 }
 
@@ -302,7 +329,7 @@ __device__ __forceinline__ void walk_chunk(const IncChunk<CH>& c, int q0, int de
         if (q0 + i < deg) {
             const unsigned r = c.r[i];
             Th th;
-            load_record<EXACT>(sm + (int)(r & 0x7fffffffu) * kRec, th);
+            load_record<EXACT>(sm + (int)(r & 0x7fffffffu) * kGRec, th);
             double ewt;
             {
 #pragma clang fp contract(off)
@@ -323,52 +350,91 @@ __device__ __forceinline__ void walk_chunk(const IncChunk<CH>& c, int q0, int de
     }
 }
 
-template <bool EXACT, int CH>
-__global__ __launch_bounds__(kBlock) void k_flux_blocked_pf(
-    const int2* __restrict__ bnode, const int* __restrict__ hptr, const int* __restrict__ halo,
-    const int* __restrict__ jbase, const int* __restrict__ pbase, const int* __restrict__ jpref,
-    const int* __restrict__ nptr, const unsigned* __restrict__ jslot, const double* __restrict__ jw, int nent,
-    const double* __restrict__ var, double* __restrict__ flux, Consts k, const int* __restrict__ status, int fresh)
+// The jagged plan of one map, as the gather kernels take it.
+struct GatherPlan {
+    const BlkInfo* blk;
+    const int* halo;
+    const int* jpref;
+    const int* nptr;            // CSR over every node: its degree
+    const unsigned* jslot;
+    const double* jw;           // w0 | w1 | w2, nent entries each
+    int nent;
+};
+
+// Steps 1 and 2 for one block: acc holds the thread's node's start value and
+// receives its edge flux (threads t < cnt); o: the node's own state.  LDS: one
+// record per staged node.  Ends without a barrier.
+template <bool EXACT, int CH, int NH>
+__device__ __forceinline__ void gather_block(const GatherPlan& G, const BlkInfo& B, const double* __restrict__ vin,
+                                             double sc, double* sm, double acc[5], Th& o)
+{
+    constexpr int FL = 5 * kPart / kBlock;
+    const int t = threadIdx.x;
+    const bool own = t < B.cnt;
+    const int last = 5 * B.cnt - 1, hmax = max(B.nh - 1, 0);
+    const size_t base = (size_t)B.n0 * 5;
+    int hn[NH];
+    double x[FL], U[NH][5];
+#pragma unroll
+    for (int k = 0; k < NH; k++) hn[k] = G.halo[B.h0 + min(t + k * kBlock, hmax)];
+#pragma unroll
+    for (int i = 0; i < FL; i++) x[i] = vin[base + min(t + i * kBlock, last)];
+    const int nd = B.n0 + min(t, B.cnt - 1);
+    const int deg = own ? G.nptr[nd + 1] - G.nptr[nd] : 0;
+    const int jb = B.j0 + t;
+    const int* jp = G.jpref + B.p0;
+    IncChunk<CH> A, C;
+    load_chunk<CH>(A, 0, deg, jb, jp, G.jslot, G.jw, G.nent);
+#pragma unroll
+    for (int k = 0; k < NH; k++)
+#pragma unroll
+        for (int v = 0; v < 5; v++) U[k][v] = vin[(size_t)hn[k] * 5 + v];
+#pragma unroll
+    for (int i = 0; i < FL; i++) {
+        const int j = t + i * kBlock;
+        if (j <= last) sm[j + (j / 5) * (kGRec - 5)] = x[i];
+    }
+#pragma unroll
+    for (int k = 0; k < NH; k++)
+        if (t + k * kBlock < B.nh) {
+            double* r = sm + (B.cnt + t + k * kBlock) * kGRec;
+#pragma unroll
+            for (int v = 0; v < 5; v++) r[v] = U[k][v];
+            derive_record<EXACT>(r);
+        }
+    __syncthreads();
+    if (own) derive_record<EXACT>(sm + t * kGRec);
+    __syncthreads();
+    if (!own) return;
+    load_record<EXACT>(sm + t * kGRec, o);
+    for (int q0 = 0; q0 < deg; q0 += 2 * CH) {
+        load_chunk<CH>(C, q0 + CH, deg, jb, jp, G.jslot, G.jw, G.nent);
+        walk_chunk<EXACT, CH>(A, q0, deg, sm, o, sc, acc);
+        if (q0 + CH >= deg) break;
+        load_chunk<CH>(A, q0 + 2 * CH, deg, jb, jp, G.jslot, G.jw, G.nent);
+        walk_chunk<EXACT, CH>(C, q0 + CH, deg, sm, o, sc, acc);
+    }
+}
+
+template <bool EXACT, int CH, int NH>
+__global__ __launch_bounds__(kBlock) void k_flux_blocked_pf(GatherPlan G, const double* __restrict__ var,
+                                                            double* __restrict__ flux, Consts k,
+                                                            const int* __restrict__ status, int fresh)
 {
     extern __shared__ double sm[];
     if (halted(status)) return;
-    const int b = xcd_block(), t = threadIdx.x;
-    const int h0 = hptr[b], nh = hptr[b + 1] - h0;
-    const int hn = (t < nh) ? halo[h0 + t] : -1;
-    const int2 bn = bnode[b];
-    const bool own = t < bn.y;
-    const int nd = bn.x + t;
-    int deg = 0;
-    if (own) deg = nptr[nd + 1] - nptr[nd];
-    const int jb = jbase[b] + t;
-    const int* jp = jpref + pbase[b];
-    IncChunk<CH> A, B;
-    load_chunk<CH>(A, 0, deg, jb, jp, jslot, jw, nent);
-    double uo[5], uh[5], acc[5];
-    if (own) {
-        load5(var, nd, uo);
-        if (fresh) {
+    const BlkInfo B = G.blk[xcd_block()];
+    const int t = threadIdx.x;
+    double acc[5];
+    if (fresh) {
 #pragma unroll
-            for (int v = 0; v < 5; v++) acc[v] = 0.0;
-        } else {
-            load5(flux, nd, acc);
-        }
+        for (int v = 0; v < 5; v++) acc[v] = 0.0;
+    } else {
+        load5(flux, B.n0 + min(t, B.cnt - 1), acc);
     }
-    if (hn >= 0) load5(var, hn, uh);
-    if (own) stage_record<EXACT>(sm + t * kRec, uo);
-    if (hn >= 0) stage_record<EXACT>(sm + (kPart + t) * kRec, uh);
-    __syncthreads();
-    if (!own) return;
     Th o;
-    load_record<EXACT>(sm + t * kRec, o);
-    for (int q0 = 0; q0 < deg; q0 += 2 * CH) {
-        load_chunk<CH>(B, q0 + CH, deg, jb, jp, jslot, jw, nent);
-        walk_chunk<EXACT, CH>(A, q0, deg, sm, o, k.sc, acc);
-        if (q0 + CH >= deg) break;
-        load_chunk<CH>(A, q0 + 2 * CH, deg, jb, jp, jslot, jw, nent);
-        walk_chunk<EXACT, CH>(B, q0 + CH, deg, sm, o, k.sc, acc);
-    }
-    store5(flux, nd, acc);
+    gather_block<EXACT, CH, NH>(G, B, var, k.sc, sm, acc, o);
+    if (t < B.cnt) store5(flux, B.n0 + t, acc);
 }
 
 // Per-incidence weight components (SoA) of k_flux_blocked_pf.

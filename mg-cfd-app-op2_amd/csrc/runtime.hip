@@ -84,11 +84,8 @@ struct InvPlan {
     int bk_blocks = 0;           // 0 = not available
     int bk_entries = 0;          // jagged-diagonal entries (= incidences)
     size_t bk_lds = 0;           // dynamic LDS bytes per workgroup
-    int2* d_bk_bnode = nullptr;  // {first node, count} per block
-    int* d_bk_hptr = nullptr;    // blocks + 1
+    BlkInfo* d_bk_info = nullptr;
     int* d_bk_halo = nullptr;    // halo node ids per block
-    int* d_bk_jbase = nullptr;   // first jagged entry of each block
-    int* d_bk_pbase = nullptr;   // start of each block's diagonal offsets in d_bk_jpref
     int* d_bk_jpref = nullptr;   // per block: offset of diagonal k (k = 0..max degree)
     unsigned* d_bk_jslot = nullptr;   // per entry: LDS slot of the other endpoint | b-role << 31
     int* d_bk_eid = nullptr;     // per entry: internal edge id (-1 = padding)
@@ -97,7 +94,7 @@ struct InvPlan {
                                  // counts targets only when some node has no incidence)
     const void* bk_wdat = nullptr;    // weight dat the packed weights came from
     unsigned bk_wver = 0;
-    int bk_max_halo = 0;
+    int bk_max_halo = 0, bk_rec_cap = 0;   // largest halo, and largest staged node count, of a block
     // part plan (edge-parallel flux over mesh parts, k_flux_part)
     int pt_parts = 0;            // 0 = not available
     long long pt_nloc = 0;       // local edges over all parts
@@ -738,13 +735,15 @@ static int upload_dat(op_dat d)
 #define TRY(x) do { if (int rc_ = (x)) return rc_; } while (0)
 
 // Blocked-gather plan.  Blocks are the kPart-node parts of the node order
-// (halved recursively while a part's halo exceeds kHaloCap: the kernel
-// stages one halo node per thread).  Per block: the sorted halo, and the
+// (halved recursively while a part's halo exceeds kHaloCap).  Per block: the sorted halo, and the
 // incidences of its nodes in jagged-diagonal order -- diagonal k holds the
 // k-th incidence (reference edge order) of every node with degree > k;
 // nodes are sorted by decreasing degree inside a part, so diagonal k is a
 // prefix of the block's threads.
-constexpr int kHaloCap = kPart;
+// A halo of two nodes per thread keeps nearly every part whole on the coarse
+// levels too, whose parts of 256 nodes have halos of 300 to 450: at one per
+// thread a 165K-node level's 645 parts became 3245 blocks.
+constexpr int kHaloCap = 448;
 
 // Runs f(i) for i in [0, n) on up to 16 host threads (the plan builders'
 // per-part work is independent); f must be thread-safe.
@@ -801,7 +800,7 @@ static void blocked_part(int lo0, int hi0, const std::vector<int>& ptr, const st
                 const int o = r.x;
                 const unsigned slot = (o >= lo && o < hi)
                     ? (unsigned)(o - lo)
-                    : (unsigned)(kPart + (std::lower_bound(hb.begin(), hb.end(), o) - hb.begin()));
+                    : (unsigned)(hi - lo + (std::lower_bound(hb.begin(), hb.end(), o) - hb.begin()));
                 out.jslot.push_back(slot | ((unsigned)r.y & 0x80000000u));
                 out.eid.push_back(r.y & 0x7fffffff);
                 off++;
@@ -825,22 +824,34 @@ static int build_blocked(InvPlan& P, op_map m, const std::vector<int>& ptr, cons
     const int np = (int)pb.size() - 1;
     std::vector<BlkOut> outs(std::max(np, 0));
     parallel_for(np, [&](int k) { blocked_part(pb[k], pb[k + 1], ptr, inc2, outs[k]); });
-    std::vector<int2> blocks;
-    std::vector<int> hptr{0}, halo, jbase, pbase, jpref, eid;
+    std::vector<BlkInfo> blocks;
+    std::vector<int> halo, jpref, eid;
     std::vector<unsigned> jslot;
-    int max_halo = 0;
+    int max_halo = 0, rec_cap = 0;
     for (auto& o : outs) {
         if (!o.err.empty()) return fail("%s", o.err.c_str());
         size_t hp = 0, pp = 0, ep = 0;
         for (size_t b = 0; b < o.blocks.size(); b++) {
-            blocks.push_back(o.blocks[b]);
-            jbase.push_back((int)(jslot.size() + ep));
-            pbase.push_back((int)(jpref.size() + pp));
+            BlkInfo bi{};
+            bi.n0 = o.blocks[b].x;
+            bi.cnt = o.blocks[b].y;
+            bi.h0 = (int)(halo.size() + hp);
+            bi.nh = o.nhalo[b];
+            bi.j0 = (int)(jslot.size() + ep);
+            bi.p0 = (int)(jpref.size() + pp);
+            // invariants the kernel relies on
+            if (bi.cnt < 1 || bi.cnt > kPart || bi.nh > kHaloCap) return fail("internal error: blocked plan block too large");
+            if (!blocks.empty() && bi.n0 != blocks.back().n0 + blocks.back().cnt)
+                return fail("internal error: blocks not contiguous");
+            for (int q = 0; q < o.nent[b]; q++)
+                if ((int)(o.jslot[ep + q] & 0x7fffffffu) >= bi.cnt + bi.nh)
+                    return fail("internal error: blocked plan slot out of range");
             hp += o.nhalo[b];
-            hptr.push_back((int)(halo.size() + hp));
             pp += o.npref[b];
             ep += o.nent[b];
-            max_halo = std::max(max_halo, o.nhalo[b]);
+            max_halo = std::max(max_halo, bi.nh);
+            rec_cap = std::max(rec_cap, bi.cnt + bi.nh);
+            blocks.push_back(bi);
         }
         halo.insert(halo.end(), o.halo.begin(), o.halo.end());
         jpref.insert(jpref.end(), o.jpref.begin(), o.jpref.end());
@@ -848,27 +859,17 @@ static int build_blocked(InvPlan& P, op_map m, const std::vector<int>& ptr, cons
         eid.insert(eid.end(), o.eid.begin(), o.eid.end());
         o = BlkOut();
     }
-    // invariants the kernel relies on
-    for (size_t bi = 0; bi < blocks.size(); bi++) {
-        const int nh = hptr[bi + 1] - hptr[bi];
-        if (blocks[bi].y > kPart || nh > kHaloCap) return fail("internal error: blocked plan block too large");
-        if (bi && blocks[bi].x != blocks[bi - 1].x + blocks[bi - 1].y) return fail("internal error: blocks not contiguous");
-    }
-    for (unsigned r : jslot) {
-        const unsigned sl = r & 0x7fffffffu;
-        if (sl >= (unsigned)(kPart + kHaloCap)) return fail("internal error: blocked plan slot out of range");
-    }
+    if (!blocks.empty() && blocks.back().n0 + blocks.back().cnt != m->to->size)
+        return fail("internal error: blocked plan does not cover the node set");
+    halo.push_back(0);   // pad: the kernel's clamped halo index loads stay in bounds when nh == 0
     auto up = [](auto*& d, const auto& h) -> int {
         using T = typename std::decay<decltype(h[0])>::type;
         HIPCHK(hipMalloc((void**)&d, sizeof(T) * std::max<size_t>(1, h.size())));
         if (!h.empty()) HIPCHK(hipMemcpy((void*)d, h.data(), sizeof(T) * h.size(), hipMemcpyHostToDevice));
         return 0;
     };
-    TRY(up(P.d_bk_bnode, blocks));
-    TRY(up(P.d_bk_hptr, hptr));
+    TRY(up(P.d_bk_info, blocks));
     TRY(up(P.d_bk_halo, halo));
-    TRY(up(P.d_bk_jbase, jbase));
-    TRY(up(P.d_bk_pbase, pbase));
     TRY(up(P.d_bk_jpref, jpref));
     TRY(up(P.d_bk_jslot, jslot));
     TRY(up(P.d_bk_eid, eid));
@@ -877,7 +878,8 @@ static int build_blocked(InvPlan& P, op_map m, const std::vector<int>& ptr, cons
     P.bk_blocks = (int)blocks.size();
     P.bk_entries = (int)eid.size();
     P.bk_max_halo = max_halo;
-    P.bk_lds = sizeof(double) * kRec * (size_t)(kPart + max_halo);
+    P.bk_rec_cap = rec_cap;
+    P.bk_lds = sizeof(double) * kGRec * (size_t)rec_cap;
     return 0;
 }
 
@@ -1278,9 +1280,8 @@ static int set_part_nodes(op_map m, int nodes)
 static void free_invplan(InvPlan& P)
 {
     if (P.d_nptr && P.d_nptr != P.d_ptr) hipFree(P.d_nptr);
-    for (void* p : {(void*)P.d_targets, (void*)P.d_ptr, (void*)P.d_inc2, (void*)P.d_inc1, (void*)P.d_bk_bnode,
-                    (void*)P.d_bk_hptr, (void*)P.d_bk_halo, (void*)P.d_bk_jbase, (void*)P.d_bk_pbase,
-                    (void*)P.d_bk_jpref, (void*)P.d_bk_jslot, (void*)P.d_bk_eid, (void*)P.d_bk_w3,
+    for (void* p : {(void*)P.d_targets, (void*)P.d_ptr, (void*)P.d_inc2, (void*)P.d_inc1, (void*)P.d_bk_info,
+                    (void*)P.d_bk_halo, (void*)P.d_bk_jpref, (void*)P.d_bk_jslot, (void*)P.d_bk_eid, (void*)P.d_bk_w3,
                     (void*)P.d_bk_nptr})
         if (p) hipFree(p);
     free_partplan(P);
@@ -1450,17 +1451,28 @@ static int refresh_plan_weights(int variant, InvPlan& P, op_dat w)
     return 0;
 }
 
+static GatherPlan gather_plan(const InvPlan& P)
+{
+    return GatherPlan{P.d_bk_info, P.d_bk_halo, P.d_bk_jpref, P.d_bk_nptr, P.d_bk_jslot, P.d_bk_w3, P.bk_entries};
+}
+
+template <bool EXACT, int NH>
+static int launch_blocked_nh(const InvPlan& P, op_dat var, op_dat flux, const int* status, int fresh)
+{
+    k_flux_blocked_pf<EXACT, 4, NH><<<P.bk_blocks, kBlock, P.bk_lds, cur_stream()>>>(gather_plan(P), dptr(var),
+                                                                                 dptr(flux), R.k, status, fresh);
+    return check_launch();
+}
+
+// Halo nodes per thread: one where the plan's largest halo allows it.
 static int launch_blocked_pf(bool exact, const InvPlan& P, op_dat var, op_dat flux, const int* status, int fresh)
 {
-    if (exact)
-        k_flux_blocked_pf<true, 4><<<P.bk_blocks, kBlock, P.bk_lds, cur_stream()>>>(
-            P.d_bk_bnode, P.d_bk_hptr, P.d_bk_halo, P.d_bk_jbase, P.d_bk_pbase, P.d_bk_jpref, P.d_bk_nptr, P.d_bk_jslot,
-            P.d_bk_w3, P.bk_entries, dptr(var), dptr(flux), R.k, status, fresh);
-    else
-        k_flux_blocked_pf<false, 4><<<P.bk_blocks, kBlock, P.bk_lds, cur_stream()>>>(
-            P.d_bk_bnode, P.d_bk_hptr, P.d_bk_halo, P.d_bk_jbase, P.d_bk_pbase, P.d_bk_jpref, P.d_bk_nptr, P.d_bk_jslot,
-            P.d_bk_w3, P.bk_entries, dptr(var), dptr(flux), R.k, status, fresh);
-    return check_launch();
+    static_assert(kHaloCap <= 2 * kBlock, "two halo nodes per thread");
+    if (P.bk_max_halo <= kBlock)
+        return exact ? launch_blocked_nh<true, 1>(P, var, flux, status, fresh)
+                     : launch_blocked_nh<false, 1>(P, var, flux, status, fresh);
+    return exact ? launch_blocked_nh<true, 2>(P, var, flux, status, fresh)
+                 : launch_blocked_nh<false, 2>(P, var, flux, status, fresh);
 }
 
 // The stage fused into a part kernel (k_flux_part_stage): its input state,
@@ -2028,7 +2040,7 @@ int mgcfd_plan_stats(op_map map, int* stats)
     TRY(ensure_flux_plan(map, MGCFD_FLUX_GATHER_EXACT));
     const InvPlan& P = M(map)->inv;
     stats[0] = P.bk_blocks;
-    stats[1] = kPart + P.bk_max_halo;
+    stats[1] = P.bk_rec_cap;
     stats[2] = P.bk_entries;
     stats[3] = P.max_deg;
     stats[4] = (int)P.bk_lds;
