@@ -85,6 +85,8 @@ struct InvPlan {
     int bk_entries = 0;          // jagged-diagonal entries (= incidences)
     size_t bk_lds = 0;           // dynamic LDS bytes per workgroup
     BlkInfo* d_bk_info = nullptr;
+    std::vector<int2> h_bk_node; // host copy: {first node, count} per block
+    unsigned bk_gen = 0;         // identifies the blocked plan (counted with pt_gen)
     int* d_bk_halo = nullptr;    // halo node ids per block
     int* d_bk_jpref = nullptr;   // per block: offset of diagonal k (k = 0..max degree)
     unsigned* d_bk_jslot = nullptr;   // per entry: LDS slot of the other endpoint | b-role << 31
@@ -103,7 +105,7 @@ struct InvPlan {
     int pt_rec_med = 0;          // median staged nodes of a part
     int pt_rs = 6;               // values per FP64 LDS record (6, or 5: see build_partplan)
     std::vector<PartInfo> h_pt_info;   // host copy of the parts
-    unsigned pt_gen = 0;         // identifies the part plan built last (process-wide count)
+    unsigned pt_gen = 0;         // identifies the part plan built last (g_plan_gen)
     int pt_max_ne = 0;           // max local edges of one part
     int pt_max_col = 0;
     size_t pt_lds = 0;
@@ -127,6 +129,9 @@ struct InvPlan {
     std::vector<int> h_ptr;          // host CSR over every target-set element, kept for re-planning (dim-2 maps)
     std::vector<int2> h_inc2;
 };
+
+// Blocked and part plans built so far in this process.
+static std::atomic<unsigned> g_plan_gen{0};
 
 struct MapImpl {
     bool on_device = false;
@@ -879,6 +884,8 @@ static int build_blocked(InvPlan& P, op_map m, const std::vector<int>& ptr, cons
     P.bk_entries = (int)eid.size();
     P.bk_max_halo = max_halo;
     P.bk_rec_cap = rec_cap;
+    for (const BlkInfo& bi : blocks) P.h_bk_node.push_back(make_int2(bi.n0, bi.cnt));
+    P.bk_gen = ++g_plan_gen;
     P.bk_lds = sizeof(double) * kGRec * (size_t)rec_cap;
     return 0;
 }
@@ -1112,8 +1119,7 @@ static int build_partplan(InvPlan& P, op_map m, const std::vector<int>& ptr, con
     HIPCHK(hipMalloc(&P.d_pt_w, sizeof(double) * 3 * std::max<size_t>(1, eid.size())));
     P.pt_parts = (int)parts.size();
     P.h_pt_info = parts;
-    static std::atomic<unsigned> gen{0};
-    P.pt_gen = ++gen;
+    P.pt_gen = ++g_plan_gen;
     P.pt_nloc = (long long)eid.size();
     P.pt_rec_cap = rec_cap;
     P.pt_halo_cap = halo_cap;
@@ -1600,13 +1606,45 @@ static int prepare_flux(int variant, op_map map, op_dat w)
     return 0;
 }
 
-// Edge flux of a part variant fused with a Runge-Kutta stage (device
-// multigrid driver); plans and weights come from prepare_flux.
-static bool fused_stage_variant(int v) { return part_variant(v) || mixed_variant(v); }
+// Edge flux of a gather or part variant fused with a Runge-Kutta stage
+// (device multigrid driver); plans and weights come from prepare_flux.
+static bool gather_variant(int v) { return v == MGCFD_FLUX_GATHER_EXACT || v == MGCFD_FLUX_GATHER_FAST; }
+static bool part_stage_variant(int v) { return part_variant(v) || mixed_variant(v); }
+static bool fused_stage_variant(int v) { return gather_variant(v) || part_stage_variant(v); }
+
+// Workgroups of a variant's kernel with the fused stage, and the first node
+// and node count of each.
+static int stage_blocks(int variant, const InvPlan& P) { return gather_variant(variant) ? P.bk_blocks : P.pt_parts; }
+static unsigned stage_gen(int variant, const InvPlan& P) { return gather_variant(variant) ? P.bk_gen : P.pt_gen; }
+static int2 stage_nodes(int variant, const InvPlan& P, int k)
+{
+    return gather_variant(variant) ? P.h_bk_node[k] : make_int2(P.h_pt_info[k].n0, P.h_pt_info[k].cnt);
+}
+
+template <bool EXACT, int NH>
+static int launch_gather_stage_nh(const InvPlan& P, const PartStage& st, int fresh)
+{
+    // records, then (in the same space) five fluxes and a factor per node
+    const size_t lds = std::max(P.bk_lds, sizeof(double) * 6 * (size_t)kPart);
+    k_gather_stage<EXACT, 4, NH><<<P.bk_blocks, kBlock, lds, cur_stream()>>>(gather_plan(P), st.pseg, st.pfirst,
+                                                                         st.vin, fresh, *st.a, R.k);
+    return check_launch();
+}
+
+static int launch_gather_stage(bool exact, const InvPlan& P, const PartStage& st, int fresh)
+{
+    if (P.bk_max_halo <= kBlock)
+        return exact ? launch_gather_stage_nh<true, 1>(P, st, fresh) : launch_gather_stage_nh<false, 1>(P, st, fresh);
+    return exact ? launch_gather_stage_nh<true, 2>(P, st, fresh) : launch_gather_stage_nh<false, 2>(P, st, fresh);
+}
 
 static int launch_flux_stage(int variant, op_map map, const PartStage& st, int fresh)
 {
     const InvPlan& P = M(map)->inv;
+    if (gather_variant(variant)) {
+        if (P.bk_blocks == 0) return fail("edge-flux variant %d has no blocked plan for map %s", variant, map->name);
+        return launch_gather_stage(variant == MGCFD_FLUX_GATHER_EXACT, P, st, fresh);
+    }
     if (!(part_variant(variant) || mixed_variant(variant)) || P.pt_parts == 0)
         return fail("edge-flux variant %d has no part plan for map %s", variant, map->name);
     if (mixed_variant(variant))

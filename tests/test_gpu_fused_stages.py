@@ -1,0 +1,105 @@
+"""The kernels that run a Runge-Kutta stage inside the edge flux
+(k_gather_stage, k_flux_part_stage) and the device-resident driver around
+them, at the sizes where their tiles can go wrong, against the oracle.
+
+Meshes are random graphs, whose parts have halos far larger than a box's or a
+nearest-neighbour mesh's: the blocked plan's parts of 256 nodes are split at
+its halo limit, and stage one or two halo nodes per thread.  Sizes sit at
+the edges of a part (255, 256, 257 nodes) and of several parts; degrees from
+2 to 12 per node give halos below 256, between 256 and the limit, and
+beyond it.  Every solve starts from a disturbed state and from non-zero flux
+dats, which the first cycle has to add to and leave zero.
+
+Bars as in the parity suite: FP64 variants 1e-12 relative per variable on the
+state after three cycles (the random graphs' weights are damped by 1e-7 as
+every mesh's, so a stage's rounding differences of ~1e-16 are not amplified),
+mixed precision 1e-6.
+"""
+import numpy as np
+import pytest
+
+import mgcfd
+from conftest import perturbed_state
+from oracle import Oracle
+from test_gpu_parity import MIXED_STATE_TOL, STATE_TOL, rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+def random_mesh(n, deg, seed):
+    """Two levels of n and n / 2 nodes at random points, node i of the first
+    restricting to i / 2 of the second; each level's edges are a ring, so that
+    every node has a volume, and random pairs up to 'deg' per node."""
+    rng = np.random.default_rng(seed)
+
+    def level(n, ne):
+        ring = np.arange(n)
+        a = np.concatenate([ring, rng.integers(0, n, max(0, ne - n))])
+        b = (a + np.concatenate([np.ones(n, np.int64), rng.integers(1, n, len(a) - n)])) % n
+        ne = len(a)
+        nb = max(1, n // 7)
+        return dict(coords=rng.uniform(0.0, 2.0, (n, 3)), edge_to_node=np.stack([a, b], 1).astype(np.int32),
+                    edge_weights=rng.uniform(-0.6, 0.6, (ne, 3)),
+                    bnd_to_node=rng.integers(0, n, nb).astype(np.int32),
+                    bnd_group=rng.integers(0, 9, nb).astype(np.int32), bnd_weights=rng.uniform(-0.4, 0.4, (nb, 3)))
+
+    fine, coarse = level(n, n * deg // 2), level((n + 1) // 2, n * deg // 3)
+    fine["node_to_mg_node"] = (np.arange(n) // 2).astype(np.int32)
+    return [fine, coarse]
+
+
+@pytest.fixture
+def rt():
+    r = mgcfd.Runtime()
+    r.set_flux_variant(mgcfd.FLUX_VARIANTS["gather_exact"])
+    yield r
+    r.close()
+
+
+@pytest.mark.parametrize("variant", ["gather_exact", "gather_fast", "part_coloured", "part_atomic", "mixed_coloured",
+                                     "mixed_atomic"])
+@pytest.mark.parametrize("n,deg", [(255, 4), (256, 6), (257, 6), (515, 2), (1100, 2), (1300, 4), (1500, 12)])
+def test_fused_solve(rt, n, deg, variant):
+    mesh = random_mesh(n, deg, seed=n + deg)
+    o = Oracle("orc")
+    state = perturbed_state(n, o.freestream(0.5, 3.0).ff_variable[:], seed=5)
+    flux = [1e-9 * perturbed_state(len(lv["coords"]), np.ones(5), seed=6 + l) for l, lv in enumerate(mesh)]
+
+    def after_setup(levels):
+        levels[0]["var"][:] = state
+        for l, a in enumerate(levels):
+            a["flux"][:] = flux[l]
+
+    cycles = 3
+    ref = o.solve(mesh, cycles, 0.5, 3.0, after_setup=after_setup)
+    for graph in (False, True):
+        s = mgcfd.Solver(rt, mesh, 0.5, 3.0)
+        s.setup()
+        rt.upload(s.lv[0].variables, state)
+        for l in range(2):
+            rt.upload(s.lv[l].fluxes, flux[l])
+        rt.set_flux_variant(mgcfd.FLUX_VARIANTS[variant])
+        st, rms = s.run_device(cycles, use_graph=graph)
+        assert st == ref["status"] == 0
+        tol = MIXED_STATE_TOL if variant.startswith("mixed") else STATE_TOL
+        for l in range(2):
+            err = rel_err(s.state(l), ref["levels"][l]["variables"])
+            assert err <= tol, f"level {l} graph {graph}: {err:.3e}"
+            assert not s.state(l, "fluxes").any(), f"level {l}: flux not zero after the run"
+
+
+def test_blocked_plan_keeps_parts_whole(rt):
+    """Parts with more than 256 and at most 448 halo nodes are one block each;
+    a part beyond that is split."""
+    import ctypes as C
+
+    def stats(mesh):
+        s = mgcfd.Solver(rt, mesh, 0.5, 3.0)
+        st = (C.c_int * 5)()
+        mgcfd._check(rt.L.mgcfd_plan_stats(s.lv[0].edge_to_node, st), "mgcfd_plan_stats")
+        return list(st)
+
+    whole = stats(random_mesh(1100, 2, seed=1102))
+    assert whole[0] == 5 and 512 < whole[1] <= 704 and whole[4] == 80 * whole[1]
+    split = stats(random_mesh(1500, 12, seed=1512))
+    assert split[0] > 6 and split[1] <= 704
