@@ -1489,10 +1489,12 @@ __device__ __forceinline__ double stage_factor(const StageArgs& a, int i, double
 // [base, base + last] of every [n][5] array: u = o + factor f
 // (time_stepping_kernels.h:66-86), the flux reset when asked, on the last
 // stage the residual with its square sum and NaN/Inf count.  fac, acc: the
-// nodes' factors and fluxes in LDS; o: the old state, T apart.
+// nodes' factors and fluxes in LDS; o: the old state, T apart.  The square
+// sum is formed node by node (thread t: node t), so that the reduction does
+// not depend on the number of threads.
 template <int T, int FL = (5 * kPart + T - 1) / T>
 __device__ __forceinline__ void stage_run(const StageArgs& a, size_t base, int last, const double o[FL],
-                                          const double* fac, const double* acc, double& s, int& nb)
+                                          const double* fac, double* acc, double& s, int& nb)
 {
 #pragma clang fp contract(off)
 #pragma unroll
@@ -1504,11 +1506,17 @@ __device__ __forceinline__ void stage_run(const StageArgs& a, size_t base, int l
             if (a.zero_flux) a.flux[base + j] = 0.0;
             if (a.res) {
                 const double r = u - o[i];
-                s += r * r;
                 nb += (isnan(u) || isinf(u)) ? 1 : 0;
                 a.res[base + j] = r;
+                if (a.part) acc[j] = r;      // this thread alone has read it
             }
         }
+    }
+    if (a.part) {
+        __syncthreads();
+        const int j = threadIdx.x * 5;
+        if (j <= last)
+            for (int v = 0; v < 5; v++) s += acc[j + v] * acc[j + v];
     }
 }
 

@@ -1490,44 +1490,42 @@ struct PartStage {
     const int* pfirst = nullptr;
 };
 
-template <typename Real, int T, int EPT, int NPT, int RS>
-static int launch_part_rs(bool coloured, const InvPlan& P, const Real* w, size_t lds, op_dat var, op_dat flux,
-                          const int* status, int fresh, const PartStage* st)
+template <typename Real, int T, int EPT, int NPT, int RS, bool COLOURED>
+static int launch_part_c(const InvPlan& P, const Real* w, size_t lds, op_dat var, op_dat flux, const int* status,
+                         int fresh, const PartStage* st)
 {
     if (st) {
         // records, accumulators and one step factor per owned node
         lds = sizeof(double) * (part_rec_doubles<Real, RS>(P.pt_rec_cap) + 6 * (size_t)kPart);
         const int pw = 8 * ((R.n_cu * P.pt_persist + 7) / 8);    // persistent grid: a multiple of the 8 XCDs
-        if (P.pt_persist > 0 && pw < P.pt_parts) {
-            if (coloured)
-                k_flux_part_stage_persistent<Real, T, EPT, NPT, true, RS><<<pw, T, lds, cur_stream()>>>(
+        if constexpr (T <= 512) {
+            if (P.pt_persist > 0 && pw < P.pt_parts) {
+                k_flux_part_stage_persistent<Real, T, EPT, NPT, COLOURED, RS><<<pw, T, lds, cur_stream()>>>(
                     P.d_pt_info, P.d_pt_halo, P.d_pt_code, w, P.pt_nloc, P.pt_rec_cap, st->vin, fresh, *st->a, R.k,
                     st->pseg, st->pfirst, P.pt_parts);
-            else
-                k_flux_part_stage_persistent<Real, T, EPT, NPT, false, RS><<<pw, T, lds, cur_stream()>>>(
-                    P.d_pt_info, P.d_pt_halo, P.d_pt_code, w, P.pt_nloc, P.pt_rec_cap, st->vin, fresh, *st->a, R.k,
-                    st->pseg, st->pfirst, P.pt_parts);
-            return check_launch();
+                return check_launch();
+            }
         }
-        if (coloured)
-            k_flux_part_stage<Real, T, EPT, NPT, true, RS><<<P.pt_parts, T, lds, cur_stream()>>>(
-                P.d_pt_info, st->pseg, st->pfirst, P.d_pt_halo, P.d_pt_code, w, P.pt_nloc, P.pt_rec_cap, st->vin,
-                fresh, *st->a, R.k);
-        else
-            k_flux_part_stage<Real, T, EPT, NPT, false, RS><<<P.pt_parts, T, lds, cur_stream()>>>(
-                P.d_pt_info, st->pseg, st->pfirst, P.d_pt_halo, P.d_pt_code, w, P.pt_nloc, P.pt_rec_cap, st->vin,
-                fresh, *st->a, R.k);
+        k_flux_part_stage<Real, T, EPT, NPT, COLOURED, RS><<<P.pt_parts, T, lds, cur_stream()>>>(
+            P.d_pt_info, st->pseg, st->pfirst, P.d_pt_halo, P.d_pt_code, w, P.pt_nloc, P.pt_rec_cap, st->vin, fresh,
+            *st->a, R.k);
         return check_launch();
     }
-    if (coloured)
-        k_flux_part<Real, T, EPT, NPT, true, RS><<<P.pt_parts, T, lds, cur_stream()>>>(
+    if constexpr (T <= 512) {
+        k_flux_part<Real, T, EPT, NPT, COLOURED, RS><<<P.pt_parts, T, lds, cur_stream()>>>(
             P.d_pt_info, P.d_pt_halo, P.d_pt_code, w, P.pt_nloc, P.pt_rec_cap, dptr(var), dptr(flux), R.k, status,
             fresh);
-    else
-        k_flux_part<Real, T, EPT, NPT, false, RS><<<P.pt_parts, T, lds, cur_stream()>>>(
-            P.d_pt_info, P.d_pt_halo, P.d_pt_code, w, P.pt_nloc, P.pt_rec_cap, dptr(var), dptr(flux), R.k, status,
-            fresh);
-    return check_launch();
+        return check_launch();
+    }
+    return fail("internal error: edge flux with %d threads per part", T);
+}
+
+template <typename Real, int T, int EPT, int NPT, int RS>
+static int launch_part_rs(bool coloured, const InvPlan& P, const Real* w, size_t lds, op_dat var, op_dat flux,
+                          const int* status, int fresh, const PartStage* st)
+{
+    return coloured ? launch_part_c<Real, T, EPT, NPT, RS, true>(P, w, lds, var, flux, status, fresh, st)
+                    : launch_part_c<Real, T, EPT, NPT, RS, false>(P, w, lds, var, flux, status, fresh, st);
 }
 
 // Record size: FP32 records have six values; FP64 ones the plan's pt_rs in
@@ -1577,16 +1575,28 @@ static int launch_part_n(bool coloured, const InvPlan& P, const Real* w, size_t 
 // mixed precision, whose smaller register footprint lets 512 threads (8
 // waves) share one part in the edge-flux kernel, which shortens each
 // workgroup's edge phase; the kernel with the fused stage needs ~96 VGPRs
-// (its epilogue), which leaves 2 such workgroups per CU, so it runs 256
-// threads per part (5 per CU): batched solves 310 -> 323 per second.
-// The autotuner may set a plan's fused-stage kernel to 512 threads per part
-// (pt_threads), which halves each thread's edges at the cost of registers.
+// (its epilogue), which leaves 2 such workgroups per CU, so on levels that
+// fill the chip it runs 256 threads per part (5 per CU): batched solves 310 ->
+// 323 per second.
+// The autotuner may set a plan's fused-stage kernel to 256 or 512 threads per
+// part (pt_threads).
 template <typename Real>
 static int launch_part(bool coloured, const InvPlan& P, const Real* w, size_t lds, op_dat var, op_dat flux,
                        const int* status, int fresh, const PartStage* st = nullptr)
 {
     if (st) {
-        if (P.pt_threads == 512) return launch_part_n<Real, 512>(coloured, P, w, lds, var, flux, status, fresh, st);
+        // A level with few parts is one workgroup's latency: where the chip
+        // holds them all at once, more threads share a part's edges (results
+        // do not depend on it).  Stage kernel of 11-40 parts 8.1-8.9 us with
+        // 256 threads, 7.7-8.0 with 1024; 106-215 parts 9.4-9.8 -> 8.5-8.8;
+        // 317 and 434 parts 13.9 -> 12.9 with 512.  Beyond two parts per CU
+        // 256 threads are as fast (645 parts) or faster (1172 parts and up).
+        const int threads = P.pt_threads             ? P.pt_threads
+                            : P.pt_parts <= R.n_cu     ? 1024
+                            : P.pt_parts <= 2 * R.n_cu ? 512
+                                                       : 256;
+        if (threads == 1024) return launch_part_n<Real, 1024>(coloured, P, w, lds, var, flux, status, fresh, st);
+        if (threads == 512) return launch_part_n<Real, 512>(coloured, P, w, lds, var, flux, status, fresh, st);
         return launch_part_n<Real, 256>(coloured, P, w, lds, var, flux, status, fresh, st);
     }
     if constexpr (sizeof(Real) == 4) return launch_part_n<Real, 512>(coloured, P, w, lds, var, flux, status, fresh, st);

@@ -103,3 +103,25 @@ def test_blocked_plan_keeps_parts_whole(rt):
     assert whole[0] == 5 and 512 < whole[1] <= 704 and whole[4] == 80 * whole[1]
     split = stats(random_mesh(1500, 12, seed=1512))
     assert split[0] > 6 and split[1] <= 704
+
+
+@pytest.mark.parametrize("variant", ["part_coloured", "mixed_coloured"])
+@pytest.mark.parametrize("n,deg", [(257, 6), (1300, 4)])
+def test_threads_per_part_change_nothing(rt, n, deg, variant):
+    """Levels with few parts run more threads per part; a deterministic
+    variant's state and RMS history do not depend on it, bit for bit."""
+    mesh = random_mesh(n, deg, seed=n + deg)
+    got = []
+    for threads in (0, 256, 512):       # 0: by the number of parts (here 1024 threads)
+        s = mgcfd.Solver(rt, mesh, 0.5, 3.0)
+        s.setup()
+        rt.upload(s.lv[0].variables, perturbed_state(n, s.fs["ff_variable"], seed=5))
+        for l in range(2):
+            rt.map_part_config(s.lv[l].edge_to_node, 256, threads)
+        rt.set_flux_variant(mgcfd.FLUX_VARIANTS[variant])
+        st, rms = s.run_device(3)
+        assert st == 0
+        got.append((s.state(0), s.state(1), rms))
+    for other in got[1:]:
+        for a, b in zip(got[0], other):
+            assert np.array_equal(a.view(np.uint64), b.view(np.uint64))
