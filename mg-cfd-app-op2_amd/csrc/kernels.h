@@ -93,18 +93,29 @@ __device__ __forceinline__ void flux_tensor(Th& t)
 // finite (2^-500).  FP32: the hardware instructions (1 ulp).
 __device__ __forceinline__ double part_rcp(double x)
 {
+#pragma clang fp contract(off)
     const double r = __builtin_amdgcn_rcp(x);
     return fma(r, fma(-x, r, 1.0), r);
 }
 __device__ __forceinline__ double part_sqrt(double x)
 {
+#pragma clang fp contract(off)
     const double z = x + 0x1p-1000;
     const double y = __builtin_amdgcn_rsq(z);
     const double g = z * y;
     return fma(fma(-g, g, z), 0.5 * y, g);
 }
 __device__ __forceinline__ float part_rcp(float x) { return __builtin_amdgcn_rcpf(x); }
-__device__ __forceinline__ float part_sqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
+// sqrt(a b + c), the guard against 0 folded into the product.
+__device__ __forceinline__ double part_sqrt(double a, double b, double c)
+{
+#pragma clang fp contract(off)
+    const double z = fma(a, b, c + 0x1p-1000);
+    const double y = __builtin_amdgcn_rsq(z);
+    const double g = z * y;
+    return fma(fma(-g, g, z), 0.5 * y, g);
+}
+__device__ __forceinline__ float part_sqrt(float a, float b, float c) { return __builtin_amdgcn_sqrtf(fmaf(a, b, c)); }
 
 // Reference order: u = m / rho, |u|^2, p, c = sqrt(gamma p / rho).
 __device__ __forceinline__ void thermo_exact(const double* U, Th& t)
@@ -489,16 +500,30 @@ struct PState {
     R rho, mx, my, mz, E, inv, p, s;   // inv = 1 / rho, s = |u| + c
 };
 
+// The multiply-adds of the part kernels' arithmetic are written out, and
+// nothing else is contracted, so that every instantiation of a kernel (threads
+// per part, edges per thread) rounds alike: a deterministic variant's result
+// is the same bit for bit whichever one a level's size selects.
+__device__ __forceinline__ double part_fma(double a, double b, double c) { return fma(a, b, c); }
+__device__ __forceinline__ float part_fma(float a, float b, float c) { return fmaf(a, b, c); }
+template <typename R>
+__device__ __forceinline__ R part_dot(R a0, R a1, R a2, R b0, R b1, R b2)
+{
+#pragma clang fp contract(off)
+    return part_fma(a2, b2, part_fma(a1, b1, a0 * b0));
+}
+
 // The derived part of an endpoint from its conserved variables: 1 / rho,
 // the pressure and (SPEED) the wave speed |u| + c, with the kinetic energy
 // taken from |m|^2 / rho so that no velocity components are formed.
 template <bool SPEED, typename R>
 __device__ __forceinline__ void part_derive(PState<R>& t)
 {
+#pragma clang fp contract(off)
     t.inv = part_rcp(t.rho);
-    const R k = (t.mx * t.mx + t.my * t.my + t.mz * t.mz) * t.inv;     // rho |u|^2
-    t.p = R(kGamma - 1.0) * (t.E - R(0.5) * k);
-    if constexpr (SPEED) t.s = part_sqrt(k * t.inv) + part_sqrt(R(kGamma) * t.p * t.inv);
+    const R k = part_dot(t.mx, t.my, t.mz, t.mx, t.my, t.mz) * t.inv;     // rho |u|^2
+    t.p = R(kGamma - 1.0) * part_fma(R(-0.5), k, t.E);
+    if constexpr (SPEED) t.s = part_sqrt(k, t.inv, R(0)) + part_sqrt(R(kGamma) * t.p, t.inv, R(0));
 }
 
 // Wave speed |u| + c of a node state, computed once per staged node and kept
@@ -526,14 +551,15 @@ template <typename R, typename O>
 __device__ __forceinline__ void part_increment(const PState<R>& a, const PState<R>& b, R f0, R f1, R f2, R sc,
                                                O inc[5])
 {
-    const R factor = -sc * part_sqrt(f0 * f0 + f1 * f1 + f2 * f2) * (a.s + b.s);
-    const R fa = f0 * a.mx + f1 * a.my + f2 * a.mz, fb = f0 * b.mx + f1 * b.my + f2 * b.mz;
+#pragma clang fp contract(off)
+    const R factor = -sc * part_sqrt(f2, f2, part_fma(f1, f1, f0 * f0)) * (a.s + b.s);
+    const R fa = part_dot(f0, f1, f2, a.mx, a.my, a.mz), fb = part_dot(f0, f1, f2, b.mx, b.my, b.mz);
     const R va = fa * a.inv, vb = fb * b.inv, ps = a.p + b.p;
-    inc[0] = (O)(factor * (a.rho - b.rho) + (fa + fb));
-    inc[1] = (O)(factor * (a.mx - b.mx) + (va * a.mx + (vb * b.mx + f0 * ps)));
-    inc[2] = (O)(factor * (a.my - b.my) + (va * a.my + (vb * b.my + f1 * ps)));
-    inc[3] = (O)(factor * (a.mz - b.mz) + (va * a.mz + (vb * b.mz + f2 * ps)));
-    inc[4] = (O)(factor * (a.E - b.E) + (va * (a.E + a.p) + vb * (b.E + b.p)));
+    inc[0] = (O)part_fma(factor, a.rho - b.rho, fa + fb);
+    inc[1] = (O)part_fma(factor, a.mx - b.mx, part_fma(va, a.mx, part_fma(vb, b.mx, f0 * ps)));
+    inc[2] = (O)part_fma(factor, a.my - b.my, part_fma(va, a.my, part_fma(vb, b.my, f1 * ps)));
+    inc[3] = (O)part_fma(factor, a.mz - b.mz, part_fma(va, a.mz, part_fma(vb, b.mz, f2 * ps)));
+    inc[4] = (O)part_fma(factor, a.E - b.E, part_fma(va, a.E + a.p, vb * (b.E + b.p)));
 }
 
 // Adds inc to owned endpoint a and -inc to owned endpoint b (FP64 adds; an
