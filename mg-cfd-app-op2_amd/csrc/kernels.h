@@ -106,7 +106,8 @@ __device__ __forceinline__ double part_sqrt(double x)
     return fma(fma(-g, g, z), 0.5 * y, g);
 }
 __device__ __forceinline__ float part_rcp(float x) { return __builtin_amdgcn_rcpf(x); }
-// sqrt(a b + c), the guard against 0 folded into the product.
+__device__ __forceinline__ float part_sqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
+// sqrt(a b + c), the guard against 0 folded into the sum.
 __device__ __forceinline__ double part_sqrt(double a, double b, double c)
 {
 #pragma clang fp contract(off)
@@ -115,7 +116,6 @@ __device__ __forceinline__ double part_sqrt(double a, double b, double c)
     const double g = z * y;
     return fma(fma(-g, g, z), 0.5 * y, g);
 }
-__device__ __forceinline__ float part_sqrt(float a, float b, float c) { return __builtin_amdgcn_sqrtf(fmaf(a, b, c)); }
 
 // Reference order: u = m / rho, |u|^2, p, c = sqrt(gamma p / rho).
 __device__ __forceinline__ void thermo_exact(const double* U, Th& t)
@@ -496,8 +496,14 @@ struct PartInfo {
 
 // One endpoint of an edge as the increment needs it.
 template <typename R>
-struct PState {
-    R rho, mx, my, mz, E, inv, p, s;   // inv = 1 / rho, s = |u| + c
+struct PState;
+template <>
+struct PState<double> {
+    double rho, mx, my, mz, E, inv, p, s;   // inv = 1 / rho, s = |u| + c
+};
+template <>
+struct PState<float> {
+    float rho, mx, my, mz, E, ux, uy, uz, e, p, s;   // e: internal energy (p = 0.4 e)
 };
 
 // The multiply-adds of the part kernels' arithmetic are written out, and
@@ -505,25 +511,37 @@ struct PState {
 // per part, edges per thread) rounds alike: a deterministic variant's result
 // is the same bit for bit whichever one a level's size selects.
 __device__ __forceinline__ double part_fma(double a, double b, double c) { return fma(a, b, c); }
-__device__ __forceinline__ float part_fma(float a, float b, float c) { return fmaf(a, b, c); }
-template <typename R>
-__device__ __forceinline__ R part_dot(R a0, R a1, R a2, R b0, R b1, R b2)
+__device__ __forceinline__ double part_dot(double a0, double a1, double a2, double b0, double b1, double b2)
 {
 #pragma clang fp contract(off)
     return part_fma(a2, b2, part_fma(a1, b1, a0 * b0));
 }
 
-// The derived part of an endpoint from its conserved variables: 1 / rho,
+// The derived part of an FP64 endpoint from its conserved variables: 1 / rho,
 // the pressure and (SPEED) the wave speed |u| + c, with the kinetic energy
 // taken from |m|^2 / rho so that no velocity components are formed.
-template <bool SPEED, typename R>
-__device__ __forceinline__ void part_derive(PState<R>& t)
+template <bool SPEED>
+__device__ __forceinline__ void part_derive(PState<double>& t)
 {
 #pragma clang fp contract(off)
     t.inv = part_rcp(t.rho);
-    const R k = part_dot(t.mx, t.my, t.mz, t.mx, t.my, t.mz) * t.inv;     // rho |u|^2
-    t.p = R(kGamma - 1.0) * part_fma(R(-0.5), k, t.E);
-    if constexpr (SPEED) t.s = part_sqrt(k, t.inv, R(0)) + part_sqrt(R(kGamma) * t.p, t.inv, R(0));
+    const double k = part_dot(t.mx, t.my, t.mz, t.mx, t.my, t.mz) * t.inv;     // rho |u|^2
+    t.p = (kGamma - 1.0) * part_fma(-0.5, k, t.E);
+    if constexpr (SPEED) t.s = part_sqrt(k, t.inv, 0.0) + part_sqrt(kGamma * t.p, t.inv, 0.0);
+}
+
+// The same of an FP32 endpoint, with its velocity (the FP32 increment goes
+// through both flux tensors).
+template <bool SPEED>
+__device__ __forceinline__ void part_derive(PState<float>& t)
+{
+#pragma clang fp contract(off)
+    const float inv = part_rcp(t.rho);
+    t.ux = t.mx * inv; t.uy = t.my * inv; t.uz = t.mz * inv;
+    const float ssq = fmaf(t.uz, t.uz, fmaf(t.ux, t.ux, t.uy * t.uy));
+    t.e = fmaf(-(0.5f * t.rho), ssq, t.E);
+    t.p = (float)(kGamma - 1.0) * t.e;
+    if constexpr (SPEED) t.s = part_sqrt(ssq) + part_sqrt((float)kGamma * t.p * inv);
 }
 
 // Wave speed |u| + c of a node state, computed once per staged node and kept
@@ -537,29 +555,52 @@ __device__ __forceinline__ R part_speed(R rho, R mx, R my, R mz, R E)
     return t.s;
 }
 
-// Increment of node a for edge (a, b) in the fast form (FP64 or FP32
-// arithmetic); node b gains -inc.  (f0, f1, f2) = -w / 2, the packed weights,
-// so |w| / 2 is |f| and the dissipation factor -|w| sc (s_a + s_b) / 2 is
-// -|f| sc (s_a + s_b).  The convective part is taken along the face: with
-// v = (m . f) / rho of each endpoint, F f = {m . f, m v + p f, (E + p) v},
-// which needs no flux tensor.  The edge phase is bound by FP64 issue once a
-// part's data is staged: 94 FP64 instructions per edge with the wave speeds
-// formed here (40-byte records), against 136 with the tensors of both
-// endpoints.  930K-edge flux 19.1 -> 17.7 us, coloured 23.3 -> 22.4 us, cycle
-// of a 1M-node solve 946 -> 908 us.
-template <typename R, typename O>
-__device__ __forceinline__ void part_increment(const PState<R>& a, const PState<R>& b, R f0, R f1, R f2, R sc,
-                                               O inc[5])
+// Increment of node a for edge (a, b); node b gains -inc.  (f0, f1, f2) =
+// -w / 2, the packed weights, so |w| / 2 is |f| and the dissipation factor
+// -|w| sc (s_a + s_b) / 2 is -|f| sc (s_a + s_b).  FP64: the convective part is
+// taken along the face: with v = (m . f) / rho of each endpoint, F f =
+// {m . f, m v + p f, (E + p) v}, which needs no flux tensor.  The edge phase is
+// bound by FP64 issue once a part's data is staged: 94 FP64 instructions per
+// edge with the wave speeds formed here (40-byte records), against 136 with
+// the tensors of both endpoints: 930K-edge flux 18.5 -> 17.8 us, cycle of a
+// 1M-node solve 946 -> 908 us.
+__device__ __forceinline__ void part_increment(const PState<double>& a, const PState<double>& b, double f0, double f1,
+                                               double f2, double sc, double inc[5])
 {
 #pragma clang fp contract(off)
-    const R factor = -sc * part_sqrt(f2, f2, part_fma(f1, f1, f0 * f0)) * (a.s + b.s);
-    const R fa = part_dot(f0, f1, f2, a.mx, a.my, a.mz), fb = part_dot(f0, f1, f2, b.mx, b.my, b.mz);
-    const R va = fa * a.inv, vb = fb * b.inv, ps = a.p + b.p;
-    inc[0] = (O)part_fma(factor, a.rho - b.rho, fa + fb);
-    inc[1] = (O)part_fma(factor, a.mx - b.mx, part_fma(va, a.mx, part_fma(vb, b.mx, f0 * ps)));
-    inc[2] = (O)part_fma(factor, a.my - b.my, part_fma(va, a.my, part_fma(vb, b.my, f1 * ps)));
-    inc[3] = (O)part_fma(factor, a.mz - b.mz, part_fma(va, a.mz, part_fma(vb, b.mz, f2 * ps)));
-    inc[4] = (O)part_fma(factor, a.E - b.E, part_fma(va, a.E + a.p, vb * (b.E + b.p)));
+    const double factor = -sc * part_sqrt(f2, f2, part_fma(f1, f1, f0 * f0)) * (a.s + b.s);
+    const double fa = part_dot(f0, f1, f2, a.mx, a.my, a.mz), fb = part_dot(f0, f1, f2, b.mx, b.my, b.mz);
+    const double va = fa * a.inv, vb = fb * b.inv, ps = a.p + b.p;
+    inc[0] = part_fma(factor, a.rho - b.rho, fa + fb);
+    inc[1] = part_fma(factor, a.mx - b.mx, part_fma(va, a.mx, part_fma(vb, b.mx, f0 * ps)));
+    inc[2] = part_fma(factor, a.my - b.my, part_fma(va, a.my, part_fma(vb, b.my, f1 * ps)));
+    inc[3] = part_fma(factor, a.mz - b.mz, part_fma(va, a.mz, part_fma(vb, b.mz, f2 * ps)));
+    inc[4] = part_fma(factor, a.E - b.E, part_fma(va, a.E + a.p, vb * (b.E + b.p)));
+}
+
+// FP32: through the flux tensors F_a + F_b (symmetric) and the energy flux.
+// FP32 issue does not bound the mixed-precision kernels (the form above gains
+// them 1%), and the tensors' rounding errors are the smaller for a uniform
+// state (8.8e-8 of the flux against 1.0e-7).
+__device__ __forceinline__ void part_increment(const PState<float>& a, const PState<float>& b, float f0, float f1,
+                                               float f2, float sc, float inc[5])
+{
+#pragma clang fp contract(off)
+    constexpr float g = (float)(kGamma - 1.0);
+    const float factor = -part_sqrt(fmaf(f2, f2, fmaf(f0, f0, f1 * f1))) * sc * (a.s + b.s);
+    const float dea = fmaf(g, a.e, a.E), deb = fmaf(g, b.e, b.E);       // E + p
+    const float sxx = fmaf(g, b.e, fmaf(b.ux, b.mx, fmaf(a.ux, a.mx, a.p)));
+    const float syy = fmaf(g, b.e, fmaf(b.uy, b.my, fmaf(a.uy, a.my, a.p)));
+    const float szz = fmaf(g, b.e, fmaf(b.uz, b.mz, fmaf(a.uz, a.mz, a.p)));
+    const float sxy = fmaf(a.ux, a.my, b.ux * b.my), sxz = fmaf(a.ux, a.mz, b.ux * b.mz);
+    const float syz = fmaf(a.uy, a.mz, b.uy * b.mz);
+    const float sdx = fmaf(a.ux, dea, b.ux * deb), sdy = fmaf(a.uy, dea, b.uy * deb);
+    const float sdz = fmaf(a.uz, dea, b.uz * deb);
+    inc[0] = fmaf(f2, a.mz + b.mz, fmaf(f1, a.my + b.my, fmaf(f0, a.mx + b.mx, factor * (a.rho - b.rho))));
+    inc[1] = fmaf(f2, sxz, fmaf(f1, sxy, fmaf(factor, a.mx - b.mx, f0 * sxx)));
+    inc[2] = fmaf(f2, syz, fmaf(f1, syy, fmaf(f0, sxy, factor * (a.my - b.my))));
+    inc[3] = fmaf(f2, szz, fmaf(f1, syz, fmaf(f0, sxz, factor * (a.mz - b.mz))));
+    inc[4] = fmaf(f2, sdz, fmaf(f1, sdy, fmaf(factor, a.E - b.E, f0 * sdx)));
 }
 
 // Adds inc to owned endpoint a and -inc to owned endpoint b (FP64 adds; an
@@ -728,7 +769,7 @@ __device__ __forceinline__ void part_edges_atomic(const R* rec, double* acc, con
         const PState<R> a = part_rec_state<R, RS>(rec + (code[i] & 1023u) * part_stride<R, RS>());
         const PState<R> b = part_rec_state<R, RS>(rec + ((code[i] >> 10) & 1023u) * part_stride<R, RS>());
         R inc[5];
-        part_increment<R, R>(a, b, w0[i], w1[i], w2[i], sc, inc);
+        part_increment(a, b, w0[i], w1[i], w2[i], sc, inc);
         part_apply(acc, code[i], inc);
     }
 }
@@ -751,7 +792,7 @@ __device__ __forceinline__ void part_edges(const PartInfo& P, const R* rec, doub
                     const PState<R> a = part_rec_state<R, RS>(rec + (code[i] & 1023u) * ST);
                     const PState<R> b = part_rec_state<R, RS>(rec + ((code[i] >> 10) & 1023u) * ST);
                     R inc[5];
-                    part_increment<R, R>(a, b, w0[i], w1[i], w2[i], sc, inc);
+                    part_increment(a, b, w0[i], w1[i], w2[i], sc, inc);
                     part_apply(acc, code[i], inc);
                 }
             __syncthreads();
@@ -763,7 +804,7 @@ __device__ __forceinline__ void part_edges(const PartInfo& P, const R* rec, doub
             if (code[i]) {
                 const PState<R> a = part_rec_state<R, RS>(rec + (code[i] & 1023u) * ST);
                 const PState<R> b = part_rec_state<R, RS>(rec + ((code[i] >> 10) & 1023u) * ST);
-                part_increment<R, R>(a, b, w0[i], w1[i], w2[i], sc, inc[i]);
+                part_increment(a, b, w0[i], w1[i], w2[i], sc, inc[i]);
             }
         for (int c = 0; c < P.ncol; c++) {
 #pragma unroll
