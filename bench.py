@@ -416,12 +416,13 @@ def pmc_dispatches(path):
 
 def cycle_windows(disp, pat):
     """The dispatches of the full multigrid cycles of one solve: the cycles
-    end with k_bump; those after the first end that follows the first
+    end with the kernel that moves the cycle counter on (the prolongation to
+    level 0, or k_bump); those after the first end that follows the first
     dispatch matching 'pat', up to the first end after its last one."""
     hits = [i for i, x in enumerate(disp) if re.search(pat, x[1])]
     if not hits:
         return None, 0
-    ends = [i for i, x in enumerate(disp) if "k_bump" in x[1] and i > hits[0]]
+    ends = [i for i, x in enumerate(disp) if re.search(r"k_bump|k_down_mg<\w+, true>", x[1]) and i > hits[0]]
     last = next(i for i in ends if i > hits[-1])
     ends = [i for i in ends if i <= last]
     return disp[ends[0] + 1:last + 1], len(ends) - 1

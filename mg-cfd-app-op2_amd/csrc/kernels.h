@@ -1195,12 +1195,12 @@ struct MinPub {
     unsigned long long* slots;  // kMinSlots per segment
 };
 
-// m: the workgroup's minimum (valid in thread 0).
-__device__ __forceinline__ void min_publish(const MinPub& p, int seg, double m)
+// m: the minimum of block b of the level (valid in thread 0).
+__device__ __forceinline__ void min_publish(const MinPub& p, int seg, int b, double m)
 {
     if (threadIdx.x == 0 && p.slots) {
         const int lo = p.sblk ? p.sblk[seg] : 0;
-        atomicMin(p.slots + (size_t)seg * kMinSlots + ((int)blockIdx.x - lo) % kMinSlots, min_key(m));
+        atomicMin(p.slots + (size_t)seg * kMinSlots + (b - lo) % kMinSlots, min_key(m));
     }
 }
 
@@ -1211,13 +1211,11 @@ __device__ __forceinline__ double min_candidate(double d) { return (d < DBL_MAX)
 // calculate_dt_kernel (time_stepping_kernels.h:13-32).  With 'old' non-null
 // it also performs copy_double_kernel (copy_double_kernel.h:6-13) and with
 // 'part' non-null it emits the per-workgroup min for get_min_dt_kernel.
-// dt of node i with state U (time_stepping_kernels.h:13-32), optionally
-// saving old = U.
+// dt of node i with state U (time_stepping_kernels.h:13-32).
 __device__ __forceinline__ double calc_dt_state(int i, const double U[5], const double* __restrict__ vol,
-                                                double* __restrict__ dt, double* __restrict__ old)
+                                                double* __restrict__ dt)
 {
 #pragma clang fp contract(off)
-    if (old) store5(old, i, U);
     const double rho = U[0], E = U[4];
     const double ux = U[1] / rho, uy = U[2] / rho, uz = U[3] / rho;
     const double ssq = ux * ux + uy * uy + uz * uz;
@@ -1235,7 +1233,8 @@ __device__ __forceinline__ double calc_dt_node(int i, const double* __restrict__
 {
     double U[5];
     load5(var, i, U);
-    return calc_dt_state(i, U, vol, dt, old);
+    if (old) store5(old, i, U);
+    return calc_dt_state(i, U, vol, dt);
 }
 
 // The next smoothing step's calculate_dt + copy (time_stepping_kernels.h:13-32,
@@ -1260,7 +1259,7 @@ __global__ __launch_bounds__(kBlock) void k_calc_dt(
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     double d = DBL_MAX;
     if (i < n) d = min_candidate(calc_dt_node(i, var, vol, dt, old));
-    if (pub.slots) min_publish(pub, 0, block_min(d));
+    if (pub.slots) min_publish(pub, 0, blockIdx.x, block_min(d));
 }
 
 // get_min_dt_kernel as a standalone loop: per-workgroup min of dt.
@@ -1338,6 +1337,8 @@ struct StageArgs {
     unsigned long long* mslots;   // minimum-dt slots (kMinSlots per segment): read by the first stage,
     int nmslots;                  // reset by the second
     int* mstatus;              // abort code 1 on a negative minimum: one status, or per segment
+    int* abort_level;          // ... and the level it arose on
+    int level;
     int* zero;                 // first stage: a counter the last stage accumulates into, cleared
     const double* vol;
     double* sf;
@@ -1387,7 +1388,10 @@ __device__ __forceinline__ double stage_min_dt(const StageArgs& a, int seg, unsi
 {
     const double mdt = wave_min(min_candidate(min_unkey(slot)));
     if (first && threadIdx.x == 0) {
-        if (mdt < 0.0 && a.mstatus[seg] == 0) a.mstatus[seg] = 1;
+        if (mdt < 0.0 && a.mstatus[seg] == 0) {
+            a.mstatus[seg] = 1;
+            *a.abort_level = a.level;
+        }
         if (a.zero) *a.zero = 0;
     }
     return mdt;
@@ -1887,27 +1891,56 @@ __device__ __forceinline__ double strided_sum(const double* __restrict__ x, cons
     return (s0 + s1) + (s2 + s3);
 }
 
-// Sum of partials; *out = init + sum.  With 'hist' the L0 RMS
-// sqrt(sum / n) is stored at hist[*cycle] (euler3d.cpp:532-537) and a
-// non-zero bad-value count raises abort code 2 (euler3d.cpp:539-548).
-__global__ __launch_bounds__(kSumBlock) void k_sum_final(int np, const double* __restrict__ part,
-                                                          double init, double* __restrict__ out,
-                                                          int nnodes, double* __restrict__ hist,
-                                                          const int* __restrict__ cycle,
-                                                          const int* __restrict__ bad,
-                                                          int* __restrict__ status)
+// Sum of partials; *out = init + sum.
+__global__ __launch_bounds__(kSumBlock) void k_sum_final(int np, const double* __restrict__ part, double init,
+                                                          double* __restrict__ out)
 {
 #pragma clang fp contract(off)
-    if (status && *status != 0) return;
     int unused = 0;
     double s = strided_sum<kSumBlock>(part, nullptr, 0, np, unused);
     s = block_sum<kSumBlock>(s);
+    if (threadIdx.x == 0) *out = init + s;
+}
+
+// The device driver's level-0 RMS sqrt(sum / n) of every mesh, stored at
+// hist[mesh][*cycle] (euler3d.cpp:532-537), and abort code 2 on a non-zero
+// bad-value count (euler3d.cpp:539-548).  One workgroup per mesh; in a cycle
+// with a restriction it is one of that kernel's workgroups (mg_sum), which
+// takes the reduction's own launch and latency off the cycle.
+struct SumArgs {
+    int n;                  // meshes
+    int np;                 // partial sums of a single mesh ...
+    const int* sblk;        // ... or each mesh's first one (n + 1)
+    const double* part;
+    const int* badpart;     // NaN/Inf counts per partial sum, or
+    const int* bad;         // one count (halting contexts)
+    int nodes;
+    const int* seg_nodes;   // nodes of each mesh (null: 'nodes')
+    double* hist;
+    int cap;                // history entries of a mesh
+    const int* cycle;
+    int* sstatus;           // per mesh
+};
+
+__device__ __forceinline__ void mg_sum(const SumArgs& a, int m)
+{
+#pragma clang fp contract(off)
+    const int lo = a.sblk ? a.sblk[m] : 0, hi = a.sblk ? a.sblk[m + 1] : a.np;
+    const int c = *a.cycle;
+    const int bad = a.bad ? *a.bad : 0;
+    int nb = 0;
+    const double s = block_sum(strided_sum<kBlock>(a.part, a.badpart, lo, hi, nb));
+    if (a.badpart) nb = block_sum_i(nb);
     if (threadIdx.x == 0) {
-        s = init + s;
-        if (out) *out = s;
-        if (hist) hist[*cycle] = sqrt(s / (double)nnodes);
-        if (status && bad && *bad > 0) *status = 2;
+        if (c < a.cap) a.hist[(size_t)m * a.cap + c] = sqrt(s / (double)(a.seg_nodes ? a.seg_nodes[m] : a.nodes));
+        if (nb + bad > 0 && a.sstatus[m] == 0) a.sstatus[m] = 2;
     }
+}
+
+__global__ __launch_bounds__(kBlock) void k_mg_sum(SumArgs a, const int* __restrict__ status)
+{
+    if (halted(status)) return;
+    mg_sum(a, blockIdx.x);
 }
 
 __global__ __launch_bounds__(kBlock) void k_count_bad(int n, const double* __restrict__ x,
@@ -2047,31 +2080,64 @@ __global__ void k_up_post(int nc, double* __restrict__ vc, const int* __restrict
     store5(vc, i, x);
 }
 
-// down_kernel (prolongation).
+// The nodes [lo, lo + cnt) of one transfer workgroup, and its segment.
+struct NodeBlock {
+    int lo, cnt, seg;
+};
+__device__ __forceinline__ NodeBlock node_block(const int4* blk, int b, int n)
+{
+    if (blk) {
+        const int4 B = blk[b];
+        return {B.y, B.z - B.y, B.x};
+    }
+    return {b * kBlock, min(kBlock, n - b * kBlock), 0};
+}
+
+// A workgroup's states in LDS (five doubles per node) written to [n][5]
+// arrays as one run, consecutive doubles by consecutive lanes.
+__device__ __forceinline__ void store_run(const NodeBlock& B, const double* lds, double* __restrict__ a,
+                                          double* __restrict__ b)
+{
+    const size_t base = (size_t)B.lo * 5;
+    for (int j = threadIdx.x; j < 5 * B.cnt; j += kBlock) {
+        const double x = lds[j];
+        if (a) a[base + j] = x;
+        b[base + j] = x;
+    }
+}
+
 // up_pre + up + up_post (mg.h:29-64) as one gather per coarse node of a
 // restriction whose every coarse node is a target (dense plan), followed by
-// the coarse level's calculate_dt.
+// the coarse level's calculate_dt.  The first sum.n workgroups reduce the
+// level-0 RMS instead (a restriction from level 0): they run beside the
+// restriction, which reads the bad-value count itself and stops as the
+// status they set would stop it.  vc null: the state is needed only as the
+// old state (the fused stages read that and write the variables).  Bound by
+// the children's gather; with the results stored per node instead of as runs
+// the 1M-node solve's restrictions took 32, 21 and 16 us, now 22, 15 and 12.
 __global__ __launch_bounds__(kBlock) void k_up_gather_dt(
     int nc, const int* __restrict__ ptr, const int* __restrict__ child, const double* __restrict__ vf,
-    double* __restrict__ vc, int* __restrict__ scratch, const int* __restrict__ status, DtArgs d)
+    const double* __restrict__ vc0, double* __restrict__ vc, int* __restrict__ scratch,
+    const int* __restrict__ status, DtArgs d, SumArgs sum)
 {
 #pragma clang fp contract(off)
+    __shared__ double run[5 * kBlock];
     if (halted(status)) return;
-    int c, lim;
-    if (d.blk) {
-        const int4 B = d.blk[blockIdx.x];
-        c = B.y + threadIdx.x;
-        lim = B.z;
-    } else {
-        c = blockIdx.x * blockDim.x + threadIdx.x;
-        lim = nc;
+    if ((int)blockIdx.x < sum.n) {
+        mg_sum(sum, blockIdx.x);
+        return;
     }
+    if (sum.bad && *sum.bad > 0) return;
+    const int b = blockIdx.x - sum.n;
+    const NodeBlock B = node_block(d.blk, b, nc);
+    const int t = threadIdx.x;
     double m = DBL_MAX;
-    if (c < lim) {
+    if (t < B.cnt) {
+        const int c = B.lo + t;
         const int beg = ptr[c], end = ptr[c + 1];
         double acc[5];
         if (beg == end) {
-            load5(vc, c, acc);             // no children: stale value kept (mg.h:58)
+            load5(vc0, c, acc);            // no children: stale value kept (mg.h:58)
         } else {
 #pragma unroll
             for (int v = 0; v < 5; v++) acc[v] = 0.0;
@@ -2086,14 +2152,18 @@ __global__ __launch_bounds__(kBlock) void k_up_gather_dt(
             const double avg = 1.0 / (double)cnt;
 #pragma unroll
             for (int v = 0; v < 5; v++) acc[v] *= avg;
-            store5(vc, c, acc);
             scratch[c] = cnt;
         }
-        m = min_candidate(calc_dt_state(c, acc, d.vol, d.dt, d.old));
+#pragma unroll
+        for (int v = 0; v < 5; v++) run[t * 5 + v] = acc[v];
+        m = min_candidate(calc_dt_state(c, acc, d.vol, d.dt));
     }
-    min_publish(d.pub, d.blk ? d.blk[blockIdx.x].x : 0, block_min(m));
+    m = block_min(m);                      // its barrier also completes the run
+    store_run(B, run, vc, d.old);
+    min_publish(d.pub, B.seg, b, m);
 }
 
+// down_kernel (prolongation).
 __global__ void k_down(int nf, const int* __restrict__ f2c, double* __restrict__ vf,
                        const double* __restrict__ rf, const double* __restrict__ xf,
                        const double* __restrict__ rc, const double* __restrict__ xc,
@@ -2197,43 +2267,68 @@ __global__ void k_down_v2_post(int n, const double* __restrict__ rp, const doubl
     store5(vf, i, u);
 }
 
-// down_kernel (mg.h:66-88) followed by the fine level's calculate_dt.
-__global__ __launch_bounds__(kBlock) void k_down_dt(
-    int nf, const int* __restrict__ f2c, double* __restrict__ vf, const double* __restrict__ rf,
+// down_kernel (mg.h:66-88) of the device driver.  DT: followed by the fine
+// level's calculate_dt.  END: the cycle's last kernel, which also moves the
+// cycle counter on.  The fine states and residuals come and go as runs of
+// doubles (consecutive lanes, consecutive doubles); each thread gathers its
+// node's coarse residual and distances into LDS, where the run's doubles
+// find them.  vf_out null: the state is needed only as the old state.  Bound by
+// memory traffic on large levels (550K nodes 33 -> 24 us, 370K 24 -> 19 us
+// against per-node loads and stores), by its latency below 50K nodes (5 us).
+template <bool DT, bool END>
+__global__ __launch_bounds__(kBlock) void k_down_mg(
+    int nf, const int* __restrict__ f2c, const double* vf, double* vf_out, const double* __restrict__ rf,
     const double* __restrict__ xf, const double* __restrict__ rc, const double* __restrict__ xc,
-    const int* __restrict__ status, DtArgs d)
+    const int* __restrict__ status, int* __restrict__ cycle, DtArgs d)
 {
 #pragma clang fp contract(off)
+    __shared__ double step[5 * kBlock], dist[4 * kBlock];
     if (halted(status)) return;
-    int i, lim;
-    if (d.blk) {
-        const int4 B = d.blk[blockIdx.x];
-        i = B.y + threadIdx.x;
-        lim = B.z;
-    } else {
-        i = blockIdx.x * blockDim.x + threadIdx.x;
-        lim = nf;
+    const int b = blockIdx.x, t = threadIdx.x;
+    if (END && b == 0 && t == 0) *cycle += 1;
+    const NodeBlock B = node_block(d.blk, b, nf);
+    const size_t base = (size_t)B.lo * 5;
+    const int last = 5 * B.cnt - 1;
+    const int i = B.lo + min(t, B.cnt - 1);
+    const int c = f2c[i];
+    double u[5], r[5];
+#pragma unroll
+    for (int k = 0; k < 5; k++) {
+        const size_t j = base + min(t + k * kBlock, last);
+        u[k] = vf[j];
+        r[k] = rf[j];
     }
-    double m = DBL_MAX;
-    if (i < lim) {
-        const int c = f2c[i];
-        const double dx = fabs(xf[3 * (size_t)i] - xc[3 * (size_t)c]);
-        const double dy = fabs(xf[3 * (size_t)i + 1] - xc[3 * (size_t)c + 1]);
-        const double dz = fabs(xf[3 * (size_t)i + 2] - xc[3 * (size_t)c + 2]);
-        const double dm = sqrt(dx * dx + dy * dy + dz * dz);
-        double u[5], r[5], ra[5];
-        load5(vf, i, u);
-        load5(rf, i, r);
-        load5(rc, c, ra);
-        u[0] -= dm * (ra[0] - r[0]);
-        u[1] -= dx * (ra[1] - r[1]);
-        u[2] -= dy * (ra[2] - r[2]);
-        u[3] -= dz * (ra[3] - r[3]);
-        u[4] -= dm * (ra[4] - r[4]);
-        store5(vf, i, u);
-        m = min_candidate(calc_dt_state(i, u, d.vol, d.dt, d.old));
+    const double dx = fabs(xf[3 * (size_t)i] - xc[3 * (size_t)c]);
+    const double dy = fabs(xf[3 * (size_t)i + 1] - xc[3 * (size_t)c + 1]);
+    const double dz = fabs(xf[3 * (size_t)i + 2] - xc[3 * (size_t)c + 2]);
+    double ra[5];
+    load5(rc, c, ra);
+#pragma unroll
+    for (int v = 0; v < 5; v++) step[t * 5 + v] = ra[v];
+    dist[t * 4] = sqrt(dx * dx + dy * dy + dz * dz);
+    dist[t * 4 + 1] = dx;
+    dist[t * 4 + 2] = dy;
+    dist[t * 4 + 3] = dz;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 5; k++) {
+        const int j = t + k * kBlock;
+        if (j <= last) {
+            const int n = j / 5, v = j % 5;
+            u[k] -= dist[n * 4 + (v & 3)] * (step[j] - r[k]);
+            if (vf_out) vf_out[base + j] = u[k];
+            if constexpr (DT) {
+                d.old[base + j] = u[k];
+                step[j] = u[k];              // this thread alone reads entry j
+            }
+        }
     }
-    min_publish(d.pub, d.blk ? d.blk[blockIdx.x].x : 0, block_min(m));
+    if constexpr (DT) {
+        __syncthreads();
+        double m = DBL_MAX;
+        if (t < B.cnt) m = min_candidate(calc_dt_state(i, step + t * 5, d.vol, d.dt));
+        min_publish(d.pub, B.seg, b, block_min(m));
+    }
 }
 
 // ------------------------------------------------------------------------
@@ -2301,31 +2396,11 @@ __global__ __launch_bounds__(kBlock) void k_calc_dt_seg(const int4* __restrict__
     const int i = B.y + threadIdx.x;
     double d = DBL_MAX;
     if (i < B.z) d = min_candidate(calc_dt_node(i, var, vol, dt, old));
-    min_publish(pub, B.x, block_min(d));
+    min_publish(pub, B.x, blockIdx.x, block_min(d));
 }
 
-__global__ __launch_bounds__(kSumBlock) void k_sum_final_seg(const int* __restrict__ sblk,
-                                                             const double* __restrict__ part,
-                                                             const int* __restrict__ badpart,
-                                                             const int* __restrict__ nnodes, double* __restrict__ hist,
-                                                             int cap, const int* __restrict__ cycle,
-                                                             int* __restrict__ sstatus, const int* __restrict__ halt)
-{
-#pragma clang fp contract(off)
-    if (halted(halt)) return;
-    const int s = blockIdx.x;
-    int nb = 0;
-    double x = strided_sum<kSumBlock>(part, badpart, sblk[s], sblk[s + 1], nb);
-    x = block_sum<kSumBlock>(x);
-    nb = block_sum_i<kSumBlock>(nb);
-    if (threadIdx.x == 0) {
-        const int c = *cycle;
-        if (c < cap) hist[(size_t)s * cap + c] = sqrt(x / (double)nnodes[s]);
-        if (nb > 0 && sstatus[s] == 0) sstatus[s] = 2;
-    }
-}
-
-// Cycle counter: counts cycles that ran (a halted context stops counting).
+// Cycle counter of one-level contexts: counts cycles that ran (a halted
+// context stops counting).
 __global__ void k_bump(int* c, const int* __restrict__ status)
 {
     if (threadIdx.x == 0 && !halted(status)) *c += 1;

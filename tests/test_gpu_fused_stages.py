@@ -125,3 +125,35 @@ def test_threads_per_part_change_nothing(rt, n, deg, variant):
     for other in got[1:]:
         for a, b in zip(got[0], other):
             assert np.array_equal(a.view(np.uint64), b.view(np.uint64))
+
+
+@pytest.mark.parametrize("variant", ["gather_exact", "part_coloured", "part_atomic", "nodal_exact"])
+@pytest.mark.parametrize("level", [0, 1])
+@pytest.mark.parametrize("graph", [False, True])
+def test_abort_keeps_the_references_state(rt, level, graph, variant):
+    """A negative minimum dt (a negative volume) on the second level, whose
+    state a restriction has just made, or on the first: every level's
+    variables are the reference's at its early return."""
+    mesh = random_mesh(515, 4, seed=9)
+    o = Oracle("orc")
+    state = perturbed_state(515, o.freestream(0.5, 3.0).ff_variable[:], seed=5)
+    vol = {}
+
+    def after_setup(levels):
+        levels[0]["var"][:] = state
+        levels[level]["vol"][3] *= -1.0
+        vol[0] = levels[level]["vol"].copy()
+
+    ref = o.solve(mesh, 3, 0.5, 3.0, after_setup=after_setup)
+    s = mgcfd.Solver(rt, mesh, 0.5, 3.0)
+    s.setup()
+    rt.upload(s.lv[0].variables, state)
+    rt.upload(s.lv[level].volumes, vol[0])
+    rt.set_flux_variant(mgcfd.FLUX_VARIANTS[variant])
+    st, _ = s.run_device(3, use_graph=graph)
+    assert st == ref["status"] == 1
+    for l in range(2):
+        err = rel_err(s.state(l), ref["levels"][l]["variables"])
+        assert err <= STATE_TOL, f"level {l}: {err:.3e}"
+        if variant != "nodal_exact":    # its flux kernel has run by the time its stage kernel aborts
+            assert not s.state(l, "fluxes").any()
