@@ -1003,6 +1003,20 @@ __global__ __launch_bounds__(kBlock) void k_stream_copy(size_t n, const double2*
     for (size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (size_t)gridDim.x * kBlock) b[i] = a[i];
 }
 
+// Rows [r0, r0 + rows) of a dat in the caller's element order, written to
+// pinned host memory: row r is the device's row idx[r] (idx null: row r).
+// Bound by the host link: consecutive lanes write consecutive elements.
+template <typename E>
+__global__ __launch_bounds__(kBlock) void k_fetch_rows(int r0, int rows, int dim, const int* __restrict__ idx,
+                                                       const E* __restrict__ src, E* __restrict__ out)
+{
+    const int n = rows * dim;
+    for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
+        const int r = i / dim, v = i - r * dim;
+        out[i] = src[(size_t)(idx ? idx[r0 + r] : r0 + r) * dim + v];
+    }
+}
+
 // Packed edge weights {w0, w1, w2, |w|} (flux.h:48-50).
 __global__ void k_pack_weights(int n, const double* __restrict__ w, double4* __restrict__ out)
 {

@@ -62,6 +62,7 @@ struct SetImpl {
     std::vector<int> seg;        // segment offsets (batched meshes), empty: one segment
     std::vector<int> parts;      // part boundaries of the node order (size parts + 1)
     std::vector<double> geo;     // node coordinates [n][3] (original order) when known: geometric order
+    int* d_iperm = nullptr;      // device copy of iperm (first fetch of a dat on the set)
     bool frozen = false;         // internal order chosen
     bool priv = false;           // declared by a batch builder, which orders and uploads it itself
     int to_int(int orig) const { return iperm.empty() ? orig : iperm[orig]; }
@@ -735,9 +736,78 @@ static int upload_dat(op_dat d)
     return 0;
 }
 
-// ---------------------------------------------------------------- plans --
-
 #define TRY(x) do { if (int rc_ = (x)) return rc_; } while (0)
+
+// ---------------------------------------------------------------- fetch --
+
+// Pinned landing buffers of fetches: kept from the first large fetch until
+// op_exit, 16 MB in all; one fetch at a time holds them.
+constexpr int kFetchSlots = 8;
+constexpr size_t kFetchBytes = 2u << 20;
+struct FetchPool {
+    std::mutex mu;
+    char* pin[kFetchSlots] = {};
+    hipEvent_t ev[kFetchSlots] = {};
+};
+static FetchPool g_fetch;
+
+static void fetch_pool_free()
+{
+    std::lock_guard<std::mutex> lk(g_fetch.mu);
+    for (int k = 0; k < kFetchSlots; k++) {
+        if (g_fetch.pin[k]) hipHostFree(g_fetch.pin[k]);
+        if (g_fetch.ev[k]) hipEventDestroy(g_fetch.ev[k]);
+        g_fetch.pin[k] = nullptr;
+        g_fetch.ev[k] = nullptr;
+    }
+}
+
+// Elements [lo, lo + cnt) of a [set][dim] device array in the set's internal
+// order, copied to dest (host) in the caller's order once everything queued
+// on the stream has run.  The device undoes
+// the renumbering while it writes 2 MB pieces over the host link, and up to
+// eight threads copy the pieces on (a copy's first touch of fresh pages is
+// what costs).  Five doubles per element, against a pageable copy permuted on
+// one host thread: 10.6K elements 201 -> 32 us, 300K 2380 -> 369 us, 1M 17.1
+// -> 1.2 ms.
+static int fetch_elements(op_set set, const void* dev, bool is_int, int dim, int lo, int cnt, void* dest,
+                          hipStream_t stream)
+{
+    if (cnt <= 0) return 0;
+    SetImpl* si = S(set);
+    const size_t rec = (is_int ? sizeof(int) : sizeof(double)) * dim;
+    std::lock_guard<std::mutex> lk(g_fetch.mu);
+    if (!si->iperm.empty() && !si->d_iperm) {
+        HIPCHK(hipMalloc(&si->d_iperm, sizeof(int) * si->iperm.size()));
+        HIPCHK(hipMemcpy(si->d_iperm, si->iperm.data(), sizeof(int) * si->iperm.size(), hipMemcpyHostToDevice));
+    }
+    const int piece = (int)std::max<size_t>(1, kFetchBytes / rec);
+    const int np = (cnt + piece - 1) / piece, nw = std::min(np, kFetchSlots);
+    for (int k = 0; k < nw; k++) {
+        if (!g_fetch.pin[k]) HIPCHK(hipHostMalloc(&g_fetch.pin[k], std::max(kFetchBytes, rec), hipHostMallocDefault));
+        if (!g_fetch.ev[k]) HIPCHK(hipEventCreateWithFlags(&g_fetch.ev[k], hipEventDisableTiming));
+    }
+    // worker w takes pieces w, w + nw, ...: its buffer is free once copied on
+    return run_tasks(nw, [&](int w) -> int {
+        for (int p = w; p < np; p += nw) {
+            const int r0 = p * piece, rows = std::min(piece, cnt - r0);
+            const unsigned grid = std::min(512u, nblk((size_t)rows * dim));
+            if (is_int)
+                k_fetch_rows<int><<<grid, kBlock, 0, stream>>>(lo + r0, rows, dim, si->d_iperm, (const int*)dev,
+                                                               (int*)g_fetch.pin[w]);
+            else
+                k_fetch_rows<double><<<grid, kBlock, 0, stream>>>(lo + r0, rows, dim, si->d_iperm,
+                                                                  (const double*)dev, (double*)g_fetch.pin[w]);
+            TRY(check_launch());
+            HIPCHK(hipEventRecord(g_fetch.ev[w], stream));
+            HIPCHK(hipEventSynchronize(g_fetch.ev[w]));
+            std::memcpy(static_cast<char*>(dest) + (size_t)r0 * rec, g_fetch.pin[w], rec * (size_t)rows);
+        }
+        return 0;
+    });
+}
+
+// ---------------------------------------------------------------- plans --
 
 // Blocked-gather plan.  Blocks are the kPart-node parts of the node order
 // (halved recursively while a part's halo exceeds kHaloCap).  Per block: the sorted halo, and the
@@ -1322,6 +1392,7 @@ static void release_set(op_set s)
 {
     RtLock lk(g_rt_mu);
     if (!s || !s->impl) return;
+    if (S(s)->d_iperm) hipFree(S(s)->d_iperm);
     delete S(s);
     s->impl = nullptr;
     s->size = 0;
@@ -1787,7 +1858,8 @@ void op_exit(void)
     mg_release_all();
     for (auto& d : R.dats) release_dat(&d);
     for (auto& m : R.maps) release_map(&m);
-    for (auto& s : R.sets) delete S(&s);
+    for (auto& s : R.sets) release_set(&s);
+    fetch_pool_free();
     R.dats.clear();
     R.maps.clear();
     R.sets.clear();
@@ -2025,16 +2097,7 @@ int op_fetch_data_char(op_dat d, char* dest)
 {
     if (!d || !dest) return fail("op_fetch_data: null argument");
     TRY(freeze());
-    DatImpl* di = D(d);
-    SetImpl* si = S(d->set);
-    const int n = d->set->size, dim = d->dim;
-    const size_t esz = di->is_int ? sizeof(int) : sizeof(double);
-    const size_t rec = esz * dim;
-    std::vector<char> aos(rec * (size_t)std::max(n, 1));
-    HIPCHK(hipStreamSynchronize(cur_stream()));
-    HIPCHK(hipMemcpy(aos.data(), di->d, rec * (size_t)n, hipMemcpyDeviceToHost));
-    for (int i = 0; i < n; i++) std::memcpy(dest + (size_t)si->to_orig(i) * rec, aos.data() + (size_t)i * rec, rec);
-    return 0;
+    return fetch_elements(d->set, D(d)->d, D(d)->is_int, d->dim, 0, d->set->size, dest, cur_stream());
 }
 
 int op_upload_data_char(op_dat d, const char* src)
