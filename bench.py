@@ -509,7 +509,7 @@ def summarize_trace(stats_or_trace, mode, pattern=None):
             out.append(f"| `{short(r['Name'])}` | {r['Calls']} | {float(r['AverageNs']) / 1e3:.2f} | "
                        f"{float(r['MinNs']) / 1e3:.2f} | {float(r['MaxNs']) / 1e3:.2f} | {float(r['Percentage']):.1f} |")
     elif mode == "cycle":
-        pat = pattern or r"k_flux_part_stage<double, 256, \d+, \d+, false"
+        pat = pattern or r"k_flux_part_stage<double, \d+, \d+, \d+, false"
         rows.sort(key=lambda r: int(r["Start_Timestamp"]))
         idx = [i for i, r in enumerate(rows) if re.search(pat, r["Kernel_Name"])]
         win = rows[idx[0]:idx[-1] + 1]

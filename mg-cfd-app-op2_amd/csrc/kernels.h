@@ -266,7 +266,7 @@ struct BlkInfo {
     int n0, cnt;    // owned nodes [n0, n0 + cnt)
     int h0, nh;     // halo ids halo[h0 .. h0 + nh)
     int j0, p0;     // first jagged entry; start of the diagonal offsets in jpref
-    int pad0, pad1;
+    int g0, pad;    // first partial sum of the block's nodes (one per 64)
 };
 
 // The derived half of a record from its conserved variables r[0..4].
@@ -311,14 +311,16 @@ struct IncChunk {
     double x0[CH], x1[CH], x2[CH];
 };
 
-template <int CH>
-__device__ __forceinline__ void load_chunk(IncChunk<CH>& c, int q0, int deg, int jb, const int* __restrict__ jp,
-                                           const unsigned* __restrict__ jslot, const double* __restrict__ jw,
-                                           int nent)
+// LPN lanes share a node: lane l takes its incidences l, l + LPN, ...; q0
+// counts a lane's own.
+template <int CH, int LPN>
+__device__ __forceinline__ void load_chunk(IncChunk<CH>& c, int q0, int l, int deg, int jb,
+                                           const int* __restrict__ jp, const unsigned* __restrict__ jslot,
+                                           const double* __restrict__ jw, int nent)
 {
 #pragma unroll
     for (int i = 0; i < CH; i++) {
-        const int q = q0 + i;
+        const int q = (q0 + i) * LPN + l;
         c.r[i] = 0;
         c.x0[i] = c.x1[i] = c.x2[i] = 0.0;
         if (q < deg) {
@@ -331,26 +333,60 @@ __device__ __forceinline__ void load_chunk(IncChunk<CH>& c, int q0, int deg, int
     }
 }
 
-template <bool EXACT, int CH>
-__device__ __forceinline__ void walk_chunk(const IncChunk<CH>& c, int q0, int deg, const double* sm, const Th& o,
-                                           double sc, double acc[5])
+// x of lane K of this lane's group of LPN lanes (LPN 2 or 4).
+template <int LPN, int K>
+__device__ __forceinline__ double group_lane(double x)
+{
+    constexpr int ctrl = LPN == 4 ? K * 0x55 : K ? 0xf5 : 0xa0;      // quad_perm
+    const int lo = __double2loint(x), hi = __double2hiint(x);
+    return __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, ctrl, 0xf, 0xf, true),
+                            __builtin_amdgcn_update_dpp(lo, lo, ctrl, 0xf, 0xf, true));
+}
+
+template <bool EXACT, int LPN, int K = 0>
+__device__ __forceinline__ void add_group(const double d[5], double acc[5])
+{
+    if constexpr (K < LPN) {
+#pragma unroll
+        for (int v = 0; v < 5; v++) acc[v] = add_exact(acc[v], group_lane<LPN, K>(d[v]));
+        add_group<EXACT, LPN, K + 1>(d, acc);
+    }
+}
+
+template <bool EXACT>
+__device__ __forceinline__ void incidence(unsigned r, double x0, double x1, double x2, const double* sm, const Th& o,
+                                          double sc, double d[5])
+{
+    Th th;
+    load_record<EXACT>(sm + (int)(r & 0x7fffffffu) * kGRec, th);
+    double ewt;
+    {
+#pragma clang fp contract(off)
+        ewt = sqrt(x0 * x0 + x1 * x1 + x2 * x2);
+    }
+    double fx = -0.5 * x0, fy = -0.5 * x1, fz = -0.5 * x2;
+    if (r & 0x80000000u) { fx = -fx; fy = -fy; fz = -fz; }   // node is endpoint b
+    edge_increment<EXACT>(o, th, ewt, sc, fx, fy, fz, d);
+}
+
+// The increments of a chunk added in incidence order.  With several lanes per
+// node each lane evaluates its own, and all of them add the group's in lane
+// order (-0.0 where a lane has none, which leaves every sum as it is), so
+// every lane holds the node's sum.  The lanes of a group agree on the loop
+// bounds, so the exchange reads active lanes only.
+template <bool EXACT, int CH, int LPN>
+__device__ __forceinline__ void walk_chunk(const IncChunk<CH>& c, int q0, int l, int deg, const double* sm,
+                                           const Th& o, double sc, double acc[5])
 {
 #pragma unroll
     for (int i = 0; i < CH; i++) {
-        if (q0 + i < deg) {
-            const unsigned r = c.r[i];
-            Th th;
-            load_record<EXACT>(sm + (int)(r & 0x7fffffffu) * kGRec, th);
-            double ewt;
-            {
-#pragma clang fp contract(off)
-                ewt = sqrt(c.x0[i] * c.x0[i] + c.x1[i] * c.x1[i] + c.x2[i] * c.x2[i]);
-            }
-            double fx = -0.5 * c.x0[i], fy = -0.5 * c.x1[i], fz = -0.5 * c.x2[i];
-            if (r & 0x80000000u) { fx = -fx; fy = -fy; fz = -fz; }   // node is endpoint b
-            double d[5];
-            edge_increment<EXACT>(o, th, ewt, sc, fx, fy, fz, d);
-            if constexpr (EXACT) {
+        if ((q0 + i) * LPN < deg) {
+            double d[5] = {-0.0, -0.0, -0.0, -0.0, -0.0};
+            if (LPN == 1 || (q0 + i) * LPN + l < deg)
+                incidence<EXACT>(c.r[i], c.x0[i], c.x1[i], c.x2[i], sm, o, sc, d);
+            if constexpr (LPN > 1) {
+                add_group<EXACT, LPN>(d, acc);
+            } else if constexpr (EXACT) {
 #pragma unroll
                 for (int v = 0; v < 5; v++) acc[v] = add_exact(acc[v], d[v]);
             } else {
@@ -372,80 +408,81 @@ struct GatherPlan {
     int nent;
 };
 
-// Steps 1 and 2 for one block: acc holds the thread's node's start value and
-// receives its edge flux (threads t < cnt); o: the node's own state.  LDS: one
-// record per staged node.  Ends without a barrier.
-template <bool EXACT, int CH, int NH>
+// Steps 1 and 2 for one block of at most PN nodes, LPN lanes to a node (PN *
+// LPN threads): acc holds the start value of the thread's node (t / LPN) and
+// receives its edge flux, in each of its lanes; o: the node's own state.
+// LDS: one record per staged node.  Ends without a barrier.
+template <bool EXACT, int CH, int NH, int PN, int LPN>
 __device__ __forceinline__ void gather_block(const GatherPlan& G, const BlkInfo& B, const double* __restrict__ vin,
                                              double sc, double* sm, double acc[5], Th& o)
 {
-    constexpr int FL = 5 * kPart / kBlock;
-    const int t = threadIdx.x;
-    const bool own = t < B.cnt;
+    constexpr int T = PN * LPN, FL = (5 * PN + T - 1) / T;
+    const int t = threadIdx.x, n = t / LPN, l = t % LPN;
+    const bool own = n < B.cnt;
     const int last = 5 * B.cnt - 1, hmax = max(B.nh - 1, 0);
     const size_t base = (size_t)B.n0 * 5;
     int hn[NH];
     double x[FL], U[NH][5];
 #pragma unroll
-    for (int k = 0; k < NH; k++) hn[k] = G.halo[B.h0 + min(t + k * kBlock, hmax)];
+    for (int k = 0; k < NH; k++) hn[k] = G.halo[B.h0 + min(t + k * T, hmax)];
 #pragma unroll
-    for (int i = 0; i < FL; i++) x[i] = vin[base + min(t + i * kBlock, last)];
-    const int nd = B.n0 + min(t, B.cnt - 1);
+    for (int i = 0; i < FL; i++) x[i] = vin[base + min(t + i * T, last)];
+    const int nd = B.n0 + min(n, B.cnt - 1);
     const int deg = own ? G.nptr[nd + 1] - G.nptr[nd] : 0;
-    const int jb = B.j0 + t;
+    const int jb = B.j0 + n;
     const int* jp = G.jpref + B.p0;
     IncChunk<CH> A, C;
-    load_chunk<CH>(A, 0, deg, jb, jp, G.jslot, G.jw, G.nent);
+    load_chunk<CH, LPN>(A, 0, l, deg, jb, jp, G.jslot, G.jw, G.nent);
 #pragma unroll
     for (int k = 0; k < NH; k++)
 #pragma unroll
         for (int v = 0; v < 5; v++) U[k][v] = vin[(size_t)hn[k] * 5 + v];
 #pragma unroll
     for (int i = 0; i < FL; i++) {
-        const int j = t + i * kBlock;
+        const int j = t + i * T;
         if (j <= last) sm[j + (j / 5) * (kGRec - 5)] = x[i];
     }
 #pragma unroll
     for (int k = 0; k < NH; k++)
-        if (t + k * kBlock < B.nh) {
-            double* r = sm + (B.cnt + t + k * kBlock) * kGRec;
+        if (t + k * T < B.nh) {
+            double* r = sm + (B.cnt + t + k * T) * kGRec;
 #pragma unroll
             for (int v = 0; v < 5; v++) r[v] = U[k][v];
             derive_record<EXACT>(r);
         }
     __syncthreads();
-    if (own) derive_record<EXACT>(sm + t * kGRec);
+    if (t < B.cnt) derive_record<EXACT>(sm + t * kGRec);
     __syncthreads();
     if (!own) return;
-    load_record<EXACT>(sm + t * kGRec, o);
-    for (int q0 = 0; q0 < deg; q0 += 2 * CH) {
-        load_chunk<CH>(C, q0 + CH, deg, jb, jp, G.jslot, G.jw, G.nent);
-        walk_chunk<EXACT, CH>(A, q0, deg, sm, o, sc, acc);
-        if (q0 + CH >= deg) break;
-        load_chunk<CH>(A, q0 + 2 * CH, deg, jb, jp, G.jslot, G.jw, G.nent);
-        walk_chunk<EXACT, CH>(C, q0 + CH, deg, sm, o, sc, acc);
+    load_record<EXACT>(sm + n * kGRec, o);
+    for (int q0 = 0; q0 * LPN < deg; q0 += 2 * CH) {
+        load_chunk<CH, LPN>(C, q0 + CH, l, deg, jb, jp, G.jslot, G.jw, G.nent);
+        walk_chunk<EXACT, CH, LPN>(A, q0, l, deg, sm, o, sc, acc);
+        if ((q0 + CH) * LPN >= deg) break;
+        load_chunk<CH, LPN>(A, q0 + 2 * CH, l, deg, jb, jp, G.jslot, G.jw, G.nent);
+        walk_chunk<EXACT, CH, LPN>(C, q0 + CH, l, deg, sm, o, sc, acc);
     }
 }
 
-template <bool EXACT, int CH, int NH>
-__global__ __launch_bounds__(kBlock) void k_flux_blocked_pf(GatherPlan G, const double* __restrict__ var,
-                                                            double* __restrict__ flux, Consts k,
-                                                            const int* __restrict__ status, int fresh)
+template <bool EXACT, int CH, int NH, int PN, int LPN>
+__global__ __launch_bounds__(PN * LPN) void k_flux_blocked_pf(GatherPlan G, const double* __restrict__ var,
+                                                              double* __restrict__ flux, Consts k,
+                                                              const int* __restrict__ status, int fresh)
 {
     extern __shared__ double sm[];
     if (halted(status)) return;
     const BlkInfo B = G.blk[xcd_block()];
-    const int t = threadIdx.x;
+    const int n = threadIdx.x / LPN;
     double acc[5];
     if (fresh) {
 #pragma unroll
         for (int v = 0; v < 5; v++) acc[v] = 0.0;
     } else {
-        load5(flux, B.n0 + min(t, B.cnt - 1), acc);
+        load5(flux, B.n0 + min(n, B.cnt - 1), acc);
     }
     Th o;
-    gather_block<EXACT, CH, NH>(G, B, var, k.sc, sm, acc, o);
-    if (t < B.cnt) store5(flux, B.n0 + t, acc);
+    gather_block<EXACT, CH, NH, PN, LPN>(G, B, var, k.sc, sm, acc, o);
+    if (n < B.cnt && threadIdx.x % LPN == 0) store5(flux, B.n0 + n, acc);
 }
 
 // Per-incidence weight components (SoA) of k_flux_blocked_pf.
@@ -491,7 +528,7 @@ struct PartInfo {
     int n0, cnt;    // owned nodes [n0, n0 + cnt)
     int h0, nh;     // halo ids halo[h0 .. h0 + nh)
     int e0, ne;     // local edges [e0, e0 + ne)
-    int ncol, pad;  // edge colours (COLOURED)
+    int ncol, g0;   // edge colours (COLOURED); first partial sum of the part's nodes (one per 64)
 };
 
 // One endpoint of an edge as the increment needs it.
@@ -1511,6 +1548,31 @@ __device__ __forceinline__ void stage_sums(const StageArgs& a, int w, double s, 
     }
 }
 
+// The same of the kernels with a fused stage: one square sum per 64 nodes
+// (thread t: node t of the workgroup's), slots g0 and up.  A level's sums
+// are the same whatever parts and threads its size selects, since parts
+// start at multiples of 64 nodes of their 256-node patch (patches at their
+// mesh's first node).
+template <int T>
+__device__ __forceinline__ void stage_group_sums(const StageArgs& a, int g0, int cnt, double s, int nb)
+{
+#pragma clang fp contract(off)
+    const int t = threadIdx.x;
+    if (a.part) {
+#pragma unroll
+        for (int o = kWave / 2; o > 0; o >>= 1) s += __shfl_down(s, o, kWave);
+        if (t % kWave == 0 && t < cnt) a.part[g0 + t / kWave] = s;
+    }
+    if (a.bad || a.badpart) {
+        nb = block_sum_i<T>(nb);
+        if (t == 0) {
+            if (a.badpart)
+                for (int k = 0; k * kWave < cnt; k++) a.badpart[g0 + k] = k ? 0 : nb;
+            else if (nb) atomicAdd(a.bad, nb);
+        }
+    }
+}
+
 // The stage's boundary table: the weights and group of each boundary
 // element, in the node -> boundary-element CSR order of 'bent', so a node
 // reads its elements as one contiguous run.
@@ -1577,7 +1639,7 @@ __device__ __forceinline__ double stage_factor(const StageArgs& a, int i, double
 // nodes' factors and fluxes in LDS; o: the old state, T apart.  The square
 // sum is formed node by node (thread t: node t), so that the reduction does
 // not depend on the number of threads.
-template <int T, int FL = (5 * kPart + T - 1) / T>
+template <int T, int FL>
 __device__ __forceinline__ void stage_run(const StageArgs& a, size_t base, int last, const double o[FL],
                                           const double* fac, double* acc, double& s, int& nb)
 {
@@ -1612,19 +1674,20 @@ __device__ __forceinline__ void stage_run(const StageArgs& a, size_t base, int l
 // flux kernel and a stage kernel of its own this saves a launch (about 4 us
 // each on a small level) and the flux's way through memory per stage: cycle of
 // a 300K-node solve 572 -> 468 us, 1M nodes 1341 -> 1187 us, 10K 280 -> 234 us.
-template <bool EXACT, int CH, int NH>
-__global__ __launch_bounds__(kBlock) void k_gather_stage(GatherPlan G, const int* __restrict__ pseg,
-                                                         const int* __restrict__ pfirst,
-                                                         const double* __restrict__ vin, int fresh, StageArgs a,
-                                                         Consts k0)
+template <bool EXACT, int CH, int NH, int PN, int LPN>
+__global__ __launch_bounds__(PN * LPN) void k_gather_stage(GatherPlan G, const int* __restrict__ pseg,
+                                                           const int* __restrict__ pfirst,
+                                                           const double* __restrict__ vin, int fresh, StageArgs a,
+                                                           Consts k0)
 {
-    constexpr int FL = 5 * kPart / kBlock;
+    constexpr int T = PN * LPN, FL = (5 * PN + T - 1) / T;
     extern __shared__ double sm[];
     const int halt = status_of(a.status);      // tested before the first global write
-    const int p = xcd_block(), t = threadIdx.x;
+    const int p = xcd_block(), t = threadIdx.x, n = t / LPN;
     const BlkInfo B = G.blk[p];
     const int seg = word_or_zero(pseg, p);
-    const int last = 5 * B.cnt - 1, own = B.n0 + min(t, B.cnt - 1);
+    const int last = 5 * B.cnt - 1, own = B.n0 + min(n, B.cnt - 1);
+    const bool head = n < B.cnt && t % LPN == 0;       // one lane per owned node
     const size_t base = (size_t)B.n0 * 5;
     const double vs = a.rk == 0 ? a.vol[own] : a.sf[own];
     const int q0 = a.bptr ? a.bptr[own] : 0, q1 = a.bptr ? a.bptr[own + 1] : 0;
@@ -1632,7 +1695,7 @@ __global__ __launch_bounds__(kBlock) void k_gather_stage(GatherPlan G, const int
     double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     if (!fresh) load5(a.flux, own, acc);
     Th o;
-    gather_block<EXACT, CH, NH>(G, B, vin, k0.sc, sm, acc, o);
+    gather_block<EXACT, CH, NH, PN, LPN>(G, B, vin, k0.sc, sm, acc, o);
     if (halt) return;
     double mdt = 0.0;
     if (a.rk == 0) {
@@ -1641,9 +1704,9 @@ __global__ __launch_bounds__(kBlock) void k_gather_stage(GatherPlan G, const int
     }
     double old[FL];
 #pragma unroll
-    for (int i = 0; i < FL; i++) old[i] = a.old[base + min(t + i * kBlock, last)];
+    for (int i = 0; i < FL; i++) old[i] = a.old[base + min(t + i * T, last)];
     double f = 0.0;
-    if (t < B.cnt) {
+    if (head) {
         if (q0 < q1) {
             const double U[5] = {o.rho, o.mx, o.my, o.mz, o.E};
             stage_bnd(a, a.kseg ? a.kseg[seg] : k0, U, q0, q1, acc);
@@ -1652,18 +1715,18 @@ __global__ __launch_bounds__(kBlock) void k_gather_stage(GatherPlan G, const int
     }
     __syncthreads();            // every record has been read: the space takes the fluxes and factors
     double* fl = sm;
-    double* fac = sm + 5 * kPart;
-    if (t < B.cnt) {
+    double* fac = sm + 5 * PN;
+    if (head) {
 #pragma unroll
-        for (int v = 0; v < 5; v++) fl[t * 5 + v] = acc[v];
-        fac[t] = f;
+        for (int v = 0; v < 5; v++) fl[n * 5 + v] = acc[v];
+        fac[n] = f;
     }
     __syncthreads();
     double s = 0.0;
     int nb = 0;
-    stage_run<kBlock>(a, base, last, old, fac, fl, s, nb);
-    stage_sums<kBlock>(a, p, s, nb);
-    stage_reset_min<kBlock>(a);
+    stage_run<T, FL>(a, base, last, old, fac, fl, s, nb);
+    stage_group_sums<T>(a, B.g0, B.cnt, s, nb);
+    stage_reset_min<T>(a);
 }
 
 // The FP64 / mixed part kernel fused with its Runge-Kutta stage (device
@@ -1685,16 +1748,17 @@ __global__ __launch_bounds__(kBlock) void k_gather_stage(GatherPlan G, const int
 // accesses at a 40-byte stride touch three times as many lines); only the
 // halo is gathered node by node.  Cycle of a 1M-node solve 908 -> 863 us,
 // 300K nodes 397 -> 384 us, 10K 213 -> 196 us (the minimum-dt slots, one per
-// lane, are loaded early too).  NPT: halo nodes per thread.
-template <typename R, int T, int EPT, int NPT, bool COLOURED, int RS>
+// lane, are loaded early too).  NPT: halo nodes per thread; PN: most owned
+// nodes.
+template <typename R, int T, int EPT, int NPT, bool COLOURED, int RS, int PN>
 __device__ __forceinline__ bool part_stage_one(
     int p, const PartInfo* __restrict__ parts, const int* __restrict__ halo, const unsigned* __restrict__ ecode,
     const R* __restrict__ ew, long long nloc, int rec_cap, const double* __restrict__ vin, int fresh,
     const StageArgs& a, const Consts& k0, const int* __restrict__ pseg, const int* __restrict__ pfirst, double* sm)
 {
     constexpr int ST = part_stride<R, RS>();
-    constexpr int FL = (5 * kPart + T - 1) / T;
-    static_assert(T >= kPart, "one owned node per thread");
+    constexpr int FL = (5 * PN + T - 1) / T;
+    static_assert(T >= PN, "one owned node per thread");
     // a halted context writes nothing: the status is tested after the edge
     // phase (which writes only LDS), so its load overlaps the staging loads
     const int halt = status_of(a.status);
@@ -1703,7 +1767,7 @@ __device__ __forceinline__ bool part_stage_one(
     const int t = threadIdx.x;
     R* rec = reinterpret_cast<R*>(sm);
     double* acc = sm + part_rec_doubles<R, RS>(rec_cap);
-    double* fac = acc + 5 * kPart;
+    double* fac = acc + 5 * PN;
     // 1. loads, all clamped into the part so that they issue without branches
     const int last = 5 * P.cnt - 1;
     const size_t base = (size_t)P.n0 * 5;
@@ -1781,20 +1845,20 @@ __device__ __forceinline__ bool part_stage_one(
     // 5. update over the run
     double s = 0.0;
     int nb = 0;
-    stage_run<T>(a, base, last, o, fac, acc, s, nb);
-    stage_sums<T>(a, p, s, nb);
+    stage_run<T, FL>(a, base, last, o, fac, acc, s, nb);
+    stage_group_sums<T>(a, P.g0, P.cnt, s, nb);
     return true;
 }
 
 // One workgroup per part.
-template <typename R, int T, int EPT, int NPT, bool COLOURED, int RS>
+template <typename R, int T, int EPT, int NPT, bool COLOURED, int RS, int PN>
 __global__ __launch_bounds__(T) void k_flux_part_stage(
     const PartInfo* __restrict__ parts, const int* __restrict__ pseg, const int* __restrict__ pfirst,
     const int* __restrict__ halo, const unsigned* __restrict__ ecode, const R* __restrict__ ew, long long nloc,
     int rec_cap, const double* __restrict__ vin, int fresh, StageArgs a, Consts k0)
 {
     extern __shared__ double sm[];
-    if (part_stage_one<R, T, EPT, NPT, COLOURED, RS>(xcd_block(), parts, halo, ecode, ew, nloc, rec_cap, vin, fresh,
+    if (part_stage_one<R, T, EPT, NPT, COLOURED, RS, PN>(xcd_block(), parts, halo, ecode, ew, nloc, rec_cap, vin, fresh,
                                                      a, k0, pseg, pfirst, sm))
         stage_reset_min<T>(a);
 }
@@ -1818,7 +1882,7 @@ __global__ __launch_bounds__(T) void k_flux_part_stage_persistent(
     const int lo = (x < rem) ? x * (per + 1) : rem * (per + 1) + (x - rem) * per;
     const int hi = lo + per + (x < rem ? 1 : 0);
     for (int p = lo + k; p < hi; p += g) {
-        if (!part_stage_one<R, T, EPT, NPT, COLOURED, RS>(p, parts, halo, ecode, ew, nloc, rec_cap, vin, fresh, a,
+        if (!part_stage_one<R, T, EPT, NPT, COLOURED, RS, kPart>(p, parts, halo, ecode, ew, nloc, rec_cap, vin, fresh, a,
                                                           k0, pseg, pfirst, sm))
             return;
         __syncthreads();        // the next part reuses the LDS

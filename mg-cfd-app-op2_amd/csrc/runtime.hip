@@ -98,11 +98,15 @@ struct InvPlan {
     const void* bk_wdat = nullptr;    // weight dat the packed weights came from
     unsigned bk_wver = 0;
     int bk_max_halo = 0, bk_rec_cap = 0;   // largest halo, and largest staged node count, of a block
+    int bk_max_cnt = 0;                    // most owned nodes of a block
+    int bk_groups = 0;                     // partial sums over all blocks (one per 64 owned nodes)
     // part plan (edge-parallel flux over mesh parts, k_flux_part)
     int pt_parts = 0;            // 0 = not available
     long long pt_nloc = 0;       // local edges over all parts
     int pt_rec_cap = 0;          // max staged nodes (owned + halo) of one part
     int pt_halo_cap = 0;         // max halo nodes of one part
+    int pt_max_cnt = 0;          // max owned nodes of one part
+    int pt_groups = 0;           // partial sums over all parts (one per 64 owned nodes)
     int pt_rec_med = 0;          // median staged nodes of a part
     int pt_rs = 6;               // values per FP64 LDS record (6, or 5: see build_partplan)
     std::vector<PartInfo> h_pt_info;   // host copy of the parts
@@ -121,7 +125,7 @@ struct InvPlan {
     const void* pt_w32dat = nullptr;
     unsigned pt_w32ver = 0;
     size_t pt_lds32 = 0;
-    int pt_psize = kPart;            // max nodes per part (autotuned)
+    int pt_psize = 0;                // max nodes per part (0: by small_part_nodes; autotuned)
     int pt_threads = 0;              // threads per part of the kernel with the fused stage (0: default; autotuned)
     int pt_persist = 0;              // fused-stage kernel: 0 one workgroup per part, else persistent workgroups
                                      // per CU (autotuned)
@@ -809,6 +813,26 @@ static int fetch_elements(op_set set, const void* dev, bool is_int, int dim, int
 
 // ---------------------------------------------------------------- plans --
 
+// Nodes per part or block of a level of np 256-node patches.  A level with
+// fewer patches than the device has CUs lasts as long as one workgroup, most
+// of which is instruction issue: patches are cut into halves or quarters while
+// the CUs hold them all at once.  (Cycle of a 10K-node solve, 11 to 40
+// patches per level: 174 -> 135 us with the part kernels, 229 -> 170 us with
+// the exact gather; a 100K-node solve's second and third level, 215 and 145
+// patches, were slower cut in two.)
+static int small_part_nodes(int np)
+{
+    return 4LL * np <= R.n_cu ? kPart / 4 : 2LL * np <= R.n_cu ? kPart / 2 : kPart;
+}
+
+// Where a part of more than 64 nodes is cut: near the middle, at a multiple
+// of 64 nodes (the kernels' partial sums run over 64-node groups).
+static int part_cut(int lo, int hi)
+{
+    const int half = (hi - lo) / 2;
+    return lo + (hi - lo > kWave ? (half + kWave - 1) / kWave * kWave : half);
+}
+
 // Blocked-gather plan.  Blocks are the kPart-node parts of the node order
 // (halved recursively while a part's halo exceeds kHaloCap).  Per block: the sorted halo, and the
 // incidences of its nodes in jagged-diagonal order -- diagonal k holds the
@@ -835,7 +859,8 @@ struct BlkOut {
     std::string err;
 };
 
-static void blocked_part(int lo0, int hi0, const std::vector<int>& ptr, const std::vector<int2>& inc2, BlkOut& out)
+static void blocked_part(int lo0, int hi0, int psize, const std::vector<int>& ptr, const std::vector<int2>& inc2,
+                         BlkOut& out)
 {
     std::vector<int2> work{make_int2(lo0, hi0)};
     std::vector<int> hb;
@@ -849,8 +874,8 @@ static void blocked_part(int lo0, int hi0, const std::vector<int>& ptr, const st
         }
         std::sort(hb.begin(), hb.end());
         hb.erase(std::unique(hb.begin(), hb.end()), hb.end());
-        if ((int)hb.size() > kHaloCap && hi - lo > 16) {
-            const int mid = lo + (hi - lo) / 2;
+        if (hi - lo > psize || ((int)hb.size() > kHaloCap && hi - lo > 16)) {
+            const int mid = part_cut(lo, hi);
             work.push_back(make_int2(mid, hi));
             work.push_back(make_int2(lo, mid));
             continue;
@@ -898,11 +923,12 @@ static int build_blocked(InvPlan& P, op_map m, const std::vector<int>& ptr, cons
     const std::vector<int> pb = set_parts(m->to);
     const int np = (int)pb.size() - 1;
     std::vector<BlkOut> outs(std::max(np, 0));
-    parallel_for(np, [&](int k) { blocked_part(pb[k], pb[k + 1], ptr, inc2, outs[k]); });
+    const int psize = small_part_nodes(np);
+    parallel_for(np, [&](int k) { blocked_part(pb[k], pb[k + 1], psize, ptr, inc2, outs[k]); });
     std::vector<BlkInfo> blocks;
     std::vector<int> halo, jpref, eid;
     std::vector<unsigned> jslot;
-    int max_halo = 0, rec_cap = 0;
+    int max_halo = 0, rec_cap = 0, max_cnt = 0, groups = 0;
     for (auto& o : outs) {
         if (!o.err.empty()) return fail("%s", o.err.c_str());
         size_t hp = 0, pp = 0, ep = 0;
@@ -914,6 +940,7 @@ static int build_blocked(InvPlan& P, op_map m, const std::vector<int>& ptr, cons
             bi.nh = o.nhalo[b];
             bi.j0 = (int)(jslot.size() + ep);
             bi.p0 = (int)(jpref.size() + pp);
+            bi.g0 = groups;
             // invariants the kernel relies on
             if (bi.cnt < 1 || bi.cnt > kPart || bi.nh > kHaloCap) return fail("internal error: blocked plan block too large");
             if (!blocks.empty() && bi.n0 != blocks.back().n0 + blocks.back().cnt)
@@ -926,6 +953,8 @@ static int build_blocked(InvPlan& P, op_map m, const std::vector<int>& ptr, cons
             ep += o.nent[b];
             max_halo = std::max(max_halo, bi.nh);
             rec_cap = std::max(rec_cap, bi.cnt + bi.nh);
+            max_cnt = std::max(max_cnt, bi.cnt);
+            groups += (bi.cnt + kWave - 1) / kWave;
             blocks.push_back(bi);
         }
         halo.insert(halo.end(), o.halo.begin(), o.halo.end());
@@ -954,6 +983,8 @@ static int build_blocked(InvPlan& P, op_map m, const std::vector<int>& ptr, cons
     P.bk_entries = (int)eid.size();
     P.bk_max_halo = max_halo;
     P.bk_rec_cap = rec_cap;
+    P.bk_max_cnt = max_cnt;
+    P.bk_groups = groups;
     for (const BlkInfo& bi : blocks) P.h_bk_node.push_back(make_int2(bi.n0, bi.cnt));
     P.bk_gen = ++g_plan_gen;
     P.bk_lds = sizeof(double) * kGRec * (size_t)rec_cap;
@@ -1031,16 +1062,68 @@ static void bank_order(std::vector<LEv>& le, std::vector<LEv>& out)
     le.swap(out);
 }
 
+// A local edge: endpoints, their LDS slots, edge id, owner flags, colour.
+struct LocalEdge {
+    int a, b, sa, sb, e;
+    unsigned flags;
+    int col;
+};
+
+// The local edges of the nodes [lo, hi): edges with an endpoint there,
+// ordered by edge id.
+static void local_edges(int lo, int hi, const std::vector<int>& ptr, const std::vector<int2>& inc2,
+                        std::vector<LocalEdge>& le)
+{
+    le.clear();
+    for (int nd = lo; nd < hi; nd++)
+        for (int q = ptr[nd]; q < ptr[nd + 1]; q++) {
+            const int o = inc2[q].x;
+            const bool role_b = (unsigned)inc2[q].y >> 31;
+            const bool other_owned = o >= lo && o < hi;
+            if (other_owned && role_b) continue;     // interior edge: taken from its a side
+            LocalEdge x{};
+            x.e = inc2[q].y & 0x7fffffff;
+            if (!role_b) { x.a = nd; x.b = o; x.flags = 1u | (other_owned ? 2u : 0u); }
+            else { x.a = o; x.b = nd; x.flags = 2u; }
+            le.push_back(x);
+        }
+    std::sort(le.begin(), le.end(), [](const LocalEdge& x, const LocalEdge& y) { return x.e < y.e; });
+}
+
+// Greedy colouring in edge order: no two edges of a colour share an owned
+// node.  Returns the number of colours, or -1 if 64 do not suffice.
+static int colour_edges(int lo, int hi, std::vector<LocalEdge>& le, std::vector<unsigned long long>& used)
+{
+    std::fill(used.begin(), used.begin() + (hi - lo), 0ull);
+    int ncol = 0;
+    for (auto& x : le) {
+        unsigned long long u = 0;
+        if (x.flags & 1u) u |= used[x.a - lo];
+        if (x.flags & 2u) u |= used[x.b - lo];
+        if (~u == 0ull) return -1;
+        const int c = __builtin_ctzll(~u);
+        x.col = c;
+        if (x.flags & 1u) used[x.a - lo] |= 1ull << c;
+        if (x.flags & 2u) used[x.b - lo] |= 1ull << c;
+        ncol = std::max(ncol, c + 1);
+    }
+    return ncol;
+}
+
 static void part_part(int lo0, int hi0, int psize, const std::vector<int>& ptr, const std::vector<int2>& inc2,
                       PartOut& out)
 {
     std::vector<int2> work{make_int2(lo0, hi0)};
     std::vector<int> hb;
     std::vector<unsigned long long> used(kPart);   // per owned node: colours taken
-    // a local edge: endpoints, their LDS slots, edge id, owner flags, colour
-    struct LE { int a, b, sa, sb, e; unsigned flags; int col; };
-    std::vector<LE> le, tmp;
+    std::vector<LocalEdge> le, tmp, whole;
     std::vector<int> ccount;
+    // The patch's edges are coloured as a whole, and every part cut from it
+    // keeps their colours, so that a node adds its edges in one order however
+    // its patch is cut.  (More than 64 colours: each part colours its own.
+    // A patch whose nodes have at most 32 edges never needs them.)
+    local_edges(lo0, hi0, ptr, inc2, whole);
+    const bool keep = colour_edges(lo0, hi0, whole, used) >= 0;
     while (!work.empty()) {
         const int lo = work.back().x, hi = work.back().y;
         work.pop_back();
@@ -1057,7 +1140,7 @@ static void part_part(int lo0, int hi0, int psize, const std::vector<int>& ptr, 
                           std::to_string(kPartSlots) + " neighbours";
                 return;
             }
-            const int mid = lo + (hi - lo) / 2;
+            const int mid = part_cut(lo, hi);
             work.push_back(make_int2(mid, hi));
             work.push_back(make_int2(lo, mid));
             continue;
@@ -1067,38 +1150,27 @@ static void part_part(int lo0, int hi0, int psize, const std::vector<int>& ptr, 
             if (nd >= lo && nd < hi) return nd - lo;
             return (hi - lo) + (int)(std::lower_bound(hb.begin(), hb.end(), nd) - hb.begin());
         };
-        le.clear();
-        for (int nd = lo; nd < hi; nd++)
-            for (int q = ptr[nd]; q < ptr[nd + 1]; q++) {
-                const int o = inc2[q].x;
-                const bool role_b = (unsigned)inc2[q].y >> 31;
-                const int e = inc2[q].y & 0x7fffffff;
-                const bool other_owned = o >= lo && o < hi;
-                if (other_owned && role_b) continue;     // interior edge: taken from its a side
-                LE x;
-                x.e = e;
-                const int so = slot(o);
-                if (!role_b) { x.a = nd; x.b = o; x.sa = nd - lo; x.sb = so; x.flags = 1u | (other_owned ? 2u : 0u); }
-                else { x.a = o; x.b = nd; x.sa = so; x.sb = nd - lo; x.flags = 2u; }
-                le.push_back(x);
-            }
-        // greedy colouring in edge order
-        std::fill(used.begin(), used.begin() + (hi - lo), 0ull);
-        std::sort(le.begin(), le.end(), [](const LE& x, const LE& y) { return x.e < y.e; });
         int ncol = 0;
-        for (auto& x : le) {
-            unsigned long long u = 0;
-            if (x.flags & 1u) u |= used[x.a - lo];
-            if (x.flags & 2u) u |= used[x.b - lo];
-            if (~u == 0ull) {
-                out.err = "edge-flux part plan: more than 64 edge colours in a part";
-                return;
+        if (lo == lo0 && hi == hi0) {
+            le.swap(whole);
+        } else {
+            local_edges(lo, hi, ptr, inc2, le);
+            if (keep) {          // both lists are in edge order
+                size_t w = 0;
+                for (auto& x : le) {
+                    while (whole[w].e != x.e) w++;
+                    x.col = whole[w].col;
+                }
             }
-            const int c = __builtin_ctzll(~u);
-            x.col = c;
-            if (x.flags & 1u) used[x.a - lo] |= 1ull << c;
-            if (x.flags & 2u) used[x.b - lo] |= 1ull << c;
-            ncol = std::max(ncol, c + 1);
+        }
+        if (!keep && colour_edges(lo, hi, le, used) < 0) {
+            out.err = "edge-flux part plan: more than 64 edge colours in a part";
+            return;
+        }
+        for (auto& x : le) {
+            x.sa = slot(x.a);
+            x.sb = slot(x.b);
+            ncol = std::max(ncol, x.col + 1);
         }
         // stable counting sort by colour (edge order kept within a colour)
         ccount.assign(ncol + 1, 0);
@@ -1116,7 +1188,7 @@ static void part_part(int lo0, int hi0, int psize, const std::vector<int>& ptr, 
         pi.e0 = (int)out.code.size();
         pi.ne = (int)le.size();
         pi.ncol = ncol;
-        pi.pad = 0;
+        pi.g0 = 0;       // set when the parts are put together
         for (const auto& x : le) {
             out.code.push_back((unsigned)x.sa | ((unsigned)x.sb << 10) | (x.flags << 20) | ((unsigned)x.col << 22));
             out.eid.push_back(x.e);
@@ -1135,17 +1207,21 @@ static int build_partplan(InvPlan& P, op_map m, const std::vector<int>& ptr, con
     const std::vector<int> pb = set_parts(m->to);
     const int np = (int)pb.size() - 1;
     std::vector<PartOut> outs(std::max(np, 0));
-    const int psize = P.pt_psize;
+    // parts smaller than a patch only where their colours are the patch's
+    const int psize = P.pt_psize ? P.pt_psize : P.max_deg <= 32 ? small_part_nodes(np) : kPart;
     parallel_for(np, [&](int k) { part_part(pb[k], pb[k + 1], psize, ptr, inc2, outs[k]); });
     std::vector<PartInfo> parts;
     std::vector<int> halo, eid;
     std::vector<unsigned> code;
-    int rec_cap = 0, halo_cap = 0, max_ne = 0, max_col = 0;
+    int rec_cap = 0, halo_cap = 0, max_cnt = 0, groups = 0, max_ne = 0, max_col = 0;
     for (auto& o : outs) {
         if (!o.err.empty()) return fail("%s", o.err.c_str());
         for (PartInfo pi : o.parts) {
             pi.h0 += (int)halo.size();
             pi.e0 += (int)code.size();
+            pi.g0 = groups;
+            groups += (pi.cnt + kWave - 1) / kWave;
+            max_cnt = std::max(max_cnt, pi.cnt);
             parts.push_back(pi);
             rec_cap = std::max(rec_cap, pi.cnt + pi.nh);
             halo_cap = std::max(halo_cap, pi.nh);
@@ -1193,6 +1269,8 @@ static int build_partplan(InvPlan& P, op_map m, const std::vector<int>& ptr, con
     P.pt_nloc = (long long)eid.size();
     P.pt_rec_cap = rec_cap;
     P.pt_halo_cap = halo_cap;
+    P.pt_max_cnt = max_cnt;
+    P.pt_groups = groups;
     {
         std::vector<int> r(parts.size());
         for (size_t i = 0; i < parts.size(); i++) r[i] = parts[i].cnt + parts[i].nh;
@@ -1533,23 +1611,43 @@ static GatherPlan gather_plan(const InvPlan& P)
     return GatherPlan{P.d_bk_info, P.d_bk_halo, P.d_bk_jpref, P.d_bk_nptr, P.d_bk_jslot, P.d_bk_w3, P.bk_entries};
 }
 
-template <bool EXACT, int NH>
-static int launch_blocked_nh(const InvPlan& P, op_dat var, op_dat flux, const int* status, int fresh)
-{
-    k_flux_blocked_pf<EXACT, 4, NH><<<P.bk_blocks, kBlock, P.bk_lds, cur_stream()>>>(gather_plan(P), dptr(var),
-                                                                                 dptr(flux), R.k, status, fresh);
-    return check_launch();
-}
-
-// Halo nodes per thread: one where the plan's largest halo allows it.
-static int launch_blocked_pf(bool exact, const InvPlan& P, op_dat var, op_dat flux, const int* status, int fresh)
+// Calls f(EXACT, NH, PN, LPN as integral constants) for a blocked plan: one
+// halo node per thread where the largest halo allows it, and several lanes per
+// node on levels whose blocks the chip holds at one per CU, so that a node's
+// serial walk over its edges is shared by idle SIMDs.  Exact stage kernel of 11
+// to 40 patches: 9.5-12.3 us whole with one lane per node, 7.2-8.4 us as
+// quarters with four; 106 patches as halves 10.3 us with four lanes, 11.5 with
+// two; 145 whole patches 11.4 us with two lanes, 12.5 with one, 13.7 with
+// four.  At more than a block per CU the lanes only add waves to busy SIMDs:
+// 434 whole patches 22.5 us with two, 17.7 with one.
+template <typename F>
+static int with_gather_shape(bool exact, const InvPlan& P, F&& f)
 {
     static_assert(kHaloCap <= 2 * kBlock, "two halo nodes per thread");
-    if (P.bk_max_halo <= kBlock)
-        return exact ? launch_blocked_nh<true, 1>(P, var, flux, status, fresh)
-                     : launch_blocked_nh<false, 1>(P, var, flux, status, fresh);
-    return exact ? launch_blocked_nh<true, 2>(P, var, flux, status, fresh)
-                 : launch_blocked_nh<false, 2>(P, var, flux, status, fresh);
+    auto shape = [&](auto pn, auto lpn) -> int {
+        constexpr int T = decltype(pn)::value * decltype(lpn)::value;
+        std::integral_constant<int, 1> one;
+        std::integral_constant<int, (kHaloCap + T - 1) / T> all;
+        if (P.bk_max_halo <= T) return exact ? f(std::true_type{}, one, pn, lpn) : f(std::false_type{}, one, pn, lpn);
+        return exact ? f(std::true_type{}, all, pn, lpn) : f(std::false_type{}, all, pn, lpn);
+    };
+    if (P.bk_blocks <= R.n_cu) {
+        if (P.bk_max_cnt <= kPart / 4) return shape(std::integral_constant<int, kPart / 4>{}, std::integral_constant<int, 4>{});
+        if (P.bk_max_cnt <= kPart / 2) return shape(std::integral_constant<int, kPart / 2>{}, std::integral_constant<int, 4>{});
+        return shape(std::integral_constant<int, kPart>{}, std::integral_constant<int, 2>{});
+    }
+    return shape(std::integral_constant<int, kPart>{}, std::integral_constant<int, 1>{});
+}
+
+static int launch_blocked_pf(bool exact, const InvPlan& P, op_dat var, op_dat flux, const int* status, int fresh)
+{
+    return with_gather_shape(exact, P, [&](auto ex, auto nh, auto pn, auto lpn) -> int {
+        constexpr int PN = decltype(pn)::value, LPN = decltype(lpn)::value;
+        k_flux_blocked_pf<decltype(ex)::value, LPN == 1 ? 4 : 2, decltype(nh)::value, PN, LPN>
+            <<<P.bk_blocks, PN * LPN, P.bk_lds, cur_stream()>>>(gather_plan(P), dptr(var), dptr(flux), R.k, status,
+                                                            fresh);
+        return check_launch();
+    });
 }
 
 // The stage fused into a part kernel (k_flux_part_stage): its input state,
@@ -1561,15 +1659,15 @@ struct PartStage {
     const int* pfirst = nullptr;
 };
 
-template <typename Real, int T, int EPT, int NPT, int RS, bool COLOURED>
+template <typename Real, int T, int PN, int EPT, int NPT, int RS, bool COLOURED>
 static int launch_part_c(const InvPlan& P, const Real* w, size_t lds, op_dat var, op_dat flux, const int* status,
                          int fresh, const PartStage* st)
 {
     if (st) {
         // records, accumulators and one step factor per owned node
-        lds = sizeof(double) * (part_rec_doubles<Real, RS>(P.pt_rec_cap) + 6 * (size_t)kPart);
+        lds = sizeof(double) * (part_rec_doubles<Real, RS>(P.pt_rec_cap) + 6 * (size_t)PN);
         const int pw = 8 * ((R.n_cu * P.pt_persist + 7) / 8);    // persistent grid: a multiple of the 8 XCDs
-        if constexpr (T <= 512) {
+        if constexpr (T <= 512 && PN == kPart) {
             if (P.pt_persist > 0 && pw < P.pt_parts) {
                 k_flux_part_stage_persistent<Real, T, EPT, NPT, COLOURED, RS><<<pw, T, lds, cur_stream()>>>(
                     P.d_pt_info, P.d_pt_halo, P.d_pt_code, w, P.pt_nloc, P.pt_rec_cap, st->vin, fresh, *st->a, R.k,
@@ -1577,12 +1675,12 @@ static int launch_part_c(const InvPlan& P, const Real* w, size_t lds, op_dat var
                 return check_launch();
             }
         }
-        k_flux_part_stage<Real, T, EPT, NPT, COLOURED, RS><<<P.pt_parts, T, lds, cur_stream()>>>(
+        k_flux_part_stage<Real, T, EPT, NPT, COLOURED, RS, PN><<<P.pt_parts, T, lds, cur_stream()>>>(
             P.d_pt_info, st->pseg, st->pfirst, P.d_pt_halo, P.d_pt_code, w, P.pt_nloc, P.pt_rec_cap, st->vin, fresh,
             *st->a, R.k);
         return check_launch();
     }
-    if constexpr (T <= 512) {
+    if constexpr (T <= 512 && PN == kPart) {
         k_flux_part<Real, T, EPT, NPT, COLOURED, RS><<<P.pt_parts, T, lds, cur_stream()>>>(
             P.d_pt_info, P.d_pt_halo, P.d_pt_code, w, P.pt_nloc, P.pt_rec_cap, dptr(var), dptr(flux), R.k, status,
             fresh);
@@ -1591,33 +1689,33 @@ static int launch_part_c(const InvPlan& P, const Real* w, size_t lds, op_dat var
     return fail("internal error: edge flux with %d threads per part", T);
 }
 
-template <typename Real, int T, int EPT, int NPT, int RS>
+template <typename Real, int T, int PN, int EPT, int NPT, int RS>
 static int launch_part_rs(bool coloured, const InvPlan& P, const Real* w, size_t lds, op_dat var, op_dat flux,
                           const int* status, int fresh, const PartStage* st)
 {
-    return coloured ? launch_part_c<Real, T, EPT, NPT, RS, true>(P, w, lds, var, flux, status, fresh, st)
-                    : launch_part_c<Real, T, EPT, NPT, RS, false>(P, w, lds, var, flux, status, fresh, st);
+    return coloured ? launch_part_c<Real, T, PN, EPT, NPT, RS, true>(P, w, lds, var, flux, status, fresh, st)
+                    : launch_part_c<Real, T, PN, EPT, NPT, RS, false>(P, w, lds, var, flux, status, fresh, st);
 }
 
 // Record size: FP32 records have six values; FP64 ones the plan's pt_rs in
 // the edge-flux kernel, and five in the kernel with the fused stage (its
 // epilogue makes each workgroup longer, and 40-byte records, staging no
 // wave speeds, shorten it: a 300K-node cycle 0.440 -> 0.418 ms).
-template <typename Real, int T, int EPT, int NPT>
+template <typename Real, int T, int PN, int EPT, int NPT>
 static int launch_part_t(bool coloured, const InvPlan& P, const Real* w, size_t lds, op_dat var, op_dat flux,
                          const int* status, int fresh, const PartStage* st)
 {
     if constexpr (sizeof(Real) == sizeof(double)) {
         if (P.pt_rs == 5 || st)
-            return launch_part_rs<Real, T, EPT, NPT, 5>(coloured, P, w, lds, var, flux, status, fresh, st);
+            return launch_part_rs<Real, T, PN, EPT, NPT, 5>(coloured, P, w, lds, var, flux, status, fresh, st);
     }
-    return launch_part_rs<Real, T, EPT, NPT, kPRec>(coloured, P, w, lds, var, flux, status, fresh,
+    return launch_part_rs<Real, T, PN, EPT, NPT, kPRec>(coloured, P, w, lds, var, flux, status, fresh,
                                                                     st);
 }
 
 // Staged nodes per thread: the smaller register array when the part plan's
 // largest part allows it.
-template <typename Real, int T, int EPT>
+template <typename Real, int T, int PN, int EPT>
 static int launch_part_e(bool coloured, const InvPlan& P, const Real* w, size_t lds, op_dat var, op_dat flux,
                          const int* status, int fresh, const PartStage* st)
 {
@@ -1625,20 +1723,25 @@ static int launch_part_e(bool coloured, const InvPlan& P, const Real* w, size_t 
     static_assert(kPartSlots <= kLarge * T, "staged nodes exceed the kernel's registers");
     // the kernel with the fused stage gathers only the halo node by node
     if ((st ? P.pt_halo_cap : P.pt_rec_cap) <= kSmall * T)
-        return launch_part_t<Real, T, EPT, kSmall>(coloured, P, w, lds, var, flux, status, fresh, st);
-    return launch_part_t<Real, T, EPT, kLarge>(coloured, P, w, lds, var, flux, status, fresh, st);
+        return launch_part_t<Real, T, PN, EPT, kSmall>(coloured, P, w, lds, var, flux, status, fresh, st);
+    return launch_part_t<Real, T, PN, EPT, kLarge>(coloured, P, w, lds, var, flux, status, fresh, st);
 }
 
 // Edges per thread from the plan's largest part.
-template <typename Real, int T>
+template <typename Real, int T, int PN = kPart>
 static int launch_part_n(bool coloured, const InvPlan& P, const Real* w, size_t lds, op_dat var, op_dat flux,
                          const int* status, int fresh, const PartStage* st)
 {
-    const int ept = (P.pt_max_ne + T - 1) / T;
-    if (ept <= 1024 / T) return launch_part_e<Real, T, 1024 / T>(coloured, P, w, lds, var, flux, status, fresh, st);
-    if (ept <= 1536 / T) return launch_part_e<Real, T, 1536 / T>(coloured, P, w, lds, var, flux, status, fresh, st);
-    if (ept <= 2048 / T) return launch_part_e<Real, T, 2048 / T>(coloured, P, w, lds, var, flux, status, fresh, st);
-    if (ept <= 3072 / T) return launch_part_e<Real, T, 3072 / T>(coloured, P, w, lds, var, flux, status, fresh, st);
+    const int ne = P.pt_max_ne;
+    auto with = [&](auto ept) -> int {
+        return launch_part_e<Real, T, PN, decltype(ept)::value>(coloured, P, w, lds, var, flux, status, fresh, st);
+    };
+    if constexpr (PN < kPart)
+        if (ne <= 2 * T) return with(std::integral_constant<int, 2>{});
+    if (ne <= 1024) return with(std::integral_constant<int, 1024 / T>{});
+    if (1536 % T == 0 && ne <= 1536) return with(std::integral_constant<int, (1536 + T - 1) / T>{});
+    if (ne <= 2048) return with(std::integral_constant<int, 2048 / T>{});
+    if (ne <= 3072) return with(std::integral_constant<int, 3072 / T>{});
     return fail("edge-flux part plan: %d local edges in one part exceed the kernel's %d", P.pt_max_ne, 3072);
 }
 
@@ -1658,15 +1761,16 @@ static int launch_part(bool coloured, const InvPlan& P, const Real* w, size_t ld
     if (st) {
         // A level with few parts is one workgroup's latency: where the chip
         // holds them all at once, more threads share a part's edges (results
-        // do not depend on it).  Stage kernel of 11-40 parts 8.1-8.9 us with
-        // 256 threads, 7.7-8.0 with 1024; 106-215 parts 9.4-9.8 -> 8.5-8.8;
-        // 317 and 434 parts 13.9 -> 12.9 with 512.  Beyond two parts per CU
-        // 256 threads are as fast (645 parts) or faster (1172 parts and up).
-        const int threads = P.pt_threads             ? P.pt_threads
-                            : P.pt_parts <= R.n_cu     ? 1024
-                            : P.pt_parts <= 2 * R.n_cu ? 512
-                                                       : 256;
-        if (threads == 1024) return launch_part_n<Real, 1024>(coloured, P, w, lds, var, flux, status, fresh, st);
+        // do not depend on it).  Stage kernel of 106-215 parts of 256 nodes
+        // 9.4-9.8 us with 256 threads, 8.5-8.8 with 1024; 317 and 434 parts
+        // 13.9 -> 12.9 with 512.  Beyond two parts per CU 256 threads are as
+        // fast (645 parts) or faster (1172 parts and up).
+        if (!P.pt_threads && P.pt_parts <= R.n_cu) {
+            if (P.pt_max_cnt <= kPart / 4) return launch_part_n<Real, 256, kPart / 4>(coloured, P, w, lds, var, flux, status, fresh, st);
+            if (P.pt_max_cnt <= kPart / 2) return launch_part_n<Real, 512, kPart / 2>(coloured, P, w, lds, var, flux, status, fresh, st);
+            return launch_part_n<Real, 1024>(coloured, P, w, lds, var, flux, status, fresh, st);
+        }
+        const int threads = P.pt_threads ? P.pt_threads : P.pt_parts <= 2 * R.n_cu ? 512 : 256;
         if (threads == 512) return launch_part_n<Real, 512>(coloured, P, w, lds, var, flux, status, fresh, st);
         return launch_part_n<Real, 256>(coloured, P, w, lds, var, flux, status, fresh, st);
     }
@@ -1696,27 +1800,24 @@ static bool fused_stage_variant(int v) { return gather_variant(v) || part_stage_
 // Workgroups of a variant's kernel with the fused stage, and the first node
 // and node count of each.
 static int stage_blocks(int variant, const InvPlan& P) { return gather_variant(variant) ? P.bk_blocks : P.pt_parts; }
+static int stage_groups(int variant, const InvPlan& P) { return gather_variant(variant) ? P.bk_groups : P.pt_groups; }
 static unsigned stage_gen(int variant, const InvPlan& P) { return gather_variant(variant) ? P.bk_gen : P.pt_gen; }
 static int2 stage_nodes(int variant, const InvPlan& P, int k)
 {
     return gather_variant(variant) ? P.h_bk_node[k] : make_int2(P.h_pt_info[k].n0, P.h_pt_info[k].cnt);
 }
 
-template <bool EXACT, int NH>
-static int launch_gather_stage_nh(const InvPlan& P, const PartStage& st, int fresh)
-{
-    // records, then (in the same space) five fluxes and a factor per node
-    const size_t lds = std::max(P.bk_lds, sizeof(double) * 6 * (size_t)kPart);
-    k_gather_stage<EXACT, 4, NH><<<P.bk_blocks, kBlock, lds, cur_stream()>>>(gather_plan(P), st.pseg, st.pfirst,
-                                                                         st.vin, fresh, *st.a, R.k);
-    return check_launch();
-}
-
 static int launch_gather_stage(bool exact, const InvPlan& P, const PartStage& st, int fresh)
 {
-    if (P.bk_max_halo <= kBlock)
-        return exact ? launch_gather_stage_nh<true, 1>(P, st, fresh) : launch_gather_stage_nh<false, 1>(P, st, fresh);
-    return exact ? launch_gather_stage_nh<true, 2>(P, st, fresh) : launch_gather_stage_nh<false, 2>(P, st, fresh);
+    return with_gather_shape(exact, P, [&](auto ex, auto nh, auto pn, auto lpn) -> int {
+        constexpr int PN = decltype(pn)::value, LPN = decltype(lpn)::value;
+        // records, then (in the same space) five fluxes and a factor per node
+        const size_t lds = std::max(P.bk_lds, sizeof(double) * 6 * (size_t)PN);
+        k_gather_stage<decltype(ex)::value, LPN == 1 ? 4 : 2, decltype(nh)::value, PN, LPN>
+            <<<P.bk_blocks, PN * LPN, lds, cur_stream()>>>(gather_plan(P), st.pseg, st.pfirst, st.vin, fresh, *st.a,
+                                                       R.k);
+        return check_launch();
+    });
 }
 
 static int launch_flux_stage(int variant, op_map map, const PartStage& st, int fresh)

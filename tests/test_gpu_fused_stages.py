@@ -88,36 +88,43 @@ def test_fused_solve(rt, n, deg, variant):
             assert not s.state(l, "fluxes").any(), f"level {l}: flux not zero after the run"
 
 
-def test_blocked_plan_keeps_parts_whole(rt):
-    """Parts with more than 256 and at most 448 halo nodes are one block each;
-    a part beyond that is split."""
+def test_blocked_plan_blocks(rt):
+    """Blocks of the blocked plan: whole 256-node patches where their halo has
+    more than 256 and at most 448 nodes, quarters on a level of few patches,
+    and smaller ones where the halo is beyond that."""
     import ctypes as C
 
-    def stats(mesh):
+    def stats(mesh, level):
         s = mgcfd.Solver(rt, mesh, 0.5, 3.0)
         st = (C.c_int * 5)()
-        mgcfd._check(rt.L.mgcfd_plan_stats(s.lv[0].edge_to_node, st), "mgcfd_plan_stats")
+        mgcfd._check(rt.L.mgcfd_plan_stats(s.lv[level].edge_to_node, st), "mgcfd_plan_stats")
         return list(st)
 
-    whole = stats(random_mesh(1100, 2, seed=1102))
-    assert whole[0] == 5 and 512 < whole[1] <= 704 and whole[4] == 80 * whole[1]
-    split = stats(random_mesh(1500, 12, seed=1512))
-    assert split[0] > 6 and split[1] <= 704
+    mesh = mgcfd.mesh_knn(70000, 217000, 2, seed=3)
+    whole = stats(mesh, 1)
+    assert whole[0] == -(-len(mesh[1]["coords"]) // 256) and 512 < whole[1] <= 704 and whole[4] == 80 * whole[1]
+    quarter = stats(random_mesh(1100, 2, seed=1102), 0)
+    assert quarter[0] == 18 and quarter[1] <= 64 + 128
+    split = stats(random_mesh(1500, 12, seed=1512), 0)
+    assert split[0] > 24 and split[1] <= 704
 
 
 @pytest.mark.parametrize("variant", ["part_coloured", "mixed_coloured"])
-@pytest.mark.parametrize("n,deg", [(257, 6), (1300, 4)])
-def test_threads_per_part_change_nothing(rt, n, deg, variant):
-    """Levels with few parts run more threads per part; a deterministic
-    variant's state and RMS history do not depend on it, bit for bit."""
+@pytest.mark.parametrize("n,deg", [(257, 6), (1100, 2), (1300, 4)])
+def test_part_shapes_change_nothing(rt, n, deg, variant):
+    """Levels with few parts run smaller parts and more threads per part; a
+    deterministic variant's state and RMS history do not depend on it, bit for
+    bit."""
     mesh = random_mesh(n, deg, seed=n + deg)
     got = []
-    for threads in (0, 256, 512):       # 0: by the number of parts (here 1024 threads)
+    # None: as the number of parts selects (64 nodes, 256 threads here)
+    for config in (None, (256, 0), (256, 256), (256, 512), (128, 0), (128, 256), (64, 512)):
         s = mgcfd.Solver(rt, mesh, 0.5, 3.0)
         s.setup()
         rt.upload(s.lv[0].variables, perturbed_state(n, s.fs["ff_variable"], seed=5))
         for l in range(2):
-            rt.map_part_config(s.lv[l].edge_to_node, 256, threads)
+            if config:
+                rt.map_part_config(s.lv[l].edge_to_node, *config)
         rt.set_flux_variant(mgcfd.FLUX_VARIANTS[variant])
         st, rms = s.run_device(3)
         assert st == 0
@@ -125,6 +132,26 @@ def test_threads_per_part_change_nothing(rt, n, deg, variant):
     for other in got[1:]:
         for a, b in zip(got[0], other):
             assert np.array_equal(a.view(np.uint64), b.view(np.uint64))
+
+
+@pytest.mark.parametrize("variant", ["gather_exact", "part_coloured", "mixed_coloured"])
+@pytest.mark.parametrize("others", [1, 40, 90, 200])
+def test_small_mesh_alone_and_in_a_batch(rt, others, variant):
+    """Alone a small mesh's levels run quarter patches; beside others the batch
+    has more patches and the shapes change (half and whole patches, fewer
+    lanes and threads): its states and RMS history stay the same, bit for bit."""
+    small, other = mgcfd.mesh_knn(1500, 4600, 2, seed=3), mgcfd.mesh_knn(700, 2100, 2, seed=4)
+
+    def result(meshes):
+        b = mgcfd.Batch(rt, meshes, [0.5] * len(meshes), [3.0] * len(meshes), variant)
+        st, rms = b.run(5)
+        out = [b.fetch(0, 0), b.fetch(0, 1), rms[0].copy()]
+        b.close()
+        assert not st.any()
+        return out
+
+    for a, b in zip(result([small]), result([small] + [other] * others)):
+        assert np.array_equal(a.view(np.uint64), b.view(np.uint64))
 
 
 @pytest.mark.parametrize("variant", ["gather_exact", "part_coloured", "part_atomic", "nodal_exact"])
