@@ -424,11 +424,15 @@ __device__ __forceinline__ void gather_block(const GatherPlan& G, const BlkInfo&
     int hn[NH];
     double x[FL], U[NH][5];
 #pragma unroll
-    for (int k = 0; k < NH; k++) hn[k] = G.halo[B.h0 + min(t + k * T, hmax)];
+    for (int k = 0; k < NH; k++) hn[k] = (G.halo + B.h0)[min((unsigned)t + k * T, (unsigned)hmax)];
+    // uniform bases and small per-lane indexes: no 64-bit address arithmetic per
+    // lane (cycle of a 300K-node solve 450 -> 424 us)
+    const double* xin = vin + base;
 #pragma unroll
-    for (int i = 0; i < FL; i++) x[i] = vin[base + min(t + i * T, last)];
-    const int nd = B.n0 + min(n, B.cnt - 1);
-    const int deg = own ? G.nptr[nd + 1] - G.nptr[nd] : 0;
+    for (int i = 0; i < FL; i++) x[i] = xin[min((unsigned)t + i * T, (unsigned)last)];
+    const int* np = G.nptr + B.n0;
+    const unsigned nd = min((unsigned)n, (unsigned)B.cnt - 1u);
+    const int deg = own ? np[nd + 1] - np[nd] : 0;
     const int jb = B.j0 + n;
     const int* jp = G.jpref + B.p0;
     IncChunk<CH> A, C;
@@ -1704,7 +1708,7 @@ __global__ __launch_bounds__(PN * LPN) void k_gather_stage(GatherPlan G, const i
     }
     double old[FL];
 #pragma unroll
-    for (int i = 0; i < FL; i++) old[i] = a.old[base + min(t + i * T, last)];
+    for (int i = 0; i < FL; i++) old[i] = (a.old + base)[min((unsigned)t + i * T, (unsigned)last)];
     double f = 0.0;
     if (head) {
         if (q0 < q1) {
