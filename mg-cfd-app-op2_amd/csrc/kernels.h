@@ -708,75 +708,6 @@ __device__ __forceinline__ void part_ready(const V& v)
     asm volatile("" ::"v"(v));
 }
 
-// Staging of one part, shared by the part kernels: node slot sl = t + k T
-// (k < NPT, NPT * T >= rec_cap) of the owned nodes [0, cnt) and the halo
-// nodes [cnt, cnt + nh).  The halo-list loads are unconditional (clamped into
-// the part's list, which the plan pads by one entry) so that they issue back
-// to back under one wait instead of one wait per divergent branch; every
-// slot then names a valid node, so the state loads are unconditional too.
-template <int T, int NPT>
-__device__ __forceinline__ void part_halo_entries(const PartInfo& P, const int* __restrict__ halo, int t,
-                                                  int nd[NPT])
-{
-    const int hmax = max(P.nh - 1, 0);
-#pragma unroll
-    for (int k = 0; k < NPT; k++) nd[k] = halo[P.h0 + min(max(t + k * T - P.cnt, 0), hmax)];
-}
-
-template <int T, int NPT>
-__device__ __forceinline__ void part_load_nodes(const PartInfo& P, const double* __restrict__ var, int t,
-                                                int nd[NPT], double U[NPT][5])
-{
-#pragma unroll
-    for (int k = 0; k < NPT; k++) {
-        part_ready(nd[k]);
-        const int sl = t + k * T;
-        nd[k] = sl < P.cnt ? P.n0 + sl : nd[k];
-    }
-#pragma unroll
-    for (int k = 0; k < NPT; k++)
-#pragma unroll
-        for (int v = 0; v < 5; v++) U[k][v] = var[(size_t)nd[k] * 5 + v];
-}
-
-// Records {rho, m, E, |u| + c} of the staged slots.
-template <typename R, int T, int NPT, int RS>
-__device__ __forceinline__ void part_store_records(const PartInfo& P, int t, const double U[NPT][5], R* rec)
-{
-    const int nrec = P.cnt + P.nh;
-#pragma unroll
-    for (int k = 0; k < NPT; k++) {
-        const int sl = t + k * T;
-        if (sl < nrec) {
-            const R x0 = (R)U[k][0], x1 = (R)U[k][1], x2 = (R)U[k][2], x3 = (R)U[k][3], x4 = (R)U[k][4];
-            R* r = rec + sl * part_stride<R, RS>();
-            r[0] = x0; r[1] = x1; r[2] = x2; r[3] = x3; r[4] = x4;
-            if constexpr (RS > 5) r[5] = part_speed<R>(x0, x1, x2, x3, x4);
-        }
-    }
-}
-
-// The owned nodes' old flux (FL flat entries per thread), or zeros for a
-// fresh start, into the FP64 accumulators.
-template <int T, int FL>
-__device__ __forceinline__ void part_load_flux(const PartInfo& P, const double* __restrict__ flux, int t,
-                                               bool fresh, double fl[FL])
-{
-    const double* fo = flux + (size_t)P.n0 * 5;
-#pragma unroll
-    for (int i = 0; i < FL; i++) fl[i] = fresh ? 0.0 : fo[min(t + i * T, P.cnt * 5 - 1)];
-}
-
-template <int T, int FL>
-__device__ __forceinline__ void part_store_flux(const PartInfo& P, int t, const double fl[FL], double* acc)
-{
-#pragma unroll
-    for (int i = 0; i < FL; i++) {
-        const int j = t + i * T;
-        if (j < P.cnt * 5) acc[j] = fl[i];
-    }
-}
-
 // Local-edge codes and weights of one part, EPT per thread (code 0: none).
 template <typename R, int T, int EPT>
 __device__ __forceinline__ void part_load_edges(const PartInfo& P, const unsigned* __restrict__ ecode,
@@ -859,59 +790,126 @@ __device__ __forceinline__ void part_edges(const PartInfo& P, const R* rec, doub
     }
 }
 
-// Stages one part and accumulates its local edges: returns the FP64
-// accumulators (in LDS, after a barrier) holding the edge flux of the part's
-// owned nodes, started from the flux dat or, with fresh, from zero.
-template <typename R, int T, int EPT, int NPT, bool COLOURED, int RS>
-__device__ __forceinline__ double* part_accumulate(const PartInfo& P, const int* __restrict__ halo,
-                                                   const unsigned* __restrict__ ecode, const R* __restrict__ ew,
-                                                   long long nloc, int rec_cap, const double* __restrict__ var,
-                                                   const double* __restrict__ flux, const Consts& k, int fresh,
-                                                   double* sm)
+// Staging of one part, shared by the part kernels.  The owned nodes' state
+// arrives as one run of 5 * cnt doubles (x, FL per thread), the halo node by
+// node (NPT per thread); all loads are clamped into the part (the plan pads
+// the halo list by one entry), so that they issue without branches and under
+// few waits.  part_records writes the records (RS 6: without the owned nodes'
+// wave speeds).
+template <int T, int NPT>
+__device__ __forceinline__ void part_load_halo(const PartInfo& P, const int* __restrict__ halo, int t, int nd[NPT])
 {
-    constexpr int FL = (5 * kPart + T - 1) / T;
-    const int t = threadIdx.x;
-    R* rec = reinterpret_cast<R*>(sm);
-    double* acc = sm + part_rec_doubles<R, RS>(rec_cap);
-    // 1. loads: halo entries, edge codes and weights, then node states and
-    // the owned flux; records (with |u| + c) and accumulators into LDS
-    int nd[NPT];
-    unsigned code[EPT];
-    R w0[EPT], w1[EPT], w2[EPT];
-    double U[NPT][5], fl[FL];
-    part_halo_entries<T, NPT>(P, halo, t, nd);
-    part_load_edges<R, T, EPT>(P, ecode, ew, nloc, t, code, w0, w1, w2);
-    part_load_nodes<T, NPT>(P, var, t, nd, U);
-    part_load_flux<T, FL>(P, flux, t, fresh != 0, fl);
-    part_store_records<R, T, NPT, RS>(P, t, U, rec);
-    part_store_flux<T, FL>(P, t, fl, acc);
-    __syncthreads();
-    // 2./3. edges
-    part_edges<R, EPT, COLOURED, RS, false>(P, rec, acc, code, w0, w1, w2, (R)k.sc);
-    return acc;
+    const int hmax = max(P.nh - 1, 0);
+#pragma unroll
+    for (int k = 0; k < NPT; k++) nd[k] = halo[P.h0 + min(t + k * T, hmax)];
+}
+
+template <typename R, int T, int NPT, int FL, int RS>
+__device__ __forceinline__ void part_records(const PartInfo& P, int t, const double x[FL], const double U[NPT][5],
+                                             R* rec)
+{
+    constexpr int ST = part_stride<R, RS>();
+    const int last = 5 * P.cnt - 1;
+#pragma unroll
+    for (int i = 0; i < FL; i++) {
+        const int j = t + i * T;
+        if (j <= last) rec[ST == 5 ? j : j + j / 5] = (R)x[i];
+    }
+#pragma unroll
+    for (int k = 0; k < NPT; k++)
+        if (t + k * T < P.nh) {
+            R* r = rec + (P.cnt + t + k * T) * ST;
+#pragma unroll
+            for (int v = 0; v < 5; v++) r[v] = (R)U[k][v];
+            if constexpr (RS == 6) r[5] = part_speed<R>(r[0], r[1], r[2], r[3], r[4]);
+        }
+}
+
+// Staging of the edge-flux kernel with six-value records: owned and halo nodes
+// alike node by node (slot t + k T, NPT * T >= rec_cap), so that each thread
+// forms its nodes' wave speeds from registers and one barrier suffices.  (As
+// runs, with the owned wave speeds formed behind a second barrier, mixed
+// precision takes 14.8 us on 930K edges against 14.0, FP64 18.4 against 18.0.)
+template <int T, int NPT>
+__device__ __forceinline__ void part_slot_entries(const PartInfo& P, const int* __restrict__ halo, int t, int nd[NPT])
+{
+    const int hmax = max(P.nh - 1, 0);
+#pragma unroll
+    for (int k = 0; k < NPT; k++) nd[k] = halo[P.h0 + min(max(t + k * T - P.cnt, 0), hmax)];
+}
+
+template <typename R, int T, int NPT>
+__device__ __forceinline__ void part_slot_records(const PartInfo& P, int t, const double U[NPT][5], R* rec)
+{
+    const int nrec = P.cnt + P.nh;
+#pragma unroll
+    for (int k = 0; k < NPT; k++)
+        if (t + k * T < nrec) {
+            R* r = rec + (t + k * T) * part_stride<R, 6>();
+            const R x0 = (R)U[k][0], x1 = (R)U[k][1], x2 = (R)U[k][2], x3 = (R)U[k][3], x4 = (R)U[k][4];
+            r[0] = x0; r[1] = x1; r[2] = x2; r[3] = x3; r[4] = x4;
+            r[5] = part_speed<R>(x0, x1, x2, x3, x4);
+        }
 }
 
 // LDS: R records [rec_cap * 6] (rounded up to doubles), then FP64
 // accumulators [cnt * 5].  R = double: the FP64 kernel; R = float: mixed
 // precision (records, weights and increment arithmetic in FP32, each
 // increment converted to FP64 and accumulated in FP64 from the FP64 flux).
-// One workgroup per part; NPT staged nodes per thread (NPT * T >= rec_cap);
-// RS values per record.
+// One workgroup per part; RS values per record; NPT: halo nodes per thread
+// (RS 5) or staged nodes per thread (RS 6).
 template <typename R, int T, int EPT, int NPT, bool COLOURED, int RS>
 __global__ __launch_bounds__(T) void k_flux_part(
     const PartInfo* __restrict__ parts, const int* __restrict__ halo, const unsigned* __restrict__ ecode,
     const R* __restrict__ ew, long long nloc, int rec_cap, const double* __restrict__ var,
     double* __restrict__ flux, Consts k, const int* __restrict__ status, int fresh)
 {
+    constexpr int FL = (5 * kPart + T - 1) / T;
     extern __shared__ double sm[];
     const int halt = status_of(status);     // tested before the store
     const PartInfo P = parts[xcd_block()];
-    const double* acc =
-        part_accumulate<R, T, EPT, NPT, COLOURED, RS>(P, halo, ecode, ew, nloc, rec_cap, var, flux, k, fresh, sm);
+    const int t = threadIdx.x;
+    R* rec = reinterpret_cast<R*>(sm);
+    double* acc = sm + part_rec_doubles<R, RS>(rec_cap);
+    const int last = 5 * P.cnt - 1;
+    const size_t base = (size_t)P.n0 * 5;
+    // 1. loads: halo entries, owned states, edge codes and weights, then halo
+    // states and the owned flux; records and accumulators into LDS
+    int nd[NPT];
+    unsigned code[EPT];
+    R w0[EPT], w1[EPT], w2[EPT];
+    double x[FL], fl[FL], U[NPT][5];
+    if constexpr (RS == 6) {
+        part_slot_entries<T, NPT>(P, halo, t, nd);
+    } else {
+        part_load_halo<T, NPT>(P, halo, t, nd);
+#pragma unroll
+        for (int i = 0; i < FL; i++) x[i] = var[base + min(t + i * T, last)];
+    }
+    part_load_edges<R, T, EPT>(P, ecode, ew, nloc, t, code, w0, w1, w2);
+#pragma unroll
+    for (int q = 0; q < NPT; q++) {
+        part_ready(nd[q]);
+        if (RS == 6) nd[q] = t + q * T < P.cnt ? P.n0 + t + q * T : nd[q];
+    }
+#pragma unroll
+    for (int q = 0; q < NPT; q++)
+#pragma unroll
+        for (int v = 0; v < 5; v++) U[q][v] = var[(size_t)nd[q] * 5 + v];
+#pragma unroll
+    for (int i = 0; i < FL; i++) fl[i] = fresh ? 0.0 : flux[base + min(t + i * T, last)];
+    if constexpr (RS == 6) part_slot_records<R, T, NPT>(P, t, U, rec);
+    else part_records<R, T, NPT, FL, RS>(P, t, x, U, rec);
+#pragma unroll
+    for (int i = 0; i < FL; i++)
+        if (t + i * T <= last) acc[t + i * T] = fl[i];
+    __syncthreads();
+    // 2./3. edges
+    part_edges<R, EPT, COLOURED, RS, false>(P, rec, acc, code, w0, w1, w2, (R)k.sc);
     if (halt) return;
     // 4. store
-    double* fw = flux + (size_t)P.n0 * 5;
-    for (int j = threadIdx.x; j < P.cnt * 5; j += T) fw[j] = acc[j];
+    double* fw = flux + base;
+    for (int j = t; j <= last; j += T) fw[j] = acc[j];
 }
 
 // Local-edge weights of the part kernels (Real: FP64, or FP32 for mixed
@@ -1317,31 +1315,33 @@ __global__ __launch_bounds__(kBlock) void k_calc_dt(
     if (pub.slots) min_publish(pub, 0, blockIdx.x, block_min(d));
 }
 
-// get_min_dt_kernel as a standalone loop: per-workgroup min of dt.
+// The standalone reduction loops (get_min_dt, calc_rms, the counts): every
+// workgroup of a grid of bounded size reduces a strided share and leaves one
+// partial result -- in pinned host memory, where the host combines them after
+// the one synchronisation the loop needs anyway (no second kernel, no copy).
+constexpr int kRedBlocks = 1024;
+
+// get_min_dt_kernel: per-workgroup min of dt.
 __global__ __launch_bounds__(kBlock) void k_min_part(int n, const double* __restrict__ x,
                                                       double* __restrict__ part)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const double d = (i < n) ? min_candidate(x[i]) : DBL_MAX;
+    double d = DBL_MAX;
+    for (long long i = (long long)blockIdx.x * kBlock + threadIdx.x; i < n; i += (long long)gridDim.x * kBlock) {
+        const double y = min_candidate(x[i]);
+        d = (y < d) ? y : d;
+    }
     const double m = block_min(d);
     if (threadIdx.x == 0) part[blockIdx.x] = m;
 }
 
-// Final min over the partials; *out = min(init, partials).  With 'status'
-// set, a negative minimum raises abort code 1 (euler3d.cpp:480-484).
-__global__ __launch_bounds__(kBlock) void k_min_final(int np, const double* __restrict__ part,
-                                                       double init, double* __restrict__ out,
-                                                       int* __restrict__ status)
+// Final min over device partials; *out = min(init, partials).
+__global__ __launch_bounds__(kBlock) void k_min_final(int np, const double* __restrict__ part, double init,
+                                                       double* __restrict__ out)
 {
-    if (status && *status != 0) return;
     double m = DBL_MAX;
     for (int i = threadIdx.x; i < np; i += kBlock) m = (part[i] < m) ? part[i] : m;
     m = block_min(m);
-    if (threadIdx.x == 0) {
-        m = (m < init) ? m : init;
-        *out = m;
-        if (status && m < 0.0) *status = 1;
-    }
+    if (threadIdx.x == 0) *out = (m < init) ? m : init;
 }
 
 // compute_step_factor_kernel (time_stepping_kernels.h:43-64): sf = min_dt / V.
@@ -1355,24 +1355,18 @@ __global__ void k_step_factor(int n, const double* __restrict__ vol, const doubl
     sf[i] = m / vol[i];
 }
 
-// time_step_kernel (time_stepping_kernels.h:66-86).
-__global__ void k_time_step(int n, int rk, const double* __restrict__ sf, double* __restrict__ flux,
-                            const double* __restrict__ old, double* __restrict__ var,
-                            const int* __restrict__ status)
+// time_step_kernel (time_stepping_kernels.h:66-86), one thread per double of
+// the [n][5] arrays.
+__global__ __launch_bounds__(kBlock) void k_time_step(long long n5, int rk, const double* __restrict__ sf,
+                                                      double* __restrict__ flux, const double* __restrict__ old,
+                                                      double* __restrict__ var)
 {
 #pragma clang fp contract(off)
-    if (halted(status)) return;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const double factor = sf[i] / (double)(3 + 1 - rk);
-    double f[5], o[5], u[5];
-    load5(flux, i, f);
-    load5(old, i, o);
-#pragma unroll
-    for (int v = 0; v < 5; v++) u[v] = o[v] + factor * f[v];
-    store5(var, i, u);
-    const double z[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    store5(flux, i, z);
+    const long long j = (long long)blockIdx.x * kBlock + threadIdx.x;
+    if (j >= n5) return;
+    const double factor = sf[j / 5] / (double)(3 + 1 - rk);
+    var[j] = old[j] + factor * flux[j];
+    flux[j] = 0.0;
 }
 
 // One Runge-Kutta stage of a multigrid smoothing step after its edge flux,
@@ -1779,9 +1773,7 @@ __device__ __forceinline__ bool part_stage_one(
     unsigned code[EPT];
     R w0[EPT], w1[EPT], w2[EPT];
     double x[FL], o[FL], U[NPT][5];
-    const int hmax = max(P.nh - 1, 0);
-#pragma unroll
-    for (int k = 0; k < NPT; k++) nd[k] = halo[P.h0 + min(t + k * T, hmax)];
+    part_load_halo<T, NPT>(P, halo, t, nd);
 #pragma unroll
     for (int i = 0; i < FL; i++) x[i] = vin[base + min(t + i * T, last)];
     part_load_edges<R, T, EPT>(P, ecode, ew, nloc, t, code, w0, w1, w2);
@@ -1801,19 +1793,9 @@ __device__ __forceinline__ bool part_stage_one(
 #pragma unroll
     for (int i = 0; i < FL; i++) {
         const int j = t + i * T;
-        if (j <= last) {
-            rec[ST == 5 ? j : j + j / 5] = (R)x[i];
-            acc[j] = fresh ? 0.0 : a.flux[base + j];
-        }
+        if (j <= last) acc[j] = fresh ? 0.0 : a.flux[base + j];
     }
-#pragma unroll
-    for (int k = 0; k < NPT; k++)
-        if (t + k * T < P.nh) {
-            R* r = rec + (P.cnt + t + k * T) * ST;
-#pragma unroll
-            for (int v = 0; v < 5; v++) r[v] = (R)U[k][v];
-            if constexpr (RS == 6) r[5] = part_speed<R>(r[0], r[1], r[2], r[3], r[4]);
-        }
+    part_records<R, T, NPT, FL, RS>(P, t, x, U, rec);
     __syncthreads();
     if constexpr (RS == 6) {
         if (t < P.cnt) {
@@ -1893,63 +1875,31 @@ __global__ __launch_bounds__(T) void k_flux_part_stage_persistent(
     }
 }
 
-// residual_kernel (validation.h:27-35); with 'part' set also the per-node
-// sum of squares of calc_rms_kernel (validation.h:37-44) and with 'bad' the
-// NaN/Inf count of count_bad_vals (validation.h:102-115).
-__global__ __launch_bounds__(kBlock) void k_residual(
-    int n, const double* __restrict__ old, const double* __restrict__ var, double* __restrict__ res,
-    double* __restrict__ part, int* __restrict__ bad, const int* __restrict__ status)
+// residual_kernel (validation.h:27-35), one thread per double.
+__global__ __launch_bounds__(kBlock) void k_residual(long long n5, const double* __restrict__ old,
+                                                     const double* __restrict__ var, double* __restrict__ res)
 {
-#pragma clang fp contract(off)
-    if (halted(status)) return;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    double s = 0.0;
-    int nb = 0;
-    if (i < n) {
-        double o[5], u[5], r[5];
-        load5(old, i, o);
-        load5(var, i, u);
-#pragma unroll
-        for (int v = 0; v < 5; v++) {
-            r[v] = u[v] - o[v];
-            s += r[v] * r[v];
-            nb += (isnan(u[v]) || isinf(u[v])) ? 1 : 0;
-        }
-        if (res) store5(res, i, r);
-    }
-    if (part) {
-        const double t = block_sum(s);
-        if (threadIdx.x == 0) part[blockIdx.x] = t;
-    }
-    if (bad) {
-        const int t = block_sum_i(nb);
-        if (threadIdx.x == 0 && t) atomicAdd(bad, t);
-    }
+    const long long j = (long long)blockIdx.x * kBlock + threadIdx.x;
+    if (j < n5) res[j] = var[j] - old[j];
 }
 
-// calc_rms_kernel as a standalone loop (sum of squares per workgroup).
-__global__ __launch_bounds__(kBlock) void k_sumsq_part(int n, const double* __restrict__ r,
+// calc_rms_kernel as a standalone loop: sum of squares of n doubles per
+// workgroup.
+__global__ __launch_bounds__(kBlock) void k_sumsq_part(long long n, const double* __restrict__ r,
                                                         double* __restrict__ part)
 {
 #pragma clang fp contract(off)
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
     double s = 0.0;
-    if (i < n) {
-        double x[5];
-        load5(r, i, x);
-#pragma unroll
-        for (int v = 0; v < 5; v++) s += x[v] * x[v];
-    }
+    for (long long i = (long long)blockIdx.x * kBlock + threadIdx.x; i < n; i += (long long)gridDim.x * kBlock)
+        s += r[i] * r[i];
     const double t = block_sum(s);
     if (threadIdx.x == 0) part[blockIdx.x] = t;
 }
 
-// Final reductions of per-workgroup partials run as one workgroup per sum.
-// Each thread keeps four partial sums over entries NT apart, so four loads
-// are in flight per thread instead of one (a level-0 sum of an 8M-node mesh
-// has 31K partials); the order is fixed, so the sum is deterministic.
-constexpr int kSumBlock = 1024;
-
+// Sum of the partials [lo, hi) by one workgroup.  Each thread keeps four
+// partial sums over entries NT apart, so four loads are in flight per thread
+// instead of one (a level-0 sum of an 8M-node mesh has 125K partials); the
+// order is fixed, so the sum is deterministic.
 template <int NT>
 __device__ __forceinline__ double strided_sum(const double* __restrict__ x, const int* __restrict__ cnt, int lo,
                                               int hi, int& nb)
@@ -1971,17 +1921,6 @@ __device__ __forceinline__ double strided_sum(const double* __restrict__ x, cons
     }
     nb = c;
     return (s0 + s1) + (s2 + s3);
-}
-
-// Sum of partials; *out = init + sum.
-__global__ __launch_bounds__(kSumBlock) void k_sum_final(int np, const double* __restrict__ part, double init,
-                                                          double* __restrict__ out)
-{
-#pragma clang fp contract(off)
-    int unused = 0;
-    double s = strided_sum<kSumBlock>(part, nullptr, 0, np, unused);
-    s = block_sum<kSumBlock>(s);
-    if (threadIdx.x == 0) *out = init + s;
 }
 
 // The device driver's level-0 RMS sqrt(sum / n) of every mesh, stored at
@@ -2025,19 +1964,18 @@ __global__ __launch_bounds__(kBlock) void k_mg_sum(SumArgs a, const int* __restr
     mg_sum(a, blockIdx.x);
 }
 
-__global__ __launch_bounds__(kBlock) void k_count_bad(int n, const double* __restrict__ x,
-                                                       int* __restrict__ out)
+// count_bad_vals (validation.h:102-115) and count_non_zeros
+// (validation.h:91-100) over n doubles: per-workgroup counts.
+template <bool BAD>
+__global__ __launch_bounds__(kBlock) void k_count(long long n, const double* __restrict__ x, int* __restrict__ part)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
     int c = 0;
-    if (i < n) {
-        double u[5];
-        load5(x, i, u);
-#pragma unroll
-        for (int v = 0; v < 5; v++) c += (isnan(u[v]) || isinf(u[v])) ? 1 : 0;
+    for (long long i = (long long)blockIdx.x * kBlock + threadIdx.x; i < n; i += (long long)gridDim.x * kBlock) {
+        const double u = x[i];
+        c += (BAD ? isnan(u) || isinf(u) : u > 0.0) ? 1 : 0;
     }
     c = block_sum_i(c);
-    if (threadIdx.x == 0 && c) atomicAdd(out, c);
+    if (threadIdx.x == 0) part[blockIdx.x] = c;
 }
 
 // identify_differences (validation.h:46-89) fused with count_non_zeros
@@ -2069,21 +2007,6 @@ __global__ __launch_bounds__(kBlock) void k_identify_differences(
         c = block_sum_i(c);
         if (threadIdx.x == 0 && c) atomicAdd(count, c);
     }
-}
-
-__global__ __launch_bounds__(kBlock) void k_count_pos(int n, const double* __restrict__ x,
-                                                       int* __restrict__ out)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    int c = 0;
-    if (i < n) {
-        double u[5];
-        load5(x, i, u);
-#pragma unroll
-        for (int v = 0; v < 5; v++) c += (u[v] > 0.0) ? 1 : 0;
-    }
-    c = block_sum_i(c);
-    if (threadIdx.x == 0 && c) atomicAdd(out, c);
 }
 
 // ------------------------------------------------------------------------
@@ -2145,21 +2068,16 @@ __global__ __launch_bounds__(kBlock) void k_up_gather(
     scratch[c] = cnt;
 }
 
-// up_post_kernel: mean over children (count 0 keeps the value).
-__global__ void k_up_post(int nc, double* __restrict__ vc, const int* __restrict__ scratch,
-                          const int* __restrict__ status)
+// up_post_kernel: mean over children (count 0 keeps the value), one thread per
+// double.
+__global__ __launch_bounds__(kBlock) void k_up_post(long long n5, double* __restrict__ vc,
+                                                    const int* __restrict__ scratch)
 {
 #pragma clang fp contract(off)
-    if (halted(status)) return;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nc) return;
-    const int s = scratch[i];
-    const double avg = s == 0 ? 1.0 : 1.0 / (double)s;
-    double x[5];
-    load5(vc, i, x);
-#pragma unroll
-    for (int v = 0; v < 5; v++) x[v] *= avg;
-    store5(vc, i, x);
+    const long long j = (long long)blockIdx.x * kBlock + threadIdx.x;
+    if (j >= n5) return;
+    const int s = scratch[j / 5];
+    vc[j] *= s == 0 ? 1.0 : 1.0 / (double)s;
 }
 
 // The nodes [lo, lo + cnt) of one transfer workgroup, and its segment.
@@ -2245,33 +2163,6 @@ __global__ __launch_bounds__(kBlock) void k_up_gather_dt(
     min_publish(d.pub, B.seg, b, m);
 }
 
-// down_kernel (prolongation).
-__global__ void k_down(int nf, const int* __restrict__ f2c, double* __restrict__ vf,
-                       const double* __restrict__ rf, const double* __restrict__ xf,
-                       const double* __restrict__ rc, const double* __restrict__ xc,
-                       const int* __restrict__ status)
-{
-#pragma clang fp contract(off)
-    if (halted(status)) return;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nf) return;
-    const int c = f2c[i];
-    const double dx = fabs(xf[3 * (size_t)i] - xc[3 * (size_t)c]);
-    const double dy = fabs(xf[3 * (size_t)i + 1] - xc[3 * (size_t)c + 1]);
-    const double dz = fabs(xf[3 * (size_t)i + 2] - xc[3 * (size_t)c + 2]);
-    const double dm = sqrt(dx * dx + dy * dy + dz * dz);
-    double u[5], r[5], ra[5];
-    load5(vf, i, u);
-    load5(rf, i, r);
-    load5(rc, c, ra);
-    u[0] -= dm * (ra[0] - r[0]);
-    u[1] -= dx * (ra[1] - r[1]);
-    u[2] -= dy * (ra[2] - r[2]);
-    u[3] -= dz * (ra[3] - r[3]);
-    u[4] -= dm * (ra[4] - r[4]);
-    store5(vf, i, u);
-}
-
 // Inverse distance 1 / |p - q| as mg.h:134,147,170,183 form it (exact:
 // no contraction, IEEE square root and division).
 __device__ __forceinline__ double down_v2_idist(const double* __restrict__ p, const double* __restrict__ q)
@@ -2349,7 +2240,7 @@ __global__ void k_down_v2_post(int n, const double* __restrict__ rp, const doubl
     store5(vf, i, u);
 }
 
-// down_kernel (mg.h:66-88) of the device driver.  DT: followed by the fine
+// down_kernel (mg.h:66-88).  DT: followed by the fine
 // level's calculate_dt.  END: the cycle's last kernel, which also moves the
 // cycle counter on.  The fine states and residuals come and go as runs of
 // doubles (consecutive lanes, consecutive doubles); each thread gathers its

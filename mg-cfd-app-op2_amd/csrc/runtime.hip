@@ -170,11 +170,7 @@ struct Runtime {
     std::deque<std::string> names;
     Consts k{};
     int flux_variant = MGCFD_FLUX_GATHER_EXACT;
-    // reduction scratch
-    double* d_part = nullptr;
-    int part_cap = 0;
-    double* d_scal = nullptr;    // [0] min_dt, [1] sum
-    int* d_iscal = nullptr;      // [0] count
+    double* h_red = nullptr;     // partial results of the reduction loops (pinned, kRedBlocks)
     double* h_pin = nullptr;     // pinned host landing zone
     int* h_pini = nullptr;
 };
@@ -231,15 +227,6 @@ static void default_consts()
     R.k.ffmz[0] = R.k.ffmx[2]; R.k.ffmz[1] = R.k.ffmy[2]; R.k.ffmz[2] = uz * R.k.ffv[3] + p;
     const double dep = R.k.ffv[4] + p;
     R.k.ffde[0] = ux * dep; R.k.ffde[1] = uy * dep; R.k.ffde[2] = uz * dep;
-}
-
-static int ensure_part(int nblocks)
-{
-    if (nblocks <= R.part_cap) return 0;
-    if (R.d_part) HIPCHK(hipFree(R.d_part));
-    R.part_cap = std::max(nblocks, 4096);
-    HIPCHK(hipMalloc(&R.d_part, sizeof(double) * R.part_cap));
-    return 0;
 }
 
 static int check_launch()
@@ -1563,6 +1550,9 @@ static int read_scalar(const double* d_src, double* out)
     return 0;
 }
 
+// Workgroups of a reduction loop over n values.
+static int red_blocks(long long n) { return (int)std::min<long long>(kRedBlocks, (n + kBlock - 1) / kBlock); }
+
 static int read_iscalar(const int* d_src, int* out)
 {
     HIPCHK(hipMemcpyAsync(R.h_pini, d_src, sizeof(int), hipMemcpyDeviceToHost, cur_stream()));
@@ -1713,16 +1703,17 @@ static int launch_part_t(bool coloured, const InvPlan& P, const Real* w, size_t 
                                                                     st);
 }
 
-// Staged nodes per thread: the smaller register array when the part plan's
-// largest part allows it.
+// Nodes gathered per thread (the halo, or all staged nodes in the edge-flux
+// kernel with six-value records): the smaller register array when the part
+// plan's largest part allows it.
 template <typename Real, int T, int PN, int EPT>
 static int launch_part_e(bool coloured, const InvPlan& P, const Real* w, size_t lds, op_dat var, op_dat flux,
                          const int* status, int fresh, const PartStage* st)
 {
     constexpr int kSmall = (512 + T - 1) / T, kLarge = (768 + T - 1) / T;
-    static_assert(kPartSlots <= kLarge * T, "staged nodes exceed the kernel's registers");
-    // the kernel with the fused stage gathers only the halo node by node
-    if ((st ? P.pt_halo_cap : P.pt_rec_cap) <= kSmall * T)
+    static_assert(kPartSlots <= kLarge * T, "halo nodes exceed the kernel's registers");
+    const bool slots = !st && (sizeof(Real) == sizeof(float) || P.pt_rs == kPRec);
+    if ((slots ? P.pt_rec_cap : P.pt_halo_cap) <= kSmall * T)
         return launch_part_t<Real, T, PN, EPT, kSmall>(coloured, P, w, lds, var, flux, status, fresh, st);
     return launch_part_t<Real, T, PN, EPT, kLarge>(coloured, P, w, lds, var, flux, status, fresh, st);
 }
@@ -1774,7 +1765,12 @@ static int launch_part(bool coloured, const InvPlan& P, const Real* w, size_t ld
         if (threads == 512) return launch_part_n<Real, 512>(coloured, P, w, lds, var, flux, status, fresh, st);
         return launch_part_n<Real, 256>(coloured, P, w, lds, var, flux, status, fresh, st);
     }
-    if constexpr (sizeof(Real) == 4) return launch_part_n<Real, 512>(coloured, P, w, lds, var, flux, status, fresh, st);
+    // the edge flux alone: FP32 records leave room for two workgroups of 512
+    // threads per CU on any level, FP64 ones are faster so on levels of few
+    // parts (256 -> 512 threads: 10K nodes 3.8 -> 3.5 us, 60K 6.1 -> 5.4,
+    // 125K 8.9 -> 8.0; coloured 5.3 -> 4.6, 8.0 -> 7.2, 10.8 -> 9.8)
+    if (sizeof(Real) == 4 || P.pt_parts <= 2 * R.n_cu)
+        return launch_part_n<Real, 512>(coloured, P, w, lds, var, flux, status, fresh, st);
     return launch_part_n<Real, 256>(coloured, P, w, lds, var, flux, status, fresh, st);
 }
 
@@ -1940,11 +1936,9 @@ int op_init(int argc, char** argv, int diags)
         R.n_cu = std::max(1, prop.multiProcessorCount);
     }
     HIPCHK(hipStreamCreateWithFlags(&R.lib_stream, hipStreamNonBlocking));
-    HIPCHK(hipMalloc(&R.d_scal, 4 * sizeof(double)));
-    HIPCHK(hipMalloc(&R.d_iscal, 4 * sizeof(int)));
+    HIPCHK(hipHostMalloc(&R.h_red, kRedBlocks * sizeof(double), hipHostMallocDefault));
     HIPCHK(hipHostMalloc(&R.h_pin, 8 * sizeof(double), hipHostMallocDefault));
     HIPCHK(hipHostMalloc(&R.h_pini, 8 * sizeof(int), hipHostMallocDefault));
-    TRY(ensure_part(4096));
     default_consts();
     R.inited = true;
     return 0;
@@ -1965,9 +1959,7 @@ void op_exit(void)
     R.maps.clear();
     R.sets.clear();
     R.names.clear();
-    if (R.d_part) hipFree(R.d_part);
-    hipFree(R.d_scal);
-    hipFree(R.d_iscal);
+    hipHostFree(R.h_red);
     hipHostFree(R.h_pin);
     hipHostFree(R.h_pini);
     hipStreamDestroy(R.lib_stream);
@@ -2465,13 +2457,13 @@ int op_par_loop_get_min_dt_kernel(const char* name, op_set set, op_arg a0, op_ar
     double init;
     std::memcpy(&init, a1.data, sizeof(double));
     if (n == 0) return 0;
-    const int nb = (int)nblk(n);
-    TRY(ensure_part(nb));
-    k_min_part<<<nb, kBlock, 0, cur_stream()>>>(n, dptr(a0.dat), R.d_part);
-    k_min_final<<<1, kBlock, 0, cur_stream()>>>(nb, R.d_part, init, R.d_scal, nullptr);
+    const int nb = red_blocks(n);
+    k_min_part<<<nb, kBlock, 0, cur_stream()>>>(n, dptr(a0.dat), R.h_red);
     TRY(check_launch());
-    double m;
-    TRY(read_scalar(R.d_scal, &m));
+    HIPCHK(hipStreamSynchronize(cur_stream()));
+    double m = DBL_MAX;
+    for (int i = 0; i < nb; i++) m = (R.h_red[i] < m) ? R.h_red[i] : m;
+    m = (m < init) ? m : init;
     std::memcpy(a1.data, &m, sizeof(double));
     return 0;
 }
@@ -2497,7 +2489,7 @@ int mgcfd_get_min_dt_noalloc(const char* name, op_set set, op_arg a0, op_arg a1)
     double* ptr = scratch_dev[R.device];
     if (!ptr) return fail("%s: no scratch address for device %d", L, R.device);
     k_min_part<<<(unsigned)nb, kBlock, 0, cur_stream()>>>(n, dptr(a0.dat), ptr);
-    k_min_final<<<1, kBlock, 0, cur_stream()>>>((int)nb, ptr, init, ptr + kNoAllocBlocks, nullptr);
+    k_min_final<<<1, kBlock, 0, cur_stream()>>>((int)nb, ptr, init, ptr + kNoAllocBlocks);
     TRY(check_launch());
     double m;
     TRY(read_scalar(ptr + kNoAllocBlocks, &m));
@@ -2571,8 +2563,8 @@ int op_par_loop_time_step_kernel(const char* name, op_set set, op_arg a0, op_arg
     int rk;
     std::memcpy(&rk, a0.data, sizeof(int));
     if (set->size)
-        k_time_step<<<nblk(set->size), kBlock, 0, cur_stream()>>>(set->size, rk, dptr(a1.dat), dptr(a2.dat), dptr(a3.dat),
-                                                              dptr(a4.dat), nullptr);
+        k_time_step<<<nblk(5 * (size_t)set->size), kBlock, 0, cur_stream()>>>(5LL * set->size, rk, dptr(a1.dat),
+                                                                          dptr(a2.dat), dptr(a3.dat), dptr(a4.dat));
     touch(a2.dat);
     touch(a4.dat);
     return check_launch();
@@ -2611,7 +2603,8 @@ int op_par_loop_residual_kernel(const char* name, op_set set, op_arg a0, op_arg 
     TRY(direct(a1, set, 5, false, L, "arg1 variables[5] OP_READ"));
     TRY(direct(a2, set, 5, false, L, "arg2 residuals[5] OP_WRITE"));
     if (set->size)
-        k_residual<<<nblk(set->size), kBlock, 0, cur_stream()>>>(set->size, dptr(a0.dat), dptr(a1.dat), dptr(a2.dat), nullptr, nullptr, nullptr);
+        k_residual<<<nblk(5 * (size_t)set->size), kBlock, 0, cur_stream()>>>(5LL * set->size, dptr(a0.dat), dptr(a1.dat),
+                                                                         dptr(a2.dat));
     touch(a2.dat);
     return check_launch();
 }
@@ -2627,26 +2620,30 @@ int op_par_loop_calc_rms_kernel(const char* name, op_set set, op_arg a0, op_arg 
     std::memcpy(&init, a1.data, sizeof(double));
     const int n = set->size;
     if (n == 0) return 0;
-    const int nb = (int)nblk(n);
-    TRY(ensure_part(nb));
-    k_sumsq_part<<<nb, kBlock, 0, cur_stream()>>>(n, dptr(a0.dat), R.d_part);
-    k_sum_final<<<1, kSumBlock, 0, cur_stream()>>>(nb, R.d_part, init, R.d_scal + 1);
+    const int nb = red_blocks(5LL * n);
+    k_sumsq_part<<<nb, kBlock, 0, cur_stream()>>>(5LL * n, dptr(a0.dat), R.h_red);
     TRY(check_launch());
-    double s;
-    TRY(read_scalar(R.d_scal + 1, &s));
+    HIPCHK(hipStreamSynchronize(cur_stream()));
+    double p[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int i = 0; i < nb; i++) p[i & 3] += R.h_red[i];
+    const double s = init + ((p[0] + p[1]) + (p[2] + p[3]));
     std::memcpy(a1.data, &s, sizeof(double));
     return 0;
 }
 
 static int count_loop(int n, op_dat d, int* out, int which)
 {
-    k_fill_i<<<1, kBlock, 0, cur_stream()>>>(1, R.d_iscal, 0);
-    if (n) {
-        if (which == 0) k_count_bad<<<nblk(n), kBlock, 0, cur_stream()>>>(n, dptr(d), R.d_iscal);
-        else k_count_pos<<<nblk(n), kBlock, 0, cur_stream()>>>(n, dptr(d), R.d_iscal);
-        TRY(check_launch());
-    }
-    return read_iscalar(R.d_iscal, out);
+    *out = 0;
+    if (n == 0) return 0;
+    const long long n5 = 5LL * n;
+    const int nb = red_blocks(n5);
+    int* part = reinterpret_cast<int*>(R.h_red);
+    if (which == 0) k_count<true><<<nb, kBlock, 0, cur_stream()>>>(n5, dptr(d), part);
+    else k_count<false><<<nb, kBlock, 0, cur_stream()>>>(n5, dptr(d), part);
+    TRY(check_launch());
+    HIPCHK(hipStreamSynchronize(cur_stream()));
+    for (int i = 0; i < nb; i++) *out += part[i];
+    return 0;
 }
 
 int op_par_loop_count_bad_vals(const char* name, op_set set, op_arg a0, op_arg a1)
@@ -2710,7 +2707,7 @@ int op_par_loop_up_post_kernel(const char* name, op_set set, op_arg a0, op_arg a
     TRY(direct(a0, set, 5, false, L, "arg0 variables[5] OP_RW"));
     TRY(direct(a1, set, 1, true, L, "arg1 up_scratch int OP_READ"));
     if (set->size)
-        k_up_post<<<nblk(set->size), kBlock, 0, cur_stream()>>>(set->size, dptr(a0.dat), iptr(a1.dat), nullptr);
+        k_up_post<<<nblk(5 * (size_t)set->size), kBlock, 0, cur_stream()>>>(5LL * set->size, dptr(a0.dat), iptr(a1.dat));
     touch(a0.dat);
     return check_launch();
 }
@@ -2727,8 +2724,9 @@ int op_par_loop_down_kernel(const char* name, op_set set, op_arg a0, op_arg a1, 
     TRY(indirect(a4, set, 0, 1, 3, L, "arg4 coarse coords via mg map"));
     TRY(need(a3.map == a4.map, L, "same mg map"));
     if (set->size)
-        k_down<<<nblk(set->size), kBlock, 0, cur_stream()>>>(set->size, M(a3.map)->d_map, dptr(a0.dat), dptr(a1.dat),
-                                                         dptr(a2.dat), dptr(a3.dat), dptr(a4.dat), nullptr);
+        k_down_mg<false, false><<<nblk(set->size), kBlock, 0, cur_stream()>>>(
+            set->size, M(a3.map)->d_map, dptr(a0.dat), dptr(a0.dat), dptr(a1.dat), dptr(a2.dat), dptr(a3.dat),
+            dptr(a4.dat), nullptr, nullptr, DtArgs{});
     touch(a0.dat);
     return check_launch();
 }
