@@ -458,24 +458,26 @@ static int build_map_device(op_map m)
     return 0;
 }
 
-// f(0) .. f(n - 1) on up to 16 host threads, in chunks of 8 (serially below
-// 64 items).
+// f(0) .. f(n - 1) on up to 16 host threads of at least four items each, in
+// chunks of up to 8 (the plan builders' patches, 25 to 110 us an item: a 10K
+// node level's 40 patches on one thread took longer than a 300K level's 1172).
 template <typename F>
 static void parallel_for(int n, F&& f)
 {
-    const int nth = std::min(16, (int)std::max(1u, std::thread::hardware_concurrency()));
-    if (n < 64 || nth <= 1) {
+    const int nth = std::min({16, (int)std::max(1u, std::thread::hardware_concurrency()), n / 4});
+    if (nth <= 1) {
         for (int i = 0; i < n; i++) f(i);
         return;
     }
+    const int chunk = std::clamp(n / (4 * nth), 1, 8);
     std::atomic<int> next{0};
     std::vector<std::thread> pool;
     for (int t = 0; t < nth; t++)
         pool.emplace_back([&] {
             for (;;) {
-                const int i0 = next.fetch_add(8);
+                const int i0 = next.fetch_add(chunk);
                 if (i0 >= n) break;
-                for (int i = i0; i < std::min(n, i0 + 8); i++) f(i);
+                for (int i = i0; i < std::min(n, i0 + chunk); i++) f(i);
             }
         });
     for (auto& th : pool) th.join();
@@ -831,9 +833,6 @@ static int part_cut(int lo, int hi)
 // thread a 165K-node level's 645 parts became 3245 blocks.
 constexpr int kHaloCap = 448;
 
-// Runs f(i) for i in [0, n) on up to 16 host threads (the plan builders'
-// per-part work is independent); f must be thread-safe.
-
 // Blocked-gather plan of one initial part (split while its halo exceeds
 // kHaloCap); offsets are local to the part and fixed up on concatenation.
 struct BlkOut {
@@ -846,22 +845,67 @@ struct BlkOut {
     std::string err;
 };
 
+// Sorts keys by their upper 32 bits, stably: counting passes over the bytes in
+// which they differ (std::sort took half of a part's planning time).
+static void sort_upper(std::vector<uint64_t>& key, std::vector<uint64_t>& tmp)
+{
+    uint64_t all = ~0ull, any = 0;
+    for (uint64_t k : key) {
+        all &= k;
+        any |= k;
+    }
+    tmp.resize(key.size());
+    for (int sh = 32; sh < 64; sh += 8) {
+        if ((((all ^ any) >> sh) & 255) == 0 || key.empty()) continue;
+        unsigned at[257] = {};
+        for (uint64_t k : key) at[((k >> sh) & 255) + 1]++;
+        for (int d = 0; d < 255; d++) at[d + 1] += at[d];
+        for (uint64_t k : key) tmp[at[(k >> sh) & 255]++] = k;
+        key.swap(tmp);
+    }
+}
+
+// The halo of the nodes [lo, hi): its nodes, sorted, and for every incidence
+// of theirs the LDS slot of the node at its other end (owned nodes take the
+// slots [0, hi - lo), the halo follows), indexed by q - ptr[lo].
+struct HaloSlots {
+    std::vector<int> nodes, slot;
+    std::vector<uint64_t> key, tmp;
+
+    void find(int lo, int hi, const std::vector<int>& ptr, const std::vector<int2>& inc2)
+    {
+        const int q0 = ptr[lo];
+        slot.resize(ptr[hi] - q0);
+        key.clear();
+        for (int q = q0; q < ptr[hi]; q++) {
+            const int o = inc2[q].x;
+            if (o >= lo && o < hi) slot[q - q0] = o - lo;
+            else key.push_back((uint64_t)(unsigned)o << 32 | (unsigned)(q - q0));
+        }
+        sort_upper(key, tmp);
+        nodes.clear();
+        for (uint64_t k : key) {
+            const int o = (int)(k >> 32);
+            if (nodes.empty() || nodes.back() != o) nodes.push_back(o);
+            slot[(unsigned)k] = hi - lo + (int)nodes.size() - 1;
+        }
+    }
+};
+
 static void blocked_part(int lo0, int hi0, int psize, const std::vector<int>& ptr, const std::vector<int2>& inc2,
                          BlkOut& out)
 {
     std::vector<int2> work{make_int2(lo0, hi0)};
-    std::vector<int> hb;
+    HaloSlots H;
     while (!work.empty()) {             // LIFO: blocks come out in node order
         const int lo = work.back().x, hi = work.back().y;
         work.pop_back();
-        hb.clear();
-        for (int q = ptr[lo]; q < ptr[hi]; q++) {
-            const int o = inc2[q].x;
-            if (o < lo || o >= hi) hb.push_back(o);
+        bool cut = hi - lo > psize;
+        if (!cut) {
+            H.find(lo, hi, ptr, inc2);
+            cut = (int)H.nodes.size() > kHaloCap && hi - lo > 16;
         }
-        std::sort(hb.begin(), hb.end());
-        hb.erase(std::unique(hb.begin(), hb.end()), hb.end());
-        if (hi - lo > psize || ((int)hb.size() > kHaloCap && hi - lo > 16)) {
+        if (cut) {
             const int mid = part_cut(lo, hi);
             work.push_back(make_int2(mid, hi));
             work.push_back(make_int2(lo, mid));
@@ -883,21 +927,17 @@ static void blocked_part(int lo0, int hi0, int psize, const std::vector<int>& pt
             for (int t = 0; t < hi - lo; t++) {
                 const int nd = lo + t;
                 if (ptr[nd + 1] - ptr[nd] <= kd) break;
-                const int2 r = inc2[ptr[nd] + kd];
-                const int o = r.x;
-                const unsigned slot = (o >= lo && o < hi)
-                    ? (unsigned)(o - lo)
-                    : (unsigned)(hi - lo + (std::lower_bound(hb.begin(), hb.end(), o) - hb.begin()));
-                out.jslot.push_back(slot | ((unsigned)r.y & 0x80000000u));
-                out.eid.push_back(r.y & 0x7fffffff);
+                const unsigned y = (unsigned)inc2[ptr[nd] + kd].y;
+                out.jslot.push_back((unsigned)H.slot[ptr[nd] + kd - ptr[lo]] | (y & 0x80000000u));
+                out.eid.push_back((int)(y & 0x7fffffffu));
                 off++;
             }
         }
         out.jpref.push_back(off);
         out.npref.push_back(maxdeg + 1);
         out.nent.push_back((int)(out.eid.size() - e0));
-        out.nhalo.push_back((int)hb.size());
-        out.halo.insert(out.halo.end(), hb.begin(), hb.end());
+        out.nhalo.push_back((int)H.nodes.size());
+        out.halo.insert(out.halo.end(), H.nodes.begin(), H.nodes.end());
     }
 }
 
@@ -1002,126 +1042,158 @@ struct PartOut {
 // per pass for 8-byte accesses (accumulators at a 40-byte stride and
 // 40-byte records: slot modulo 16).  Each position takes, among the next
 // candidates of its colour, the edge whose endpoint slots (sa, sb) collide
-// least with those already in its 8- and 16-lane groups.  The result is
-// left in 'le'; 'out' is scratch space.
-template <typename LEv>
-static void bank_order(std::vector<LEv>& le, std::vector<LEv>& out)
-{
-    constexpr size_t kLook = 48;
-    out.clear();
-    out.reserve(le.size());
-    auto sa = [&](size_t i) { return le[i].sa; };
-    auto sb = [&](size_t i) { return le[i].sb; };
-    std::vector<size_t> rest;
-    unsigned m8a = 0, m8b = 0, m16a = 0, m16b = 0;
-    for (size_t lo = 0; lo < le.size();) {
-        size_t hi = lo;
-        while (hi < le.size() && le[hi].col == le[lo].col) hi++;
-        rest.clear();
-        for (size_t i = lo; i < hi; i++) rest.push_back(i);
-        size_t head = 0;
-        while (head < rest.size()) {
-            const size_t pos = out.size();
-            if (pos % 16 == 0) m16a = m16b = 0;
-            if (pos % 8 == 0) m8a = m8b = 0;
-            size_t best = head;
-            int bc = 1 << 30;
-            for (size_t k = head; k < rest.size() && k < head + kLook; k++) {
-                const size_t i = rest[k];
-                const int c = ((m8a >> (sa(i) & 7)) & 1) + ((m8b >> (sb(i) & 7)) & 1) +
-                              ((m16a >> (sa(i) & 15)) & 1) + ((m16b >> (sb(i) & 15)) & 1);
-                if (c < bc) {
-                    bc = c;
-                    best = k;
-                    if (c == 0) break;
-                }
-            }
-            std::swap(rest[head], rest[best]);
-            const size_t i = rest[head++];
-            m8a |= 1u << (sa(i) & 7);
-            m8b |= 1u << (sb(i) & 7);
-            m16a |= 1u << (sa(i) & 15);
-            m16b |= 1u << (sb(i) & 15);
-            out.push_back(le[i]);
-        }
-        lo = hi;
-    }
-    le.swap(out);
-}
-
-// A local edge: endpoints, their LDS slots, edge id, owner flags, colour.
-struct LocalEdge {
-    int a, b, sa, sb, e;
-    unsigned flags;
-    int col;
+// least with those already in its 8- and 16-lane groups.  'le' holds the
+// edges by colour (code: sa | sb << 10 | flags << 20 | colour << 22).
+struct PartEdge {
+    unsigned code;
+    int e;
 };
 
-// The local edges of the nodes [lo, hi): edges with an endpoint there,
-// ordered by edge id.
-static void local_edges(int lo, int hi, const std::vector<int>& ptr, const std::vector<int2>& inc2,
-                        std::vector<LocalEdge>& le)
+//
+// The next 48 candidates are bits of 64-bit words, position modulo 64: one
+// word per slot value and end, and four (8 and 16 lanes, either end) that say
+// who collides, so that a choice is a few word operations instead of a scan.
+static void bank_order(std::vector<PartEdge>& le)
 {
-    le.clear();
-    for (int nd = lo; nd < hi; nd++)
-        for (int q = ptr[nd]; q < ptr[nd + 1]; q++) {
-            const int o = inc2[q].x;
-            const bool role_b = (unsigned)inc2[q].y >> 31;
-            const bool other_owned = o >= lo && o < hi;
-            if (other_owned && role_b) continue;     // interior edge: taken from its a side
-            LocalEdge x{};
-            x.e = inc2[q].y & 0x7fffffff;
-            if (!role_b) { x.a = nd; x.b = o; x.flags = 1u | (other_owned ? 2u : 0u); }
-            else { x.a = o; x.b = nd; x.flags = 2u; }
-            le.push_back(x);
+    constexpr size_t kLook = 48;
+    struct End {
+        uint64_t with[16] = {}, c8 = 0, c16 = 0;    // candidates by slot modulo 16; those that collide
+        unsigned m8 = 0, m16 = 0;                   // slots taken by the group
+        void add(unsigned s, uint64_t bit)
+        {
+            s &= 15;
+            with[s] |= bit;
+            if ((m8 >> (s & 7)) & 1) c8 |= bit;
+            if ((m16 >> s) & 1) c16 |= bit;
         }
-    std::sort(le.begin(), le.end(), [](const LocalEdge& x, const LocalEdge& y) { return x.e < y.e; });
+        void drop(unsigned s, uint64_t bit)
+        {
+            with[s & 15] &= ~bit;
+            c8 &= ~bit;
+            c16 &= ~bit;
+        }
+        void take(unsigned s)
+        {
+            m8 |= 1u << (s & 7);
+            m16 |= 1u << (s & 15);
+            c8 |= with[s & 7] | with[(s & 7) + 8];
+            c16 |= with[s & 15];
+        }
+    } A, B;
+    uint64_t live = 0;
+    size_t hi = 0, tail = 0;
+    auto bit_of = [](size_t k) { return 1ull << (k & 63); };
+    for (size_t pos = 0; pos < le.size(); pos++) {
+        if (pos % 8 == 0) A.m8 = B.m8 = 0, A.c8 = B.c8 = 0;
+        if (pos % 16 == 0) A.m16 = B.m16 = 0, A.c16 = B.c16 = 0;
+        if (pos == hi)
+            while (hi < le.size() && le[hi].code >> 22 == le[pos].code >> 22) hi++;
+        for (; tail < std::min(hi, pos + kLook); tail++) {
+            live |= bit_of(tail);
+            A.add(le[tail].code, bit_of(tail));
+            B.add(le[tail].code >> 10, bit_of(tail));
+        }
+        // the first candidate of the fewest collisions: 0, 1, 2, 3 or 4
+        const uint64_t oa = A.c8 ^ A.c16, ob = B.c8 ^ B.c16, ta = A.c8 & A.c16, tb = B.c8 & B.c16;
+        const uint64_t odd = oa ^ ob, four = ta & tb;
+        uint64_t z = live & ~(A.c8 | A.c16 | B.c8 | B.c16);
+        if (!z) z = live & odd & ~(ta | tb);
+        if (!z) z = live & ~odd & ~four;
+        if (!z) z = live & odd;
+        if (!z) z = live;
+        const unsigned turn = pos & 63;
+        const size_t best = pos + __builtin_ctzll(z >> turn | (turn ? z << (64 - turn) : 0));
+        const PartEdge x = le[best], first = le[pos];
+        A.drop(x.code, bit_of(best));
+        B.drop(x.code >> 10, bit_of(best));
+        if (best != pos) {
+            A.drop(first.code, bit_of(pos));
+            B.drop(first.code >> 10, bit_of(pos));
+            A.add(first.code, bit_of(best));
+            B.add(first.code >> 10, bit_of(best));
+        }
+        live &= ~bit_of(pos);
+        le[best] = first;
+        le[pos] = x;
+        A.take(x.code);
+        B.take(x.code >> 10);
+    }
 }
 
-// Greedy colouring in edge order: no two edges of a colour share an owned
-// node.  Returns the number of colours, or -1 if 64 do not suffice.
-static int colour_edges(int lo, int hi, std::vector<LocalEdge>& le, std::vector<unsigned long long>& used)
+// An edge of a patch: its ends, their incidences (-1 where the end is outside
+// the patch) and its colour.
+struct PatchEdge {
+    int e, a, b, qa, qb, col;
+};
+
+// The edges with an end in [lo, hi), ordered by edge id: the incidences of
+// the patch's nodes sorted by edge, the two of an inner edge side by side.
+static void patch_edges(int lo, int hi, const std::vector<int>& ptr, const std::vector<int2>& inc2,
+                        std::vector<PatchEdge>& out)
 {
-    std::fill(used.begin(), used.begin() + (hi - lo), 0ull);
-    int ncol = 0;
-    for (auto& x : le) {
-        unsigned long long u = 0;
-        if (x.flags & 1u) u |= used[x.a - lo];
-        if (x.flags & 2u) u |= used[x.b - lo];
-        if (~u == 0ull) return -1;
-        const int c = __builtin_ctzll(~u);
-        x.col = c;
-        if (x.flags & 1u) used[x.a - lo] |= 1ull << c;
-        if (x.flags & 2u) used[x.b - lo] |= 1ull << c;
-        ncol = std::max(ncol, c + 1);
+    std::vector<uint64_t> key, tmp;
+    std::vector<int> owner;
+    const int q0 = ptr[lo];
+    key.reserve(ptr[hi] - q0);
+    owner.reserve(ptr[hi] - q0);
+    for (int nd = lo; nd < hi; nd++)
+        for (int q = ptr[nd]; q < ptr[nd + 1]; q++) {
+            key.push_back((uint64_t)((unsigned)inc2[q].y & 0x7fffffffu) << 32 | (unsigned)(q - q0));
+            owner.push_back(nd);
+        }
+    sort_upper(key, tmp);
+    out.clear();
+    for (uint64_t k : key) {
+        const int e = (int)(k >> 32), q = q0 + (int)(unsigned)k;
+        const bool role_b = (unsigned)inc2[q].y >> 31;
+        if (out.empty() || out.back().e != e)
+            out.push_back(role_b ? PatchEdge{e, inc2[q].x, owner[q - q0], -1, q, 0}
+                                 : PatchEdge{e, owner[q - q0], inc2[q].x, q, -1, 0});
+        else
+            (role_b ? out.back().qb : out.back().qa) = q;
     }
-    return ncol;
+}
+
+// Greedy colouring in edge order: no two edges of a colour share a node of
+// [lo, hi); edges without an end there are passed over.  Returns false if 64
+// colours do not suffice.
+static bool colour_edges(int lo, int hi, std::vector<PatchEdge>& le)
+{
+    unsigned long long used[kPart] = {};
+    for (auto& x : le) {
+        const bool ina = x.a >= lo && x.a < hi, inb = x.b >= lo && x.b < hi;
+        if (!ina && !inb) continue;
+        const unsigned long long u = (ina ? used[x.a - lo] : 0) | (inb ? used[x.b - lo] : 0);
+        if (~u == 0ull) return false;
+        x.col = __builtin_ctzll(~u);
+        if (ina) used[x.a - lo] |= 1ull << x.col;
+        if (inb) used[x.b - lo] |= 1ull << x.col;
+    }
+    return true;
 }
 
 static void part_part(int lo0, int hi0, int psize, const std::vector<int>& ptr, const std::vector<int2>& inc2,
                       PartOut& out)
 {
     std::vector<int2> work{make_int2(lo0, hi0)};
-    std::vector<int> hb;
-    std::vector<unsigned long long> used(kPart);   // per owned node: colours taken
-    std::vector<LocalEdge> le, tmp, whole;
-    std::vector<int> ccount;
+    HaloSlots H;
+    std::vector<PatchEdge> edges;
+    std::vector<PartEdge> le, tmp;
     // The patch's edges are coloured as a whole, and every part cut from it
     // keeps their colours, so that a node adds its edges in one order however
     // its patch is cut.  (More than 64 colours: each part colours its own.
     // A patch whose nodes have at most 32 edges never needs them.)
-    local_edges(lo0, hi0, ptr, inc2, whole);
-    const bool keep = colour_edges(lo0, hi0, whole, used) >= 0;
+    patch_edges(lo0, hi0, ptr, inc2, edges);
+    const bool keep = colour_edges(lo0, hi0, edges);
     while (!work.empty()) {
         const int lo = work.back().x, hi = work.back().y;
         work.pop_back();
-        hb.clear();
-        for (int q = ptr[lo]; q < ptr[hi]; q++) {
-            const int o = inc2[q].x;
-            if (o < lo || o >= hi) hb.push_back(o);
+        bool cut = hi - lo > psize;
+        if (!cut) {
+            H.find(lo, hi, ptr, inc2);
+            cut = (hi - lo) + (int)H.nodes.size() > kPartSlots;
         }
-        std::sort(hb.begin(), hb.end());
-        hb.erase(std::unique(hb.begin(), hb.end()), hb.end());
-        if ((hi - lo) + (int)hb.size() > kPartSlots || (hi - lo) > psize) {
+        if (cut) {
             if (hi - lo <= 8) {
                 out.err = "edge-flux part plan: node " + std::to_string(lo) + " has more than " +
                           std::to_string(kPartSlots) + " neighbours";
@@ -1132,55 +1204,43 @@ static void part_part(int lo0, int hi0, int psize, const std::vector<int>& ptr, 
             work.push_back(make_int2(lo, mid));
             continue;
         }
-        // owned nodes take slots [0, hi - lo), the sorted halo the rest
-        auto slot = [&](int nd) -> int {
-            if (nd >= lo && nd < hi) return nd - lo;
-            return (hi - lo) + (int)(std::lower_bound(hb.begin(), hb.end(), nd) - hb.begin());
-        };
-        int ncol = 0;
-        if (lo == lo0 && hi == hi0) {
-            le.swap(whole);
-        } else {
-            local_edges(lo, hi, ptr, inc2, le);
-            if (keep) {          // both lists are in edge order
-                size_t w = 0;
-                for (auto& x : le) {
-                    while (whole[w].e != x.e) w++;
-                    x.col = whole[w].col;
-                }
-            }
-        }
-        if (!keep && colour_edges(lo, hi, le, used) < 0) {
+        if (!keep && !colour_edges(lo, hi, edges)) {
             out.err = "edge-flux part plan: more than 64 edge colours in a part";
             return;
         }
-        for (auto& x : le) {
-            x.sa = slot(x.a);
-            x.sb = slot(x.b);
+        // the part's edges, then a stable counting sort by colour (edge order
+        // kept within a colour)
+        int count[65] = {}, ncol = 0;
+        tmp.clear();
+        for (const auto& x : edges) {
+            const bool ina = x.a >= lo && x.a < hi, inb = x.b >= lo && x.b < hi;
+            if (!ina && !inb) continue;
+            // the slot of an end outside the part is found at the other end
+            const unsigned sa = ina ? x.a - lo : H.slot[x.qb - ptr[lo]];
+            const unsigned sb = inb ? x.b - lo : H.slot[x.qa - ptr[lo]];
+            const unsigned flags = (ina ? 1u : 0u) | (inb ? 2u : 0u);
+            tmp.push_back(PartEdge{sa | sb << 10 | flags << 20 | (unsigned)x.col << 22, x.e});
+            count[x.col + 1]++;
             ncol = std::max(ncol, x.col + 1);
         }
-        // stable counting sort by colour (edge order kept within a colour)
-        ccount.assign(ncol + 1, 0);
-        for (const auto& x : le) ccount[x.col + 1]++;
-        for (int c = 0; c < ncol; c++) ccount[c + 1] += ccount[c];
-        tmp.resize(le.size());
-        for (const auto& x : le) tmp[ccount[x.col]++] = x;
-        le.swap(tmp);
-        bank_order(le, tmp);
+        for (int c = 0; c < ncol; c++) count[c + 1] += count[c];
+        le.resize(tmp.size());
+        for (const auto& x : tmp) le[count[x.code >> 22]++] = x;
+        bank_order(le);
         PartInfo pi;
         pi.n0 = lo;
         pi.cnt = hi - lo;
         pi.h0 = (int)out.halo.size();
-        pi.nh = (int)hb.size();
+        pi.nh = (int)H.nodes.size();
         pi.e0 = (int)out.code.size();
         pi.ne = (int)le.size();
         pi.ncol = ncol;
         pi.g0 = 0;       // set when the parts are put together
         for (const auto& x : le) {
-            out.code.push_back((unsigned)x.sa | ((unsigned)x.sb << 10) | (x.flags << 20) | ((unsigned)x.col << 22));
+            out.code.push_back(x.code);
             out.eid.push_back(x.e);
         }
-        out.halo.insert(out.halo.end(), hb.begin(), hb.end());
+        out.halo.insert(out.halo.end(), H.nodes.begin(), H.nodes.end());
         out.parts.push_back(pi);
     }
 }
