@@ -102,6 +102,7 @@ struct InvPlan {
     int bk_groups = 0;                     // partial sums over all blocks (one per 64 owned nodes)
     // part plan (edge-parallel flux over mesh parts, k_flux_part)
     int pt_parts = 0;            // 0 = not available
+    int pt_load = 0;             // parts, a patch of the last round's cut into several as one
     long long pt_nloc = 0;       // local edges over all parts
     int pt_rec_cap = 0;          // max staged nodes (owned + halo) of one part
     int pt_halo_cap = 0;         // max halo nodes of one part
@@ -814,6 +815,30 @@ static int small_part_nodes(int np)
     return 4LL * np <= R.n_cu ? kPart / 4 : 2LL * np <= R.n_cu ? kPart / 2 : kPart;
 }
 
+// Nodes per part or block of patch k of np.  A level of more patches than CUs
+// fills them in rounds, and lasts as long as a CU that got one patch more than
+// the others.  So, in each XCD's slice of the launch (patches in node order,
+// an eighth of them), the patches beyond the last full round are cut into
+// quarters if those need at most one per CU, or halves if those do: they come
+// last, and a CU takes one at most.  (One stage, part kernels: 317 patches
+// 13.0 -> 11.1 us, 352 11.5 -> 10.2, 602 17.2 -> 16.3, 1094 22.1 -> 21.1,
+// 2149 38.1 -> 37.3; mixed 317 11.5 -> 10.1; exact gather 18.6 -> 17.7 and
+// 35.3 -> 34.7.  With one piece too many per XCD the gain is lost, cycles of
+// 300K nodes with 645 patches in halves 427 -> 439 us; quarters that take
+// three per CU were slower, 434 patches 13.2 -> 16.6; from 9 rounds on there is nothing to gain, 2344 patches 35.6
+// -> 35.9.)
+constexpr int kXcds = 8;
+static int patch_part_nodes(int k, int np)
+{
+    const int cu = R.n_cu / kXcds, most = (np + kXcds - 1) / kXcds;    // CUs, patches of a slice
+    if (np <= R.n_cu || cu < 1) return small_part_nodes(np);
+    const int per = np / kXcds, lead = np % kXcds * (per + 1);          // the first slices hold one more
+    const int i = k < lead ? k % (per + 1) : (k - lead) % per;
+    const int r = most % cu;
+    if (most >= 9 * cu || i < most - r) return kPart;
+    return 4 * r <= cu ? kPart / 4 : 2 * r <= cu ? kPart / 2 : kPart;
+}
+
 // Where a part of more than 64 nodes is cut: near the middle, at a multiple
 // of 64 nodes (the kernels' partial sums run over 64-node groups).
 static int part_cut(int lo, int hi)
@@ -950,8 +975,7 @@ static int build_blocked(InvPlan& P, op_map m, const std::vector<int>& ptr, cons
     const std::vector<int> pb = set_parts(m->to);
     const int np = (int)pb.size() - 1;
     std::vector<BlkOut> outs(std::max(np, 0));
-    const int psize = small_part_nodes(np);
-    parallel_for(np, [&](int k) { blocked_part(pb[k], pb[k + 1], psize, ptr, inc2, outs[k]); });
+    parallel_for(np, [&](int k) { blocked_part(pb[k], pb[k + 1], patch_part_nodes(k, np), ptr, inc2, outs[k]); });
     std::vector<BlkInfo> blocks;
     std::vector<int> halo, jpref, eid;
     std::vector<unsigned> jslot;
@@ -1255,14 +1279,17 @@ static int build_partplan(InvPlan& P, op_map m, const std::vector<int>& ptr, con
     const int np = (int)pb.size() - 1;
     std::vector<PartOut> outs(std::max(np, 0));
     // parts smaller than a patch only where their colours are the patch's
-    const int psize = P.pt_psize ? P.pt_psize : P.max_deg <= 32 ? small_part_nodes(np) : kPart;
-    parallel_for(np, [&](int k) { part_part(pb[k], pb[k + 1], psize, ptr, inc2, outs[k]); });
+    auto psize = [&](int k) { return P.pt_psize ? P.pt_psize : P.max_deg <= 32 ? patch_part_nodes(k, np) : kPart; };
+    parallel_for(np, [&](int k) { part_part(pb[k], pb[k + 1], psize(k), ptr, inc2, outs[k]); });
     std::vector<PartInfo> parts;
     std::vector<int> halo, eid;
     std::vector<unsigned> code;
     int rec_cap = 0, halo_cap = 0, max_cnt = 0, groups = 0, max_ne = 0, max_col = 0;
-    for (auto& o : outs) {
+    P.pt_load = 0;
+    for (int k = 0; k < np; k++) {
+        PartOut& o = outs[k];
         if (!o.err.empty()) return fail("%s", o.err.c_str());
+        P.pt_load += np > R.n_cu && !P.pt_psize && psize(k) < kPart ? 1 : (int)o.parts.size();
         for (PartInfo pi : o.parts) {
             pi.h0 += (int)halo.size();
             pi.e0 += (int)code.size();
@@ -1816,12 +1843,12 @@ static int launch_part(bool coloured, const InvPlan& P, const Real* w, size_t ld
         // 9.4-9.8 us with 256 threads, 8.5-8.8 with 1024; 317 and 434 parts
         // 13.9 -> 12.9 with 512.  Beyond two parts per CU 256 threads are as
         // fast (645 parts) or faster (1172 parts and up).
-        if (!P.pt_threads && P.pt_parts <= R.n_cu) {
+        if (!P.pt_threads && P.pt_load <= R.n_cu) {
             if (P.pt_max_cnt <= kPart / 4) return launch_part_n<Real, 256, kPart / 4>(coloured, P, w, lds, var, flux, status, fresh, st);
             if (P.pt_max_cnt <= kPart / 2) return launch_part_n<Real, 512, kPart / 2>(coloured, P, w, lds, var, flux, status, fresh, st);
             return launch_part_n<Real, 1024>(coloured, P, w, lds, var, flux, status, fresh, st);
         }
-        const int threads = P.pt_threads ? P.pt_threads : P.pt_parts <= 2 * R.n_cu ? 512 : 256;
+        const int threads = P.pt_threads ? P.pt_threads : P.pt_load <= 2 * R.n_cu ? 512 : 256;
         if (threads == 512) return launch_part_n<Real, 512>(coloured, P, w, lds, var, flux, status, fresh, st);
         return launch_part_n<Real, 256>(coloured, P, w, lds, var, flux, status, fresh, st);
     }
@@ -1829,7 +1856,7 @@ static int launch_part(bool coloured, const InvPlan& P, const Real* w, size_t ld
     // threads per CU on any level, FP64 ones are faster so on levels of few
     // parts (256 -> 512 threads: 10K nodes 3.8 -> 3.5 us, 60K 6.1 -> 5.4,
     // 125K 8.9 -> 8.0; coloured 5.3 -> 4.6, 8.0 -> 7.2, 10.8 -> 9.8)
-    if (sizeof(Real) == 4 || P.pt_parts <= 2 * R.n_cu)
+    if (sizeof(Real) == 4 || P.pt_load <= 2 * R.n_cu)
         return launch_part_n<Real, 512>(coloured, P, w, lds, var, flux, status, fresh, st);
     return launch_part_n<Real, 256>(coloured, P, w, lds, var, flux, status, fresh, st);
 }

@@ -184,3 +184,43 @@ def test_abort_keeps_the_references_state(rt, level, graph, variant):
         assert err <= STATE_TOL, f"level {l}: {err:.3e}"
         if variant != "nodal_exact":    # its flux kernel has run by the time its stage kernel aborts
             assert not s.state(l, "fluxes").any()
+
+
+@pytest.mark.parametrize("n", [65537, 80003, 97537, 131073])
+def test_patches_beyond_the_last_full_round(rt, n):
+    """Levels of more patches than CUs cut the patches beyond the last full
+    round (257, 313, 382 and 513 patches on 256 CUs: quarters, quarters,
+    halves, quarters).  Against the oracle, and the coloured variants bit for
+    bit as with whole patches."""
+    import ctypes as C
+
+    mesh = mgcfd.mesh_knn(n, int(3.1 * n), 2, seed=n)
+    o = Oracle("orc")
+    state = perturbed_state(n, o.freestream(0.5, 3.0).ff_variable[:], seed=5)
+    ref = o.solve(mesh, 2, 0.5, 3.0, after_setup=lambda lv: lv[0]["var"].__setitem__(slice(None), state))
+
+    def solve(variant, part_nodes=0):
+        s = mgcfd.Solver(rt, mesh, 0.5, 3.0)
+        s.setup()
+        rt.upload(s.lv[0].variables, state)
+        if part_nodes:
+            for l in range(2):
+                rt.map_part_config(s.lv[l].edge_to_node, part_nodes, 0)
+        rt.set_flux_variant(mgcfd.FLUX_VARIANTS[variant])
+        st, rms = s.run_device(2)
+        assert st == 0
+        stats = (C.c_int * 6)()
+        if not variant.startswith("gather"):
+            mgcfd._check(rt.L.mgcfd_part_plan_stats(s.lv[0].edge_to_node, stats), "mgcfd_part_plan_stats")
+        return s.state(0), s.state(1), rms, stats[0]
+
+    for variant in ("gather_exact", "gather_fast", "part_atomic", "part_coloured", "mixed_coloured"):
+        got = solve(variant)
+        tol = MIXED_STATE_TOL if variant.startswith("mixed") else STATE_TOL
+        for l in range(2):
+            assert rel_err(got[l], ref["levels"][l]["variables"]) <= tol, (variant, l)
+        if variant.endswith("coloured"):
+            whole = solve(variant, 256)
+            assert got[3] > whole[3] == -(-n // 256)
+            for a, b in zip(got[:3], whole):
+                assert np.array_equal(a.view(np.uint64), b.view(np.uint64)), variant
