@@ -747,10 +747,14 @@ __device__ __forceinline__ void part_edges_atomic(const R* rec, double* acc, con
 }
 
 // Accumulates the part's local edges (codes and weights in registers) into
-// the LDS accumulators; ends with a barrier.  LAZY (coloured only): form each
-// edge's increment in its colour's phase instead of all of them up front, so
-// no increments are held across the phases (fewer registers, for the kernel
-// with the fused stage).
+// the LDS accumulators; ends with a barrier.  Coloured: all increments are
+// formed first, then one short phase per colour adds them, so that the colour
+// walk is a chain of LDS additions and not of whole edge increments.  LAZY:
+// each increment is formed in its colour's phase, which holds none across the
+// phases.  (One stage with fused update, formed in the phases -> up front:
+// 30K nodes 10.0 -> 7.8 us, 645 parts 25.9 -> 20.8, 3907 parts 77.5 -> 70.6;
+// FP32 with six or more edges per thread, whose workgroups the registers
+// limit to fewer per CU, 3907 parts 60.8 -> 64.0: it alone stays LAZY.)
 template <typename R, int EPT, bool COLOURED, int RS, bool LAZY>
 __device__ __forceinline__ void part_edges(const PartInfo& P, const R* rec, double* acc, const unsigned code[EPT],
                                            const R w0[EPT], const R w1[EPT], const R w2[EPT], R sc)
@@ -1805,7 +1809,7 @@ __device__ __forceinline__ bool part_stage_one(
         __syncthreads();
     }
     // 3. edges
-    part_edges<R, EPT, COLOURED, RS, true>(P, rec, acc, code, w0, w1, w2, (R)k0.sc);
+    part_edges<R, EPT, COLOURED, RS, (sizeof(R) == 4 && EPT > 4)>(P, rec, acc, code, w0, w1, w2, (R)k0.sc);
     if (halt) return false;
     // 4. the owned nodes' boundary increments and step factors
     double mdt = 0.0;

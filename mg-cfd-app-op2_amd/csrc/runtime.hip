@@ -1848,7 +1848,14 @@ static int launch_part(bool coloured, const InvPlan& P, const Real* w, size_t ld
             if (P.pt_max_cnt <= kPart / 2) return launch_part_n<Real, 512, kPart / 2>(coloured, P, w, lds, var, flux, status, fresh, st);
             return launch_part_n<Real, 1024>(coloured, P, w, lds, var, flux, status, fresh, st);
         }
-        const int threads = P.pt_threads ? P.pt_threads : P.pt_load <= 2 * R.n_cu ? 512 : 256;
+        // Coloured parts of more edges than 256 threads hold in six registers'
+        // worth each (dense coarse levels) are faster with 512: 1147 parts 43.4
+        // -> 36.0 us, 2891 parts 90.0 -> 76.1; mixed only up to some ten per
+        // CU, 1147 parts 36.7 -> 32.4, 2294 57.0 -> 55.0, 2891 65.1 -> 66.4.
+        // The uncoloured ones are not (1446 parts 31.3 -> 33.8).
+        const bool dense = coloured && P.pt_max_ne > 6 * 256 &&
+                           (sizeof(Real) == sizeof(double) || P.pt_load <= 10 * R.n_cu);
+        const int threads = P.pt_threads ? P.pt_threads : P.pt_load <= 2 * R.n_cu || dense ? 512 : 256;
         if (threads == 512) return launch_part_n<Real, 512>(coloured, P, w, lds, var, flux, status, fresh, st);
         return launch_part_n<Real, 256>(coloured, P, w, lds, var, flux, status, fresh, st);
     }
