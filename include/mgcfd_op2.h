@@ -157,10 +157,10 @@ int op_par_loop_get_min_dt_kernel(const char* name, op_set set, op_arg a0, op_ar
  * Same arguments, checks and result as op_par_loop_get_min_dt_kernel, but
  * the per-workgroup minima live in a fixed device array of the library
  * (65536 workgroups: sets of at most 16,777,216 elements; larger sets are
- * refused with an error) instead of a buffer the library grows with
- * hipMalloc.  It allocates nothing, so it refuses to run while sets, maps
- * or dats declared since the last loop are pending (the next loop's
- * renumbering allocates).  Every call on one GPU shares that array: calls
+ * refused with an error) instead of the loop's pinned host buffer, and a
+ * second kernel combines them.  It allocates nothing, so it refuses to run
+ * while sets, maps or dats declared since the last loop are pending (the next
+ * loop's renumbering allocates).  Every call on one GPU shares that array: calls
  * that overlap on one GPU race. */
 int mgcfd_get_min_dt_noalloc(const char* name, op_set set, op_arg a0, op_arg a1);
 /* time_stepping_kernels.h:43-64, site euler3d.cpp:485-489 */
@@ -263,7 +263,7 @@ int mgcfd_set_flux_variant(int variant);
 int mgcfd_get_flux_variant(void);
 
 /* Blocked-gather plan of an edge->node map (variants GATHER_*): stats[0]
- * workgroups, [1] staged node slots per workgroup, [2] incidences (2 per
+ * workgroups, [1] largest staged nodes of a workgroup, [2] incidences (2 per
  * edge), [3] max node degree, [4] dynamic LDS bytes per workgroup. */
 int mgcfd_plan_stats(op_map map, int* stats);
 
