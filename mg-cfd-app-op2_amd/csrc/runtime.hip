@@ -1826,10 +1826,8 @@ static int launch_part_n(bool coloured, const InvPlan& P, const Real* w, size_t 
 // Real = double: the FP64 part kernel, 256 threads per part.  Real = float:
 // mixed precision, whose smaller register footprint lets 512 threads (8
 // waves) share one part in the edge-flux kernel, which shortens each
-// workgroup's edge phase; the kernel with the fused stage needs ~96 VGPRs
-// (its epilogue), which leaves 2 such workgroups per CU, so on levels that
-// fill the chip it runs 256 threads per part (5 per CU): batched solves 310 ->
-// 323 per second.
+// workgroup's edge phase; with the fused stage, uncoloured levels that fill
+// the chip run 256 threads per part (batched solves 310 -> 323 per second).
 // The autotuner may set a plan's fused-stage kernel to 256 or 512 threads per
 // part (pt_threads).
 template <typename Real>
