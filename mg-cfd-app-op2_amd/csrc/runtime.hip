@@ -29,6 +29,7 @@
 #include <vector>
 
 #include "mgcfd_op2.h"
+#include "host_rules.h"
 #include "kernels.h"
 
 namespace mgcfd {
@@ -734,10 +735,8 @@ static int upload_dat(op_dat d)
 
 // ---------------------------------------------------------------- fetch --
 
-// Pinned landing buffers of fetches: kept from the first large fetch until
-// op_exit, 16 MB in all; one fetch at a time holds them.
-constexpr int kFetchSlots = 8;
-constexpr size_t kFetchBytes = 2u << 20;
+// Pinned landing buffers of fetches: kept from the first fetch that needs them
+// until op_exit, 16 MB in all; one fetch at a time holds them.
 struct FetchPool {
     std::mutex mu;
     char* pin[kFetchSlots] = {};
@@ -756,35 +755,49 @@ static void fetch_pool_free()
     }
 }
 
+// A fetch without the landing buffers: one pageable copy, the renumbering
+// undone by the host.
+static int fetch_pageable(op_set set, const void* dev, size_t rec, int lo, int cnt, void* dest, hipStream_t stream)
+{
+    std::vector<char> aos(rec * (size_t)cnt);
+    HIPCHK(hipStreamSynchronize(stream));
+    HIPCHK(hipMemcpy(aos.data(), static_cast<const char*>(dev) + rec * (size_t)lo, aos.size(), hipMemcpyDeviceToHost));
+    const SetImpl* si = S(set);
+    for (int i = 0; i < cnt; i++)
+        std::memcpy(static_cast<char*>(dest) + rec * (size_t)(si->to_orig(lo + i) - lo), aos.data() + rec * (size_t)i,
+                    rec);
+    return 0;
+}
+
 // Elements [lo, lo + cnt) of a [set][dim] device array in the set's internal
-// order, copied to dest (host) in the caller's order once everything queued
-// on the stream has run.  The device undoes
-// the renumbering while it writes 2 MB pieces over the host link, and up to
-// eight threads copy the pieces on (a copy's first touch of fresh pages is
-// what costs).  Five doubles per element, against a pageable copy permuted on
-// one host thread: 10.6K elements 201 -> 32 us, 300K 2380 -> 369 us, 1M 17.1
-// -> 1.2 ms.
+// order (a range that the order maps to itself), copied to dest (host) in the
+// caller's order once everything queued on the stream has run.  The device
+// undoes the renumbering while it writes 2 MB pieces over the host link, and
+// up to eight threads copy the pieces on (a copy's first touch of fresh pages
+// is what costs).  Five doubles per element, against a pageable copy permuted
+// on one host thread: 10.6K elements 201 -> 32 us, 300K 2380 -> 369 us, 1M
+// 17.1 -> 1.2 ms.  Elements larger than a piece take the pageable copy.
 static int fetch_elements(op_set set, const void* dev, bool is_int, int dim, int lo, int cnt, void* dest,
                           hipStream_t stream)
 {
     if (cnt <= 0) return 0;
     SetImpl* si = S(set);
     const size_t rec = (is_int ? sizeof(int) : sizeof(double)) * dim;
+    const FetchPieces fp = fetch_pieces(rec, cnt);
+    if (fp.rows == 0) return fetch_pageable(set, dev, rec, lo, cnt, dest, stream);
     std::lock_guard<std::mutex> lk(g_fetch.mu);
     if (!si->iperm.empty() && !si->d_iperm) {
         HIPCHK(hipMalloc(&si->d_iperm, sizeof(int) * si->iperm.size()));
         HIPCHK(hipMemcpy(si->d_iperm, si->iperm.data(), sizeof(int) * si->iperm.size(), hipMemcpyHostToDevice));
     }
-    const int piece = (int)std::max<size_t>(1, kFetchBytes / rec);
-    const int np = (cnt + piece - 1) / piece, nw = std::min(np, kFetchSlots);
-    for (int k = 0; k < nw; k++) {
-        if (!g_fetch.pin[k]) HIPCHK(hipHostMalloc(&g_fetch.pin[k], std::max(kFetchBytes, rec), hipHostMallocDefault));
+    for (int k = 0; k < fp.slots; k++) {
+        if (!g_fetch.pin[k]) HIPCHK(hipHostMalloc(&g_fetch.pin[k], kFetchBytes, hipHostMallocDefault));
         if (!g_fetch.ev[k]) HIPCHK(hipEventCreateWithFlags(&g_fetch.ev[k], hipEventDisableTiming));
     }
-    // worker w takes pieces w, w + nw, ...: its buffer is free once copied on
-    return run_tasks(nw, [&](int w) -> int {
-        for (int p = w; p < np; p += nw) {
-            const int r0 = p * piece, rows = std::min(piece, cnt - r0);
+    // worker w takes pieces w, w + slots, ...: its buffer is free once copied on
+    return run_tasks(fp.slots, [&](int w) -> int {
+        for (int p = w; p < fp.pieces; p += fp.slots) {
+            const int r0 = p * fp.rows, rows = std::min(fp.rows, cnt - r0);
             const unsigned grid = std::min(512u, nblk((size_t)rows * dim));
             if (is_int)
                 k_fetch_rows<int><<<grid, kBlock, 0, stream>>>(lo + r0, rows, dim, si->d_iperm, (const int*)dev,

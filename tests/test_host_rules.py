@@ -1,0 +1,50 @@
+"""Sizes that the library's host code derives for copies and launches
+(csrc/host_rules.h), compiled and checked without a GPU."""
+import ctypes as C
+import os
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "mg-cfd-app-op2_amd", "csrc")
+
+SOURCE = r"""
+#include "host_rules.h"
+extern "C" long long slot_bytes() { return (long long)mgcfd::kFetchBytes; }
+extern "C" int slot_count() { return mgcfd::kFetchSlots; }
+extern "C" void pieces(long long rec, int cnt, int* out)
+{
+    const mgcfd::FetchPieces p = mgcfd::fetch_pieces((std::size_t)rec, cnt);
+    out[0] = p.rows; out[1] = p.pieces; out[2] = p.slots;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    d = tmp_path_factory.mktemp("rules")
+    (d / "rules.cpp").write_text(SOURCE)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-shared", "-fPIC", "-I", CSRC, "-o",
+                    str(d / "rules.so"), str(d / "rules.cpp")], check=True)
+    L = C.CDLL(str(d / "rules.so"))
+    L.slot_bytes.restype = C.c_longlong
+    L.pieces.argtypes = [C.c_longlong, C.c_int, C.c_void_p]
+    return L
+
+
+# bytes of an element: an int, five doubles, up to, at and beyond a buffer
+RECS = [4, 8, 12, 40, 2**20, 2**21 - 8, 2**21, 2**21 + 4, 2**21 + 8, 2**33]
+
+
+@pytest.mark.parametrize("rec", RECS)
+@pytest.mark.parametrize("cnt", [1, 2, 7, 8, 9, 52428, 52429, 524289, 2**31 - 1])
+def test_fetch_pieces_fit_their_buffers(rules, rec, cnt):
+    out = (C.c_int * 3)()
+    rules.pieces(rec, cnt, out)
+    rows, pieces, slots = out
+    if rec > rules.slot_bytes():
+        assert rows == 0                       # not through the buffers
+        return
+    assert 1 <= rows and rows * rec <= rules.slot_bytes()
+    assert (pieces - 1) * rows < cnt <= pieces * rows
+    assert slots == min(pieces, rules.slot_count())
