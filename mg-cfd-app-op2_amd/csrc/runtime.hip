@@ -785,6 +785,9 @@ static int fetch_elements(op_set set, const void* dev, bool is_int, int dim, int
     const size_t rec = (is_int ? sizeof(int) : sizeof(double)) * dim;
     const FetchPieces fp = fetch_pieces(rec, cnt);
     if (fp.rows == 0) return fetch_pageable(set, dev, rec, lo, cnt, dest, stream);
+    // what the stream holds is waited for before the buffers are taken, so that
+    // other threads' fetches wait for this one's copy only
+    HIPCHK(hipStreamSynchronize(stream));
     std::lock_guard<std::mutex> lk(g_fetch.mu);
     if (!si->iperm.empty() && !si->d_iperm) {
         HIPCHK(hipMalloc(&si->d_iperm, sizeof(int) * si->iperm.size()));
