@@ -769,6 +769,36 @@ static int fetch_pageable(op_set set, const void* dev, size_t rec, int lo, int c
     return 0;
 }
 
+// The device copy of a set's order and up to 'slots' buffers (g_fetch.mu held):
+// how many buffers there are, 0 when either is not to be had.
+static int fetch_scratch(SetImpl* si, int slots)
+{
+    if (!si->iperm.empty() && !si->d_iperm) {
+        const size_t bytes = sizeof(int) * si->iperm.size();
+        int* d = nullptr;
+        if (hipMalloc(&d, bytes) != hipSuccess ||
+            hipMemcpy(d, si->iperm.data(), bytes, hipMemcpyHostToDevice) != hipSuccess) {
+            if (d) hipFree(d);
+            (void)hipGetLastError();     // not the next launch's
+            return 0;
+        }
+        si->d_iperm = d;
+    }
+    for (int k = 0; k < slots; k++) {
+        char* pin = g_fetch.pin[k];
+        hipEvent_t ev = g_fetch.ev[k];
+        if ((!pin && hipHostMalloc(&pin, kFetchBytes, hipHostMallocDefault) != hipSuccess) ||
+            (!ev && hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess)) {
+            if (pin && !g_fetch.pin[k]) hipHostFree(pin);
+            (void)hipGetLastError();
+            return k;
+        }
+        g_fetch.pin[k] = pin;
+        g_fetch.ev[k] = ev;
+    }
+    return slots;
+}
+
 // Elements [lo, lo + cnt) of a [set][dim] device array in the set's internal
 // order (a range that the order maps to itself), copied to dest (host) in the
 // caller's order once everything queued on the stream has run.  The device
@@ -776,7 +806,8 @@ static int fetch_pageable(op_set set, const void* dev, size_t rec, int lo, int c
 // up to eight threads copy the pieces on (a copy's first touch of fresh pages
 // is what costs).  Five doubles per element, against a pageable copy permuted
 // on one host thread: 10.6K elements 201 -> 32 us, 300K 2380 -> 369 us, 1M
-// 17.1 -> 1.2 ms.  Elements larger than a piece take the pageable copy.
+// 17.1 -> 1.2 ms.  Elements larger than a piece take the pageable copy, and so
+// does a fetch that finds no memory for the order's device copy or a buffer.
 static int fetch_elements(op_set set, const void* dev, bool is_int, int dim, int lo, int cnt, void* dest,
                           hipStream_t stream)
 {
@@ -788,18 +819,15 @@ static int fetch_elements(op_set set, const void* dev, bool is_int, int dim, int
     // what the stream holds is waited for before the buffers are taken, so that
     // other threads' fetches wait for this one's copy only
     HIPCHK(hipStreamSynchronize(stream));
-    std::lock_guard<std::mutex> lk(g_fetch.mu);
-    if (!si->iperm.empty() && !si->d_iperm) {
-        HIPCHK(hipMalloc(&si->d_iperm, sizeof(int) * si->iperm.size()));
-        HIPCHK(hipMemcpy(si->d_iperm, si->iperm.data(), sizeof(int) * si->iperm.size(), hipMemcpyHostToDevice));
+    std::unique_lock<std::mutex> lk(g_fetch.mu);
+    const int nw = fetch_scratch(si, fp.slots);
+    if (nw == 0) {
+        lk.unlock();
+        return fetch_pageable(set, dev, rec, lo, cnt, dest, stream);
     }
-    for (int k = 0; k < fp.slots; k++) {
-        if (!g_fetch.pin[k]) HIPCHK(hipHostMalloc(&g_fetch.pin[k], kFetchBytes, hipHostMallocDefault));
-        if (!g_fetch.ev[k]) HIPCHK(hipEventCreateWithFlags(&g_fetch.ev[k], hipEventDisableTiming));
-    }
-    // worker w takes pieces w, w + slots, ...: its buffer is free once copied on
-    return run_tasks(fp.slots, [&](int w) -> int {
-        for (int p = w; p < fp.pieces; p += fp.slots) {
+    // worker w takes pieces w, w + nw, ...: its buffer is free once copied on
+    return run_tasks(nw, [&](int w) -> int {
+        for (int p = w; p < fp.pieces; p += nw) {
             const int r0 = p * fp.rows, rows = std::min(fp.rows, cnt - r0);
             const unsigned grid = std::min(512u, nblk((size_t)rows * dim));
             if (is_int)

@@ -1,8 +1,14 @@
 """Fetches beyond what the pinned landing buffers are made for."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
+import hip_shim
 import mgcfd
+from conftest import ROOT
 from test_gpu_fetch import ring
 
 pytestmark = pytest.mark.gpu
@@ -27,3 +33,63 @@ def test_elements_larger_than_a_buffer(rt, dim, typ, ordered):
     d, little = rt.decl_dat(st, dim, data, "d", typ), rt.decl_dat(st, 5, rng.normal(size=(n, 5)), "little")
     assert rt.fetch(little).shape == (n, 5)
     assert np.array_equal(rt.fetch(d), data)
+
+
+def run_script(tmp_path, body, **env):
+    """body in a process of its own, with the shim loaded as 'shim'; it has a
+    set 'st' with an order of its own, values 'data' and their dat 'd'."""
+    head = f"""
+import sys
+sys.path[:0] = {[os.path.join(ROOT, "tests"), os.path.join(ROOT, "mg-cfd-app-op2_amd")]!r}
+import numpy as np
+import hip_shim
+shim = hip_shim.load({hip_shim.build(tmp_path)!r})
+"""
+    script = tmp_path / "script.py"
+    script.write_text(head + body)
+    r = subprocess.run([sys.executable, "-u", str(script)], env=dict(os.environ, **env), capture_output=True,
+                       text=True, timeout=100)
+    assert r.returncode == 0, r.stdout + r.stderr
+    assert r.stdout.split()[-1] == "ok"
+
+
+PREPARE = """
+import mgcfd
+from test_gpu_fetch import ring
+rt = mgcfd.Runtime()
+n = 300000
+st = ring(rt, n, 3)[0]
+data = np.random.default_rng(1).normal(size=(n, 5))
+d = rt.decl_dat(st, 5, data, "d")
+mgcfd._check(rt.L.op_renumber(None), "op_renumber")
+"""
+
+
+def test_fetch_needs_no_device_memory(tmp_path):
+    """Device memory is gone when a set's first dat is fetched; a later fetch,
+    with memory again, takes the buffers; no error is left for later calls."""
+    run_script(tmp_path, PREPARE + """
+shim.shim_refuse_device(1)
+for _ in range(2):
+    assert np.array_equal(rt.fetch(d), data)
+rt.sync()
+rt.par_loop("zero_5d_array_kernel", st, rt.arg(d, -1, None, 5, acc=mgcfd.OP_WRITE))
+assert not rt.fetch(d).any()
+rt.upload(d, data)
+shim.shim_refuse_device(0)
+assert np.array_equal(rt.fetch(d), data)
+print("ok")
+""")
+
+
+@pytest.mark.parametrize("left", [0, 1, 3])
+def test_fetch_with_fewer_pinned_buffers(tmp_path, left):
+    """Six buffers' worth of pieces with none, one or three buffers to be had."""
+    run_script(tmp_path, PREPARE + f"""
+shim.shim_pinned_left({left})
+for _ in range(2):
+    assert np.array_equal(rt.fetch(d), data)
+shim.shim_pinned_left(-1)
+assert np.array_equal(rt.fetch(d), data)
+print("ok")
+""")
