@@ -26,6 +26,7 @@
 #include <mutex>
 #include <numeric>
 #include <string>
+#include <system_error>
 #include <vector>
 
 #include "mgcfd_op2.h"
@@ -825,24 +826,48 @@ static int fetch_elements(op_set set, const void* dev, bool is_int, int dim, int
         lk.unlock();
         return fetch_pageable(set, dev, rec, lo, cnt, dest, stream);
     }
-    // worker w takes pieces w, w + nw, ...: its buffer is free once copied on
-    return run_tasks(nw, [&](int w) -> int {
-        for (int p = w; p < fp.pieces; p += nw) {
-            const int r0 = p * fp.rows, rows = std::min(fp.rows, cnt - r0);
-            const unsigned grid = std::min(512u, nblk((size_t)rows * dim));
-            if (is_int)
-                k_fetch_rows<int><<<grid, kBlock, 0, stream>>>(lo + r0, rows, dim, si->d_iperm, (const int*)dev,
-                                                               (int*)g_fetch.pin[w]);
-            else
-                k_fetch_rows<double><<<grid, kBlock, 0, stream>>>(lo + r0, rows, dim, si->d_iperm,
-                                                                  (const double*)dev, (double*)g_fetch.pin[w]);
-            TRY(check_launch());
-            HIPCHK(hipEventRecord(g_fetch.ev[w], stream));
-            HIPCHK(hipEventSynchronize(g_fetch.ev[w]));
-            std::memcpy(static_cast<char*>(dest) + (size_t)r0 * rec, g_fetch.pin[w], rec * (size_t)rows);
-        }
+    // worker w takes one piece after another through its buffer; worker 0 is
+    // this thread, and copies all when no other can be started
+    std::atomic<int> next{0};
+    std::vector<int> rc(nw, 0);
+    std::vector<std::string> msg(nw);
+    auto piece = [&](int w, int p) -> int {
+        const int r0 = p * fp.rows, rows = std::min(fp.rows, cnt - r0);
+        const unsigned grid = std::min(512u, nblk((size_t)rows * dim));
+        if (is_int)
+            k_fetch_rows<int><<<grid, kBlock, 0, stream>>>(lo + r0, rows, dim, si->d_iperm, (const int*)dev,
+                                                           (int*)g_fetch.pin[w]);
+        else
+            k_fetch_rows<double><<<grid, kBlock, 0, stream>>>(lo + r0, rows, dim, si->d_iperm, (const double*)dev,
+                                                              (double*)g_fetch.pin[w]);
+        TRY(check_launch());
+        HIPCHK(hipEventRecord(g_fetch.ev[w], stream));
+        HIPCHK(hipEventSynchronize(g_fetch.ev[w]));
+        std::memcpy(static_cast<char*>(dest) + (size_t)r0 * rec, g_fetch.pin[w], rec * (size_t)rows);
         return 0;
-    });
+    };
+    auto worker = [&](int w) {
+        for (int p; !rc[w] && (p = next.fetch_add(1)) < fp.pieces;) rc[w] = piece(w, p);
+        if (rc[w]) msg[w] = g_err;
+    };
+    std::vector<std::thread> pool;
+    pool.reserve(nw);
+    try {
+        for (int w = 1; w < nw; w++)
+            pool.emplace_back([&, w] {
+                hipSetDevice(R.device);
+                worker(w);
+            });
+    } catch (const std::system_error&) {
+    }
+    worker(0);
+    for (auto& th : pool) th.join();
+    for (int w = 0; w < nw; w++)
+        if (rc[w]) {
+            g_err = msg[w];
+            return rc[w];
+        }
+    return 0;
 }
 
 // ---------------------------------------------------------------- plans --

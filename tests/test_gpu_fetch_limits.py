@@ -50,6 +50,7 @@ shim = hip_shim.load({hip_shim.build(tmp_path)!r})
     r = subprocess.run([sys.executable, "-u", str(script)], env=dict(os.environ, **env), capture_output=True,
                        text=True, timeout=100)
     assert r.returncode == 0, r.stdout + r.stderr
+    print(r.stdout)
     assert r.stdout.split()[-1] == "ok"
 
 
@@ -91,5 +92,23 @@ for _ in range(2):
     assert np.array_equal(rt.fetch(d), data)
 shim.shim_pinned_left(-1)
 assert np.array_equal(rt.fetch(d), data)
+print("ok")
+""")
+
+
+def test_fetch_without_further_threads(tmp_path):
+    """No thread can be started (a limit that holds for ordinary users): the
+    calling thread copies every piece."""
+    run_script(tmp_path, PREPARE + """
+import resource, threading
+assert np.array_equal(rt.fetch(d), data)
+resource.setrlimit(resource.RLIMIT_NPROC, (1, resource.getrlimit(resource.RLIMIT_NPROC)[1]))
+try:
+    threading.Thread(target=int).start()
+    print("threads still start")
+except RuntimeError:
+    print("no threads")
+for _ in range(2):
+    assert np.array_equal(rt.fetch(d), data)
 print("ok")
 """)
