@@ -203,6 +203,21 @@ constexpr int kMaxDevices = 64;
 static __device__ __align__(256) double scratch[kNoAllocBlocks + 1];
 static double* scratch_dev[kMaxDevices];        // device address of 'scratch' on each device (op_init)
 
+// The library's device as the calling thread's current one, for entry points
+// that allocate or launch on whichever thread calls them.
+struct DeviceScope {
+    int saved = 0;
+    bool moved = false;
+    DeviceScope()
+    {
+        moved = hipGetDevice(&saved) == hipSuccess && saved != R.device && hipSetDevice(R.device) == hipSuccess;
+    }
+    ~DeviceScope()
+    {
+        if (moved) hipSetDevice(saved);
+    }
+};
+
 static SetImpl* S(op_set s) { return static_cast<SetImpl*>(s->impl); }
 static MapImpl* M(op_map m) { return static_cast<MapImpl*>(m->impl); }
 static DatImpl* D(op_dat d) { return static_cast<DatImpl*>(d->impl); }
@@ -817,6 +832,9 @@ static int fetch_elements(op_set set, const void* dev, bool is_int, int dim, int
     const size_t rec = (is_int ? sizeof(int) : sizeof(double)) * dim;
     const FetchPieces fp = fetch_pieces(rec, cnt);
     if (fp.rows == 0) return fetch_pageable(set, dev, rec, lo, cnt, dest, stream);
+    // the order's copy and the buffers must be the library's device's, whatever
+    // device the calling thread uses (a thread starts on device 0)
+    DeviceScope device;
     // what the stream holds is waited for before the buffers are taken, so that
     // other threads' fetches wait for this one's copy only
     HIPCHK(hipStreamSynchronize(stream));

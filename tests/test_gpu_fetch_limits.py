@@ -112,3 +112,26 @@ for _ in range(2):
     assert np.array_equal(rt.fetch(d), data)
 print("ok")
 """)
+
+
+@pytest.mark.parametrize("n", [1000, 300000])
+def test_fetch_from_a_thread_on_another_device(tmp_path, n):
+    """The library on the second of two devices (one, shown as two): the first
+    fetch, made by a thread that has chosen no device, allocates and launches
+    on the library's; the thread's own choice is left alone."""
+    run_script(tmp_path, "shim.shim_devices(2)\n" + PREPARE.replace("n = 300000", f"n = {n}") + """
+import ctypes as C, threading
+got = []
+def work():
+    got.append(rt.fetch(d))
+    dev = C.c_int(-1)
+    shim.hipGetDevice(C.byref(dev))
+    got.append(dev.value)
+shim.shim_expect(1)
+t = threading.Thread(target=work)
+t.start()
+t.join()
+assert shim.shim_misplaced() == 0, shim.shim_misplaced()
+assert np.array_equal(got[0], data) and got[1] == 0
+print("ok")
+""", MGCFD_DEVICE="1")
