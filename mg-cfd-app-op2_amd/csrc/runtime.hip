@@ -421,6 +421,7 @@ static std::vector<int> partition_order(int n, const std::vector<const MapImpl*>
 }
 
 static int upload_dat(op_dat d);
+static int await_zeros(op_dat d);
 static void mg_release_all();
 static void mg_join_admissions();
 
@@ -683,12 +684,14 @@ static int freeze_objects(const std::vector<op_set>& sets, const std::vector<op_
     // maps and dats in one pool: the largest of each (a level's edge map and
     // edge weights) upload side by side
     const int nm = (int)ml.size();
-    return run_tasks(nm + (int)dl.size(), [&](int k) -> int {
+    if (int rc = run_tasks(nm + (int)dl.size(), [&](int k) -> int {
         if (k >= nm) return upload_dat(dl[k - nm]);
         if (int r = build_map_device(ml[k])) return r;
         M(ml[k])->on_device = true;
         return 0;
-    });
+    }))
+        return rc;
+    return dl.empty() ? 0 : await_zeros(dl.back());
 }
 
 // Chooses the internal order of every set declared since the last call, then
@@ -712,6 +715,16 @@ static int freeze()
     if (int rc = freeze_objects(sets, maps, dats)) return rc;
     R.frozen = true;
     R.dirty = false;
+    return 0;
+}
+
+// The zeros of new dats (upload_dat) are written on the null stream after the
+// call that asks for them has returned, and the loops' streams do not wait for
+// that stream: one readback on it, from any dat, does.
+static int await_zeros(op_dat d)
+{
+    char x;
+    HIPCHK(hipMemcpy(&x, D(d)->d, 1, hipMemcpyDeviceToHost));
     return 0;
 }
 
@@ -2299,7 +2312,7 @@ static op_dat add_dat(op_set set, int dim, const char* type, int size, const cha
     d->name = keep_name(name);
     d->impl = di;
     if (S(set)->frozen) {
-        if (upload_dat(d)) return nullptr;
+        if (upload_dat(d) || await_zeros(d)) return nullptr;
     } else {
         R.dirty = true;
     }
