@@ -26,4 +26,18 @@ inline FetchPieces fetch_pieces(std::size_t rec, int cnt)
     return {rows, pieces, std::min(pieces, kFetchSlots)};
 }
 
+// Elements per launch of a loop with a thread for each of an element's five
+// doubles: a launch takes fewer than 2^32 threads, so larger sets (from
+// 858,993,459 elements) take several launches.
+constexpr int kFlatElements = 1 << 29;
+
+// f(first element, elements) for each launch; its first non-zero result ends it.
+template <typename F>
+int flat_launches(int n, F&& f)
+{
+    for (long long at = 0; at < n; at += kFlatElements)
+        if (int rc = f((std::size_t)at, (int)std::min<long long>(kFlatElements, n - at))) return rc;
+    return 0;
+}
+
 }  // namespace mgcfd

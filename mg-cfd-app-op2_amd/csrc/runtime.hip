@@ -2618,9 +2618,13 @@ int op_par_loop_copy_double_kernel(const char* name, op_set set, op_arg a0, op_a
     TRY(chk_ready(L));
     TRY(direct(a0, set, 5, false, L, "arg0 variables[5] OP_READ"));
     TRY(direct(a1, set, 5, false, L, "arg1 old_variables[5] OP_WRITE"));
-    if (set->size) k_copy<<<nblk(5 * (size_t)set->size), kBlock, 0, cur_stream()>>>(5 * (size_t)set->size, dptr(a0.dat), dptr(a1.dat), nullptr);
+    TRY(flat_launches(set->size, [&](size_t e, int n) -> int {
+        k_copy<<<nblk(5 * (size_t)n), kBlock, 0, cur_stream()>>>(5 * (size_t)n, dptr(a0.dat) + 5 * e,
+                                                             dptr(a1.dat) + 5 * e, nullptr);
+        return check_launch();
+    }));
     touch(a1.dat);
-    return check_launch();
+    return 0;
 }
 
 int op_par_loop_calculate_dt_kernel(const char* name, op_set set, op_arg a0, op_arg a1, op_arg a2)
@@ -2754,12 +2758,14 @@ int op_par_loop_time_step_kernel(const char* name, op_set set, op_arg a0, op_arg
     TRY(direct(a4, set, 5, false, L, "arg4 variables[5] OP_WRITE"));
     int rk;
     std::memcpy(&rk, a0.data, sizeof(int));
-    if (set->size)
-        k_time_step<<<nblk(5 * (size_t)set->size), kBlock, 0, cur_stream()>>>(5LL * set->size, rk, dptr(a1.dat),
-                                                                          dptr(a2.dat), dptr(a3.dat), dptr(a4.dat));
+    TRY(flat_launches(set->size, [&](size_t e, int n) -> int {
+        k_time_step<<<nblk(5 * (size_t)n), kBlock, 0, cur_stream()>>>(
+            5LL * n, rk, dptr(a1.dat) + e, dptr(a2.dat) + 5 * e, dptr(a3.dat) + 5 * e, dptr(a4.dat) + 5 * e);
+        return check_launch();
+    }));
     touch(a2.dat);
     touch(a4.dat);
-    return check_launch();
+    return 0;
 }
 
 int op_par_loop_unstructured_stream_kernel(const char* name, op_set set, op_arg a0, op_arg a1, op_arg a2,
@@ -2794,11 +2800,13 @@ int op_par_loop_residual_kernel(const char* name, op_set set, op_arg a0, op_arg 
     TRY(direct(a0, set, 5, false, L, "arg0 old_variables[5] OP_READ"));
     TRY(direct(a1, set, 5, false, L, "arg1 variables[5] OP_READ"));
     TRY(direct(a2, set, 5, false, L, "arg2 residuals[5] OP_WRITE"));
-    if (set->size)
-        k_residual<<<nblk(5 * (size_t)set->size), kBlock, 0, cur_stream()>>>(5LL * set->size, dptr(a0.dat), dptr(a1.dat),
-                                                                         dptr(a2.dat));
+    TRY(flat_launches(set->size, [&](size_t e, int n) -> int {
+        k_residual<<<nblk(5 * (size_t)n), kBlock, 0, cur_stream()>>>(5LL * n, dptr(a0.dat) + 5 * e,
+                                                                 dptr(a1.dat) + 5 * e, dptr(a2.dat) + 5 * e);
+        return check_launch();
+    }));
     touch(a2.dat);
-    return check_launch();
+    return 0;
 }
 
 int op_par_loop_calc_rms_kernel(const char* name, op_set set, op_arg a0, op_arg a1)
@@ -2898,10 +2906,12 @@ int op_par_loop_up_post_kernel(const char* name, op_set set, op_arg a0, op_arg a
     TRY(chk_ready(L));
     TRY(direct(a0, set, 5, false, L, "arg0 variables[5] OP_RW"));
     TRY(direct(a1, set, 1, true, L, "arg1 up_scratch int OP_READ"));
-    if (set->size)
-        k_up_post<<<nblk(5 * (size_t)set->size), kBlock, 0, cur_stream()>>>(5LL * set->size, dptr(a0.dat), iptr(a1.dat));
+    TRY(flat_launches(set->size, [&](size_t e, int n) -> int {
+        k_up_post<<<nblk(5 * (size_t)n), kBlock, 0, cur_stream()>>>(5LL * n, dptr(a0.dat) + 5 * e, iptr(a1.dat) + e);
+        return check_launch();
+    }));
     touch(a0.dat);
-    return check_launch();
+    return 0;
 }
 
 int op_par_loop_down_kernel(const char* name, op_set set, op_arg a0, op_arg a1, op_arg a2, op_arg a3, op_arg a4)
@@ -2930,14 +2940,14 @@ int op_par_loop_down_v2_kernel_pre(const char* name, op_set set, op_arg a0, op_a
     TRY(chk_ready(L));
     TRY(direct(a0, set, 1, false, L, "arg0 prolonged weight sums OP_WRITE"));
     TRY(direct(a1, set, 5, false, L, "arg1 prolonged residuals[5] OP_WRITE"));
-    const size_t n = (size_t)set->size;
-    if (n) {
-        k_fill<<<nblk(n), kBlock, 0, cur_stream()>>>(n, dptr(a0.dat), 0.0);
-        k_fill<<<nblk(5 * n), kBlock, 0, cur_stream()>>>(5 * n, dptr(a1.dat), 0.0);
-    }
+    TRY(flat_launches(set->size, [&](size_t e, int n) -> int {
+        k_fill<<<nblk(n), kBlock, 0, cur_stream()>>>((size_t)n, dptr(a0.dat) + e, 0.0);
+        k_fill<<<nblk(5 * (size_t)n), kBlock, 0, cur_stream()>>>(5 * (size_t)n, dptr(a1.dat) + 5 * e, 0.0);
+        return check_launch();
+    }));
     touch(a0.dat);
     touch(a1.dat);
-    return check_launch();
+    return 0;
 }
 
 int op_par_loop_down_v2_kernel(const char* name, op_set set, op_arg a0, op_arg a1, op_arg a2, op_arg a3,

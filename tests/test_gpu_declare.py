@@ -36,3 +36,16 @@ def test_first_loop_follows_the_zeros(rt, n, late):
     for d in (dats[2], dats[0]):
         rt.par_loop("initialize_variables_kernel", st, rt.arg(d, -1, None, 5, acc=mgcfd.OP_WRITE))
     assert [sumsq(rt, st, d) for d in dats] == [5.0 * n, 0.0, 5.0 * n]
+
+
+def test_first_loop_follows_an_upload(rt):
+    """A loop right after op_upload_data reads all of the new values."""
+    n = 10_000_000
+    st = rt.decl_set(n, "s")
+    d = rt.decl_dat(st, 5, None, "d")
+    ones, twos = np.ones((n, 5)), np.full((n, 5), 2.0)
+    for _ in range(3):
+        rt.upload(d, ones)
+        assert sumsq(rt, st, d) == 5.0 * n
+        rt.upload(d, twos)
+        assert sumsq(rt, st, d) == 20.0 * n

@@ -17,6 +17,19 @@ extern "C" void pieces(long long rec, int cnt, int* out)
     const mgcfd::FetchPieces p = mgcfd::fetch_pieces((std::size_t)rec, cnt);
     out[0] = p.rows; out[1] = p.pieces; out[2] = p.slots;
 }
+// launches of a flat loop over n elements: {first, elements} each
+extern "C" int launches(int n, long long* out)
+{
+    int k = 0;
+    const int rc = mgcfd::flat_launches(n, [&](std::size_t at, int cnt) { out[2 * k] = at; out[2 * k + 1] = cnt; k++; return 0; });
+    return rc ? -1 : k;
+}
+extern "C" int stops_at(int n, int bad)
+{
+    int k = 0;
+    const int rc = mgcfd::flat_launches(n, [&](std::size_t, int) { return k++ == bad ? 7 : 0; });
+    return rc == 7 ? k : -1;
+}
 """
 
 
@@ -48,3 +61,22 @@ def test_fetch_pieces_fit_their_buffers(rules, rec, cnt):
     assert 1 <= rows and rows * rec <= rules.slot_bytes()
     assert (pieces - 1) * rows < cnt <= pieces * rows
     assert slots == min(pieces, rules.slot_count())
+
+
+@pytest.mark.parametrize("n", [0, 1, 2**29 - 1, 2**29, 2**29 + 1, 858993458, 858993459, 2**31 - 1])
+def test_flat_launches_cover_the_set(rules, n):
+    """Consecutive runs over the whole set, each of fewer than 2^32 threads
+    (five per element, in workgroups of 256)."""
+    out = (C.c_longlong * 16)()
+    k = rules.launches(n, out)
+    at = 0
+    for i in range(k):
+        assert out[2 * i] == at and out[2 * i + 1] > 0
+        assert -(-5 * out[2 * i + 1] // 256) * 256 < 2**32
+        at += out[2 * i + 1]
+    assert at == n
+    assert k == -(-n // 2**29)
+
+
+def test_flat_launches_stop_at_an_error(rules):
+    assert rules.stops_at(2**31 - 1, 1) == 2
