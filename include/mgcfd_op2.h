@@ -304,12 +304,19 @@ typedef struct mgcfd_level_bind {
 } mgcfd_level_bind;
 
 int mgcfd_mg_bind(int levels, const mgcfd_level_bind* binds);
-/* Runs 'cycles' multigrid cycles.  use_graph != 0 captures one cycle in a
- * hipGraph and replays it.  rms_hist (host, may be NULL) receives the L0 RMS
+/* Runs 'cycles' multigrid cycles.  use_graph != 0 replays cycles captured in
+ * hipGraphs: those between a run's first and last from its first run on, and
+ * a run's first and last cycle, or its only one, from the second run on with
+ * the same binding, flux variant, constants and part plans (until then they
+ * are launched plainly, which costs less than a capture).  rms_hist (host, may be NULL) receives the L0 RMS
  * per cycle.  *status: 0 ok, 1 negative min_dt (euler3d.cpp:480-484),
  * 2 NaN/Inf at L0 (euler3d.cpp:544-548); on an abort the state stops
  * changing at the failing smoothing step.  Returns 0 or a negative code. */
 int mgcfd_mg_run(int cycles, int use_graph, double* rms_hist, int* status);
+
+/* Cycles that this process's device-resident and batched runs have replayed
+ * from graphs so far. */
+long long mgcfd_graph_replays(void);
 
 /* Times 'iters' back-to-back launches of the edge-flux loop with HIP events
  * on the library stream; *ms_per_call receives the mean.  The launches are
