@@ -275,7 +275,8 @@ int mgcfd_plan_stats(op_map map, int* stats);
 int mgcfd_part_plan_stats(op_map map, int* stats);
 
 /* Part plan configuration of an edge->node map (variants PART_* / MIXED_*):
- * part_nodes in [16, 256] owned nodes per part; part_threads 0 (default),
+ * part_nodes in [16, 256] owned nodes per part, or 0 (as the map's number of
+ * 256-node patches selects, the default); part_threads 0 (default),
  * 256 or 512 for the kernel with the fused Runge-Kutta stage; record_bytes
  * 0 (by the plan's rule), 40 or 48 for the FP64 edge-flux kernel's LDS node
  * records.  Re-plans the map. */
@@ -360,8 +361,10 @@ int mgcfd_batch_create(int n, const mgcfd_mesh* meshes, const double* mach, cons
  * (256, 192 or 128), threads per part (256 or 512) and launch form (one
  * workgroup per part, or 2 or 4 persistent workgroups per CU walking their
  * XCD's parts) that give the fastest captured multigrid cycle of the whole
- * batch ('iters' timed cycles per candidate, levels tuned in turn).  The
- * batch's state is left as it was.  part_nodes / part_threads /
+ * batch ('iters' timed replays per candidate, levels tuned in turn).  256
+ * nodes with 256 threads and one workgroup per part stand for the level's own
+ * shape, which it starts with: smaller parts and more threads where it has
+ * few, by the library's rule.  The batch's state is left as it was.  part_nodes / part_threads /
  * persistent_per_cu [levels] (nullable) receive the choice; variants
  * without a part plan have nothing to tune (0s).  mgcfd_batch_autotune is
  * the same tuning, reporting level 0's part size. */
@@ -370,7 +373,8 @@ int mgcfd_batch_autotune_levels(mgcfd_batch b, int iters, int* part_nodes, int* 
                                 int* persistent_per_cu);
 /* Sets one level's part configuration directly (a tuning found earlier):
  * part_nodes in [16, 256], part_threads 256 or 512, persistent_per_cu 0
- * (one workgroup per part) or 1..8.  Re-plans the level. */
+ * (one workgroup per part) or 1..8; (256, 256, 0) returns the level to its own
+ * shape.  Re-plans the level. */
 int mgcfd_batch_set_part_config(mgcfd_batch b, int level, int part_nodes, int part_threads, int persistent_per_cu);
 /* Runs 'cycles' multigrid cycles from the setup state; rms receives
  * [n][cycles] L0 RMS residuals and status [n] (0 ok, 1 negative min dt,

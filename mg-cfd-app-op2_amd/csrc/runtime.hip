@@ -1587,11 +1587,17 @@ static void free_partplan(InvPlan& P)
     P.pt_wver = P.pt_w32ver = 0;
 }
 
+static int check_part_nodes(int nodes)
+{
+    return nodes >= 16 && nodes <= kPart ? 0 : fail("set_part_nodes: %d nodes per part outside [16, %d]", nodes, kPart);
+}
+
 // Re-plans the edge-parallel flux of an edge map with parts of at most
-// 'nodes' nodes (the autotuner's knob).
+// 'nodes' nodes (the autotuner's knob), 0: as the number of patches selects
+// (patch_part_nodes).
 static int set_part_nodes(op_map m, int nodes)
 {
-    if (nodes < 16 || nodes > kPart) return fail("set_part_nodes: %d nodes per part outside [16, %d]", nodes, kPart);
+    if (nodes) TRY(check_part_nodes(nodes));
     TRY(build_inverse(m));
     InvPlan& P = M(m)->inv;
     if (P.h_ptr.empty()) return fail("set_part_nodes: map %s has no part plan", m->name);

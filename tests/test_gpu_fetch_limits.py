@@ -1,14 +1,9 @@
 """Fetches beyond what the pinned landing buffers are made for."""
-import os
-import subprocess
-import sys
-
 import numpy as np
 import pytest
 
 import hip_shim
 import mgcfd
-from conftest import ROOT
 from test_gpu_fetch import ring
 
 pytestmark = pytest.mark.gpu
@@ -35,25 +30,6 @@ def test_elements_larger_than_a_buffer(rt, dim, typ, ordered):
     assert np.array_equal(rt.fetch(d), data)
 
 
-def run_script(tmp_path, body, **env):
-    """body in a process of its own, with the shim loaded as 'shim'; it has a
-    set 'st' with an order of its own, values 'data' and their dat 'd'."""
-    head = f"""
-import sys
-sys.path[:0] = {[os.path.join(ROOT, "tests"), os.path.join(ROOT, "mg-cfd-app-op2_amd")]!r}
-import numpy as np
-import hip_shim
-shim = hip_shim.load({hip_shim.build(tmp_path)!r})
-"""
-    script = tmp_path / "script.py"
-    script.write_text(head + body)
-    r = subprocess.run([sys.executable, "-u", str(script)], env=dict(os.environ, **env), capture_output=True,
-                       text=True, timeout=100)
-    assert r.returncode == 0, r.stdout + r.stderr
-    print(r.stdout)
-    assert r.stdout.split()[-1] == "ok"
-
-
 PREPARE = """
 import mgcfd
 from test_gpu_fetch import ring
@@ -69,7 +45,7 @@ mgcfd._check(rt.L.op_renumber(None), "op_renumber")
 def test_fetch_needs_no_device_memory(tmp_path):
     """Device memory is gone when a set's first dat is fetched; a later fetch,
     with memory again, takes the buffers; no error is left for later calls."""
-    run_script(tmp_path, PREPARE + """
+    hip_shim.run_script(tmp_path, PREPARE + """
 shim.shim_refuse_device(1)
 for _ in range(2):
     assert np.array_equal(rt.fetch(d), data)
@@ -86,7 +62,7 @@ print("ok")
 @pytest.mark.parametrize("left", [0, 1, 3])
 def test_fetch_with_fewer_pinned_buffers(tmp_path, left):
     """Six buffers' worth of pieces with none, one or three buffers to be had."""
-    run_script(tmp_path, PREPARE + f"""
+    hip_shim.run_script(tmp_path, PREPARE + f"""
 shim.shim_pinned_left({left})
 for _ in range(2):
     assert np.array_equal(rt.fetch(d), data)
@@ -99,7 +75,7 @@ print("ok")
 def test_fetch_without_further_threads(tmp_path):
     """No thread can be started (a limit that holds for ordinary users): the
     calling thread copies every piece."""
-    run_script(tmp_path, PREPARE + """
+    hip_shim.run_script(tmp_path, PREPARE + """
 import resource, threading
 assert np.array_equal(rt.fetch(d), data)
 resource.setrlimit(resource.RLIMIT_NPROC, (1, resource.getrlimit(resource.RLIMIT_NPROC)[1]))
@@ -119,7 +95,7 @@ def test_fetch_from_a_thread_on_another_device(tmp_path, n):
     """The library on the second of two devices (one, shown as two): the first
     fetch, made by a thread that has chosen no device, allocates and launches
     on the library's; the thread's own choice is left alone."""
-    run_script(tmp_path, "shim.shim_devices(2)\n" + PREPARE.replace("n = 300000", f"n = {n}") + """
+    hip_shim.run_script(tmp_path, "shim.shim_devices(2)\n" + PREPARE.replace("n = 300000", f"n = {n}") + """
 import ctypes as C, threading
 got = []
 def work():
