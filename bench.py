@@ -69,6 +69,7 @@ FP64_PEAK_TFLOPS = 78.6         # MI355X FP64 vector peak
 FLOP_PER_EDGE = 201             # flux.h:48-207 as written: 186 add/mul + 8 div + 7 sqrt
 N_NODES, N_EDGES = 300_000, 930_000
 MACH, AOA = 0.5, 3.0
+WARMUP_CYCLES = 3       # a run's first and last cycle are launched plainly, those between captured and replayed
 PROFILE_TRAFFIC = os.path.join(ROOT, "profiles", "flux_traffic.json")
 PROFILE_LARGE_TRAFFIC = os.path.join(ROOT, "profiles", "mg_cycle_traffic_8m.json")
 # served requests queued behind a busy server share a context in groups of at
@@ -166,15 +167,15 @@ def bench_shard(rt, variant, steps, warmup, n=1_000_000, e=3_100_000, copies=3):
 
 def bench_solve(rt, cycles=50):
     """Whole multigrid solve on the 300K-node mesh with its 4 levels (the
-    euler3d.cpp -g N loop, device-resident, one captured graph per cycle):
-    'cycles' cycles after one warm-up cycle, per flux variant, with each
-    state's largest per-variable difference from the FP64 exact one."""
+    euler3d.cpp -g N loop, device-resident, cycles replayed from a graph):
+    'cycles' cycles after the warm-up that captures it, per flux variant, with
+    each state's largest per-variable difference from the FP64 exact one."""
     mesh = mgcfd.mesh_knn(N_NODES, N_EDGES, 4, seed=2)
     out = dict(level_nodes=[len(l["coords"]) for l in mesh], cycles=cycles)
     ref = None
     for variant in ("gather_exact", "part_atomic", "part_coloured", "mixed_atomic"):
         b = mgcfd.Batch(rt, [mesh], [MACH], [AOA], variant)
-        b.run(1)
+        b.run(WARMUP_CYCLES)
         t0 = time.perf_counter()
         st, _ = b.run(cycles)
         el = time.perf_counter() - t0
@@ -243,7 +244,7 @@ def bench_large(rt, cycles=20, n=8_000_000, mach=0.7, aoa=2.0):
     """One large solve (8M level-0 nodes, E = 3.1 N, 4 levels, M0.7 a2deg):
     'cycles' cycles in mixed precision (MIXED_ATOMIC) against the same cycles
     in FP64 with the fastest FP64 variant within 1e-12 (PART_ATOMIC), each
-    after one warm-up cycle that captures its graph; the level-0 state's
+    after the warm-up cycles that capture the graph; the level-0 state's
     per-variable difference."""
     t = time.perf_counter()
     mesh = mgcfd.mesh_knn(n, int(round(3.1 * n)), 4, seed=8)
@@ -254,7 +255,7 @@ def bench_large(rt, cycles=20, n=8_000_000, mach=0.7, aoa=2.0):
     for variant in ("part_atomic", "mixed_atomic"):
         t = time.perf_counter()
         b = mgcfd.Batch(rt, [mesh], [mach], [aoa], variant)
-        b.run(1)
+        b.run(WARMUP_CYCLES)
         setup = time.perf_counter() - t
         t0 = time.perf_counter()
         st, _ = b.run(cycles)
@@ -564,14 +565,14 @@ def bench_batched(rt, n_meshes, cycles, fp64_variant, seed=40):
     """64 independent solves (N log-uniform in [20K, 500K], E = 3.1 N, 4
     levels, Mach U(0.3, 0.8), angle U(-2, 6) deg), 30 cycles each:
       - back to back in plain FP64 with 'fp64_variant' (the fastest FP64
-        flux within 1e-12 of the oracle), one captured graph per solve;
+        flux within 1e-12 of the oracle), one captured cycle per solve;
       - batched in the same FP64 variant (the gain from batching alone);
       - batched in mixed precision (MIXED_ATOMIC: FP32 increments summed
         by LDS FP64 atomics; 1.1x the batched MIXED_COLOURED rate on this
         workload) with the autotuned part plans (batching and precision
         together).
-    Setup is outside every timing; each form's first cycle (graph capture) is
-    an untimed warm-up."""
+    Setup is outside every timing, and so are each form's warm-up cycles (graph
+    capture)."""
     rng = np.random.default_rng(seed)
     sizes = np.exp(rng.uniform(np.log(20_000), np.log(500_000), n_meshes)).astype(int)
     mach = rng.uniform(0.3, 0.8, n_meshes)
@@ -584,7 +585,7 @@ def bench_batched(rt, n_meshes, cycles, fp64_variant, seed=40):
     ref0 = []
     for i, m in enumerate(meshes):
         b = mgcfd.Batch(rt, [m], [mach[i]], [aoa[i]], fp64_variant)
-        b.run(1)
+        b.run(WARMUP_CYCLES)
         t0 = time.perf_counter()
         st, _ = b.run(cycles)
         t_fp64 += time.perf_counter() - t0
@@ -598,7 +599,7 @@ def bench_batched(rt, n_meshes, cycles, fp64_variant, seed=40):
         b = mgcfd.Batch(rt, meshes, mach, aoa, variant)
         part = b.autotune(5) if tune else None
         t_setup = time.perf_counter() - t
-        b.run(1)
+        b.run(WARMUP_CYCLES)
         t0 = time.perf_counter()
         st, _ = b.run(cycles)
         el = time.perf_counter() - t0
