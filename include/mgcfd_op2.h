@@ -345,8 +345,8 @@ int mgcfd_time_stream(int n_copies, const op_map* edge_maps, const op_dat* vars,
  * Batched solves (no counterpart in the reference, which runs one mesh per
  * process): n independent multigrid meshes, all with the same number of
  * levels, concatenated level by level behind offset tables and advanced
- * together -- one launch per loop for the whole batch, one captured graph per
- * cycle.  Each mesh has its own freestream (mach[i], aoa_deg[i]), min dt, RMS
+ * together -- one launch per loop for the whole batch, its cycles replayed from
+ * captured graphs.  Each mesh has its own freestream (mach[i], aoa_deg[i]), min dt, RMS
  * history and status; a mesh's result equals its solve alone up to the
  * summation order of the chosen flux variant (bitwise for GATHER_EXACT).
  * Batches run on their own HIP stream.

@@ -623,8 +623,9 @@ __device__ __forceinline__ R part_speed(R rho, R mx, R my, R mz, R E)
 // {m . f, m v + p f, (E + p) v}, which needs no flux tensor.  The edge phase is
 // bound by FP64 issue once a part's data is staged: 94 FP64 instructions per
 // edge with the wave speeds formed here (40-byte records), against 136 with
-// the tensors of both endpoints: 930K-edge flux 18.5 -> 17.8 us, cycle of a
-// 1M-node solve 946 -> 908 us.
+// the tensors of both endpoints.  Tensors -> along the face, three alternating
+// runs: 930K-edge flux over five rotating meshes 18.8 -> 18.3 us, cycle of a
+// 300K-node solve 345 -> 341 us, of a 1M-node solve 768 -> 746 us.
 __device__ __forceinline__ void part_increment(const PState<double>& a, const PState<double>& b, double f0, double f1,
                                                double f2, double sc, double inc[5])
 {
@@ -2372,11 +2373,9 @@ __global__ void k_cell_volumes_node(int n_targets, const int* __restrict__ targe
     vol[n] = acc;
 }
 
-// Multigrid cycle counter, bumped once per cycle on the device.
 // ------------------------------------------------------------------------
-// Batched solves: the per-node reductions over a segment block table
-// {segment, lo, hi} whose blocks never straddle two meshes, then one final
-// reduction block per mesh.
+// Batched solves: per-node work over a segment block table {segment, lo, hi}
+// whose blocks never straddle two meshes.
 // ------------------------------------------------------------------------
 __global__ __launch_bounds__(kBlock) void k_calc_dt_seg(const int4* __restrict__ blk, const double* __restrict__ var,
                                                         const double* __restrict__ vol, double* __restrict__ dt,

@@ -256,14 +256,6 @@ static int check_launch()
 
 // ---------------------------------------------------------- renumbering --
 
-// Node order of a set from all dim-2 maps into it: recursive graph bisection
-// into parts of exactly kPart nodes (the last part takes the remainder).
-// Each split orders the segment by breadth-first distance from a
-// pseudo-peripheral node and cuts it at a multiple of kPart, so every part
-// is a compact, mostly connected patch of the mesh: the workgroup that owns
-// a part finds most neighbours of its nodes inside the part.
-// Morton (Z-order) key of each node of [lo, hi): coordinates quantised to
-// 21 bits per axis over the range's bounding box, bits interleaved.
 // n independent host-only tasks (no HIP calls), at most 16 threads.
 template <typename F>
 static void host_tasks(int n, F&& f)
@@ -317,6 +309,12 @@ static void morton_order(const std::vector<double>& geo, int lo, int hi, std::ve
     for (int i = lo; i < hi; i++) order[i] = key[i - lo].second;
 }
 
+// Node order of a set from all dim-2 maps into it: recursive graph bisection
+// into parts of exactly kPart nodes (the last part takes the remainder).
+// Each split orders the segment by breadth-first distance from a
+// pseudo-peripheral node and cuts it at a multiple of kPart, so every part
+// is a compact, mostly connected patch of the mesh: the workgroup that owns
+// a part finds most neighbours of its nodes inside the part.
 static std::vector<int> partition_order(int n, const std::vector<const MapImpl*>& emaps,
                                         const std::vector<int>& from_sizes, const std::vector<int>& segs,
                                         std::vector<int>& parts, const std::vector<double>& geo)
@@ -422,7 +420,7 @@ static std::vector<int> partition_order(int n, const std::vector<const MapImpl*>
 
 static int upload_dat(op_dat d);
 static int await_zeros(op_dat d);
-static void mg_release_all();
+static void mg_release_all();          // multigrid contexts and batches (mgrun.inc)
 static void mg_join_admissions();
 
 // Node coordinates [n][3] of a set not yet ordered: its internal order will
@@ -447,7 +445,7 @@ struct HostTimer {
         const double ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
         std::fprintf(stderr, "mgcfd timing: %s %s %.1f ms\n", what, name, ms);
     }
-};     // multigrid contexts and batches (mgrun.inc)
+};
 
 // Part boundaries of a node set's internal order (kPart-node chunks when the
 // set was not partitioned).
@@ -947,9 +945,10 @@ static int part_cut(int lo, int hi)
     return lo + (hi - lo > kWave ? (half + kWave - 1) / kWave * kWave : half);
 }
 
-// Blocked-gather plan.  Blocks are the kPart-node parts of the node order
-// (halved recursively while a part's halo exceeds kHaloCap).  Per block: the sorted halo, and the
-// incidences of its nodes in jagged-diagonal order -- diagonal k holds the
+// Blocked-gather plan.  Blocks are the kPart-node parts of the node order (cut
+// further on levels of few patches, see patch_part_nodes, and while a part's
+// halo exceeds kHaloCap).  Per block: the sorted halo, and the incidences of
+// its nodes in jagged-diagonal order -- diagonal k holds the
 // k-th incidence (reference edge order) of every node with degree > k;
 // nodes are sorted by decreasing degree inside a part, so diagonal k is a
 // prefix of the block's threads.
@@ -1158,22 +1157,23 @@ struct PartOut {
     std::string err;
 };
 
-// LDS bank-aware order of a part's local edges, within each colour (so the
-// coloured kernel's colour phases, and with them its sums, are unchanged).
-// The kernels give consecutive local edges to consecutive lanes, and the LDS
-// serves a wave's lanes in groups: 8 lanes per pass for the 16-byte record
-// reads of 48-byte records (whose bank is fixed by the slot modulo 8), 16
-// per pass for 8-byte accesses (accumulators at a 40-byte stride and
-// 40-byte records: slot modulo 16).  Each position takes, among the next
-// candidates of its colour, the edge whose endpoint slots (sa, sb) collide
-// least with those already in its 8- and 16-lane groups.  'le' holds the
-// edges by colour (code: sa | sb << 10 | flags << 20 | colour << 22).
+// A local edge of a part: its code (slot a | slot b << 10 | owner flags << 20 |
+// colour << 22) and the edge's id.
 struct PartEdge {
     unsigned code;
     int e;
 };
 
-//
+// LDS bank-aware order of a part's local edges, within each colour (so the
+// coloured kernel's colour phases, and with them its sums, are unchanged); 'le'
+// holds the edges by colour.
+// The kernels give consecutive local edges to consecutive lanes, and the LDS
+// serves a wave's lanes in groups: 8 lanes per pass for the 16-byte record
+// reads of 48-byte records (whose bank is fixed by the slot modulo 8), 16
+// per pass for 8-byte accesses (accumulators at a 40-byte stride and
+// 40-byte records: slot modulo 16).  Each position takes, among the next
+// candidates of its colour, the edge whose endpoint slots collide least with
+// those already in its 8- and 16-lane groups.
 // The next 48 candidates are bits of 64-bit words, position modulo 64: one
 // word per slot value and end, and four (8 and 16 lanes, either end) that say
 // who collides, so that a choice is a few word operations instead of a scan.
