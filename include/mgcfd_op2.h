@@ -309,10 +309,11 @@ int mgcfd_mg_bind(int levels, const mgcfd_level_bind* binds);
  * hipGraphs: those between a run's first and last from its first run on, and
  * a run's first and last cycle, or its only one, from the second run on with
  * the same binding, flux variant, constants and part plans (until then they
- * are launched plainly, which costs less than a capture).  rms_hist (host, may be NULL) receives the L0 RMS
- * per cycle.  *status: 0 ok, 1 negative min_dt (euler3d.cpp:480-484),
- * 2 NaN/Inf at L0 (euler3d.cpp:544-548); on an abort the state stops
- * changing at the failing smoothing step.  Returns 0 or a negative code. */
+ * are launched plainly, which costs less than a capture).  rms_hist (host,
+ * may be NULL) receives the L0 RMS per cycle.  *status: 0 ok, 1 negative
+ * min_dt (euler3d.cpp:480-484), 2 NaN/Inf at L0 (euler3d.cpp:544-548); on an
+ * abort the state stops changing at the failing smoothing step.  Returns 0 or
+ * a negative code. */
 int mgcfd_mg_run(int cycles, int use_graph, double* rms_hist, int* status);
 
 /* Cycles that this process's device-resident and batched runs have replayed
@@ -346,9 +347,9 @@ int mgcfd_time_stream(int n_copies, const op_map* edge_maps, const op_dat* vars,
  * process): n independent multigrid meshes, all with the same number of
  * levels, concatenated level by level behind offset tables and advanced
  * together -- one launch per loop for the whole batch, its cycles replayed from
- * captured graphs.  Each mesh has its own freestream (mach[i], aoa_deg[i]), min dt, RMS
- * history and status; a mesh's result equals its solve alone up to the
- * summation order of the chosen flux variant (bitwise for GATHER_EXACT).
+ * captured graphs.  Each mesh has its own freestream (mach[i], aoa_deg[i]),
+ * min dt, RMS history and status; a mesh's result equals its solve alone up to
+ * the summation order of the chosen flux variant (bitwise for GATHER_EXACT).
  * Batches run on their own HIP stream.
  */
 typedef struct mgcfd_batch_s* mgcfd_batch;
@@ -364,10 +365,10 @@ int mgcfd_batch_create(int n, const mgcfd_mesh* meshes, const double* mach, cons
  * batch ('iters' timed replays per candidate, levels tuned in turn).  256
  * nodes with 256 threads and one workgroup per part stand for the level's own
  * shape, which it starts with: smaller parts and more threads where it has
- * few, by the library's rule.  The batch's state is left as it was.  part_nodes / part_threads /
- * persistent_per_cu [levels] (nullable) receive the choice; variants
- * without a part plan have nothing to tune (0s).  mgcfd_batch_autotune is
- * the same tuning, reporting level 0's part size. */
+ * few, by the library's rule.  The batch's state is left as it was.
+ * part_nodes / part_threads / persistent_per_cu [levels] (nullable) receive
+ * the choice; variants without a part plan have nothing to tune (0s).
+ * mgcfd_batch_autotune is the same tuning, reporting level 0's part size. */
 int mgcfd_batch_autotune(mgcfd_batch b, int iters, int* part_nodes);
 int mgcfd_batch_autotune_levels(mgcfd_batch b, int iters, int* part_nodes, int* part_threads,
                                 int* persistent_per_cu);
